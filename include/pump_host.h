@@ -351,6 +351,12 @@ int pump_find_optimal_path(float dt, const float *xs, int n_wp, float *split, in
 /* single-pair helpers (host) for tests */
 float pump_host_topt(const float *x0, const float *x1, float tmax);
 float pump_host_cost(float tau, const float *x0, const float *x1);
+/* one pair of the pair pass as its kernel computes it: arrival time and cost,
+ * and (optional, 3 values) the steps of toptBisection with the final cost, how
+ * many of them evaluated the cost, and how often its shortened form did not
+ * settle a rounding */
+void pump_host_pair(const float *x0, const float *x1, float tmax, float *topt, float *cost,
+                    int *steps);
 /* pathPoint (2pBVP.cu:117-131) with the kernels' arithmetic */
 void pump_host_path_point(float t, float tau, const float *x0, const float *x1, float *x);
 /* the kernels' FP64 division a/b (reciprocal + residual steps), n pairs */

@@ -261,6 +261,7 @@ _SIGS = {
     "pump_timer_destroy": (None, [c_void_p]),
     "pump_host_topt": (c_float, [f32p, f32p, c_float]),
     "pump_host_cost": (c_float, [c_float, f32p, f32p]),
+    "pump_host_pair": (None, [f32p, f32p, c_float, f32p, f32p, i32p]),
     "pump_host_path_point": (None, [c_float, c_float, f32p, f32p, f32p]),
     "pump_host_div_rn": (None, [S, S, S, c_int64]),
     "pump_host_div_sq": (None, [S, S, S, c_int64]),

@@ -3,14 +3,19 @@
 // cost-to-goal heuristic (mainPUMP.cu:351-355) and the FP64 Newton polish of
 // arrival times.
 //
-// One lane per pair.  Pairs are enumerated directly in the output order
-// idx = i*(num-1) + k (k skips the diagonal), so stores of copts/topts are
-// fully coalesced and the source state x_i is uniform across most of a wave.
-// The work per pair is a few dozen FP64 cost evaluations (12.3 bisection
-// steps of two evaluations per pair on average for 16000 uniform samples):
-// the kernel is bound by VALU issue.  Lanes finish their bisection
-// after different iteration counts; to keep them busy each wave pulls pairs
-// from a shared counter when its lanes run dry (persistent waves).
+// Pairs are enumerated in the output order idx = i*(num-1) + k (k skips the
+// diagonal).  The reference's bisection (12.3 steps of two cost evaluations
+// per pair on average for 16000 uniform samples) runs in two parts with the
+// same decisions (pump_device.hpp): its leading steps from the sign of the
+// derivative, 64 fresh pairs of a wave in lockstep, and the remaining ones
+// (5.1 per pair and the final cost) by certified cost evaluations, as a
+// per-lane state machine over persistent waves, since lanes need between 1
+// and 32 of them.  The kernel is bound by VALU issue: 256 million pairs
+// (16000 samples) in 7.9 ms, 3.2e10 pairs/s, against 17.3 ms with every step
+// two full cost evaluations; a million pairs (1000 samples) 72 us against
+// 590, 65 thousand 24 us against 45, where the longest lane's steps decide.
+#include <algorithm>
+
 #include "pump_device.hpp"
 #include "pump_internal.hpp"
 
@@ -33,42 +38,25 @@ __device__ __forceinline__ void pair_of(int64_t idx, int num, int &i, int &j)
     j = k + (k >= i ? 1 : 0);
 }
 
-// Straight one-lane-per-pair form (used for small launches and as the
-// simplest statement of the mapping).
-__global__ __launch_bounds__(256) void k_fill_pairs(const float *__restrict__ samples, int num,
-                                                    float tmax, float *__restrict__ copts,
-                                                    float *__restrict__ topts, int64_t n_pairs)
-{
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < n_pairs;
-         idx += stride) {
-        int i, j;
-        pair_of(idx, num, i, j);
-        float a[kDim], b[kDim];
-        load_state(samples, i, a);
-        load_state(samples, j, b);
-        CostTerms c;
-        cost_terms(c, a, b);
-        float tau = topt_bisection(c, tmax);
-        topts[idx] = tau;
-        copts[idx] = cost_eval(c, tau);
-    }
-}
+// A pair set up for the state machine, in the wave's LDS queue: its terms and
+// bisection state, the states' indices, and the problem (batched launch).
+struct alignas(16) PairEntry {
+    PairTerms T;
+    float tl, tu, x, w;
+    int state_itr; // state in the low 3 bits
+    int i, j, inst;
+};
+static_assert(sizeof(PairEntry) == 112, "28 dwords: seven 16-byte LDS accesses");
 
-// Bisection as a per-lane state machine so that a lane that finishes takes
-// the next pair while its wave-mates are still iterating.  Every step
-// evaluates cost at two points per lane: the two of one dcost (tau +- h/2,
-// as dcost forms them), or, in the final phase, cost(topt) for the output.
-// The sequence of dcost evaluations per pair is the one toptBisection
-// performs, so the results are identical.  Idle lanes are refilled only
-// once kRefill of them have gathered (or none is busy), so that the
-// wave-wide cost of setting up new pairs is paid once for many lanes.
-enum : int { ST_TMAX = 0, ST_LOW = 1, ST_BIS = 2, ST_FIN = 3 };
+constexpr int kPairBlock = 256;
+constexpr int kSet = 64;     // pairs set up together by a wave
+// Idle lanes that are refilled together: 8, 16, 24, 32 give 8.25, 8.05, 8.27
+// and 8.63 ms at 16000 samples.
 constexpr int kRefill = 16;
-constexpr int kChunk = 2048; // pairs per claim of the work counter
+constexpr int kMaxChunk = 2048; // pairs per claim of the work counter at most
 
-// Pair sources: map a global pair index to the pair's cost terms, tmax and
-// output slots.  One instance (idx in the reference's output order) ...
+// Pair sources: the states behind a global pair index, and where a finished
+// pair's results go.  One instance, idx in the reference's output order.
 // With fewer than 2^32 pairs the row i = g / (num - 1) is found by a
 // multiply-high with the divisor's magic number (DivMagic).
 struct OnePairSource {
@@ -77,10 +65,8 @@ struct OnePairSource {
     float tmax;
     float *copts, *topts;
     DivMagic dm;
-    __device__ void take(int64_t g, CostTerms &c, float &tm, float *&oc, float *&ot,
-                         int64_t &oi) const
+    __device__ void load(int64_t g, float *a, float *b, float &tm, int &i, int &j, int &) const
     {
-        int i, j;
         if (dm.m) {
             const uint32_t n = (uint32_t)g;
             const uint32_t q = div_magic_apply(n, dm);
@@ -90,46 +76,64 @@ struct OnePairSource {
         } else {
             pair_of(g, num, i, j);
         }
-        float a[kDim], b[kDim];
         load_state(samples, i, a);
         load_state(samples, j, b);
-        cost_terms(c, a, b);
         tm = tmax;
-        oc = copts;
-        ot = topts;
-        oi = g;
+    }
+    __device__ void states(int i, int j, int, float *a, float *b) const
+    {
+        load_state(samples, i, a);
+        load_state(samples, j, b);
+    }
+    __device__ void store(int i, int j, int, float tau, float cost) const
+    {
+        const int64_t o = (int64_t)i * (num - 1) + j - (j > i ? 1 : 0);
+        topts[o] = tau;
+        copts[o] = cost;
     }
 };
 
-// ... or many: instance k owns global indices [prefix[k], prefix[k+1]).
+// Every sample to the goal (mainPUMP.cu:351-355): the cost alone.
+struct GoalSource {
+    const float *samples;
+    float goal[kDim];
+    float tmax;
+    float *h;
+    __device__ void states(int i, int, int, float *a, float *b) const
+    {
+        load_state(samples, i, a);
+        for (int d = 0; d < kDim; ++d)
+            b[d] = goal[d];
+    }
+    __device__ void load(int64_t g, float *a, float *b, float &tm, int &i, int &, int &) const
+    {
+        i = (int)g;
+        states(i, 0, 0, a, b);
+        tm = tmax;
+    }
+    __device__ void store(int i, int, int, float, float cost) const { h[i] = cost; }
+};
+
+// Many instances: instance k owns global indices [prefix[k], prefix[k+1]).
 // A lane keeps the range of the instance its last pair came from, so the
 // search over the prefix table runs only when a lane crosses into another
-// instance (a wave's 2048-pair chunks mostly lie inside one).
+// instance (a wave's chunks mostly lie inside one).
 struct ManyPairSource {
     const PairJob *jobs;
     const int64_t *prefix;
     int n_inst;
     mutable int cur = 0;
     mutable int64_t cur_lo = 0, cur_hi = 0;
-    __device__ void take(int64_t g, CostTerms &c, float &tm, float *&oc, float *&ot,
-                         int64_t &oi) const
+    __device__ void load(int64_t g, float *a, float *b, float &tm, int &i, int &j,
+                         int &inst) const
     {
         if (!(g >= cur_lo && g < cur_hi)) {
-            int lo = 0, hi = n_inst;
-            while (hi - lo > 1) {
-                const int mid = (lo + hi) >> 1;
-                if (prefix[mid] <= g)
-                    lo = mid;
-                else
-                    hi = mid;
-            }
-            cur = lo;
-            cur_lo = prefix[lo];
-            cur_hi = prefix[lo + 1];
+            cur = instance_of(prefix, n_inst, g);
+            cur_lo = prefix[cur];
+            cur_hi = prefix[cur + 1];
         }
         const PairJob J = global_job(jobs[cur]);
         const int64_t idx = g - cur_lo;
-        int i, j;
         if (J.dm_m) {
             const uint32_t n = (uint32_t)idx;
             const uint32_t q = div_magic_apply(n, DivMagic{J.dm_m, J.dm_s1, J.dm_s2});
@@ -139,194 +143,200 @@ struct ManyPairSource {
         } else {
             pair_of(idx, J.num, i, j);
         }
-        float a[kDim], b[kDim];
+        inst = cur;
         load_state(J.samples, i, a);
         load_state(J.samples, j, b);
-        cost_terms(c, a, b);
         tm = J.tmax;
-        oc = J.copts;
-        ot = J.topts;
-        oi = idx;
+    }
+    __device__ void states(int i, int j, int inst, float *a, float *b) const
+    {
+        const float *s = gptr(jobs[inst].samples);
+        load_state(s, i, a);
+        load_state(s, j, b);
+    }
+    __device__ void store(int i, int j, int inst, float tau, float cost) const
+    {
+        const PairJob J = global_job(jobs[inst]);
+        const int64_t o = (int64_t)i * (J.num - 1) + j - (j > i ? 1 : 0);
+        J.topts[o] = tau;
+        J.copts[o] = cost;
     }
 };
 
-// steps_out (may be null) receives the number of (lane, step) pairs
-// executed, i.e. the bisection steps of all pairs: each step is two cost
-// evaluations.
+// cost_eval from the states themselves, where cost_certified fails; out of
+// line, so that its registers stay off the loop
+__device__ __noinline__ float cost_of_states(float a0, float a1, float a2, float a3, float a4,
+                                             float a5, float b0, float b1, float b2, float b3,
+                                             float b4, float b5, float x)
+{
+    const float a[kDim] = {a0, a1, a2, a3, a4, a5}, b[kDim] = {b0, b1, b2, b3, b4, b5};
+    CostTerms c;
+    cost_terms(c, a, b);
+    return cost_eval(c, x);
+}
+
+// A persistent wave.  It owns the first chunk with its own number and claims
+// further ones from next_chunk (null: none).  Whenever kRefill lanes are
+// idle, they store the results they finished with and take set-up pairs from
+// the wave's queue; when that is empty the whole wave sets up the next kSet
+// pairs (bisect_start) into it.  Every other lane then makes one step.
+// steps_out (may be null) receives the number of toptBisection's steps over
+// all pairs, the derivative's and the final cost's included.
 template <class Src>
-__device__ __forceinline__ void pairs_persistent(const Src &src, int64_t n_pairs,
+__device__ __forceinline__ void pairs_persistent(const Src &src, int64_t n_pairs, int chunk,
                                                  unsigned long long *__restrict__ next_chunk,
                                                  unsigned long long *__restrict__ steps_out)
 {
+    __shared__ PairEntry queue[kPairBlock / 64][kSet];
     const int lane = threadIdx.x & 63;
-    // each wave claims kChunk pairs at a time from the global counter (one
-    // counter for the whole launch: small claims would serialise on it)
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    PairEntry *q = queue[wid];
+    const int64_t n_waves = (int64_t)gridDim.x * (kPairBlock / 64);
+    int64_t pool = ((int64_t)blockIdx.x * (kPairBlock / 64) + wid) * chunk;
+    int64_t pool_end = pool + chunk < n_pairs ? pool + chunk : n_pairs;
+    bool more = next_chunk != nullptr;
+    int qh = 0, qn = 0; // the queue holds q[qh .. qn)
 
-    int64_t my = -1;     // current pair of this lane, -1 when idle
-    int64_t pool = 0;    // next unclaimed pair index in the wave's chunk
-    int64_t pool_end = 0;
-    CostTerms c;
-    float tu = 0, tl = 0, topt = 0, tmax = 0;
-    float dcval = 0; // numerator ca - cb of the last dcost (1 before the first)
-    float *oc = nullptr, *ot = nullptr;
-    int64_t oi = 0;
-    int state = ST_TMAX, itr = 0, halvings = 0;
-    bool done_all = false;
-    unsigned long long steps = 0; // wave-uniform
+    PairTerms T;
+    BisectState S;
+    S.state = ST_IDLE;
+    int i = 0, j = 0, inst = 0;
+    float cost = 0.0f;
+    int steps = 0;
+    const auto cost_at = [&](float x) {
+        float a[kDim], b[kDim];
+        src.states(i, j, inst, a, b);
+        return cost_of_states(a[0], a[1], a[2], a[3], a[4], a[5], b[0], b[1], b[2], b[3], b[4],
+                              b[5], x);
+    };
 
     while (true) {
-        // refill idle lanes from the wave's chunk, claiming a new chunk as needed
-        unsigned long long idle = __ballot(my < 0);
-        const bool refill = __popcll(idle) >= kRefill || idle == ~0ull;
-        while (refill && idle != 0 && !done_all) {
-            if (pool >= pool_end) {
-                unsigned long long claimed = 0;
-                if (lane == 0)
-                    claimed = atomicAdd(next_chunk, (unsigned long long)kChunk);
-                // every lane is active here, so the first active lane is lane 0
-                const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)claimed);
-                const uint32_t hi =
-                    (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(claimed >> 32));
-                int64_t b = (int64_t)(((uint64_t)hi << 32) | lo);
-                if (b >= n_pairs) {
-                    done_all = true;
-                    break;
-                }
-                pool = b;
-                pool_end = b + kChunk < n_pairs ? b + kChunk : n_pairs;
+        unsigned long long idle = __ballot(S.state >= ST_DONE);
+        if (__popcll(idle) >= kRefill) {
+            if (S.state == ST_DONE) {
+                if (cost == 0.0f) // the sign of a zero
+                    cost = cost_at(S.x);
+                src.store(i, j, inst, S.x, cost);
+                S.state = ST_IDLE;
             }
-            // rank of this lane among idle lanes
-            int rank = __popcll(idle & ((1ull << lane) - 1ull));
-            int64_t avail = pool_end - pool;
-            bool take = (my < 0) && (rank < avail);
-            if (take) {
-                my = pool + rank;
-                src.take(my, c, tmax, oc, ot, oi);
-                state = ST_TMAX;
-                tu = tmax;
-                tl = 0.01f;
-                topt = 0.0f;
-                dcval = 1.0f;
-                itr = 0;
-                halvings = 0;
-            }
-            int took = __popcll(idle) < avail ? __popcll(idle) : (int)avail;
-            pool += took;
-            idle = __ballot(my < 0);
-        }
-        const unsigned long long busy = __ballot(my >= 0);
-        if (busy == 0) {
-            if (done_all)
-                break;
-            continue;
-        }
-        steps += (unsigned long long)__popcll(busy);
-        if (my >= 0) {
-            // the step's two cost evaluations
-            const float x = (state == ST_FIN)    ? topt
-                            : (state == ST_TMAX) ? tmax
-                            : (state == ST_LOW)  ? tl
-                                                 : (tu + tl) / 2.0f;
-            const float h = 0.000001f;
-            const float xa = state == ST_FIN ? x : x + h / 2.0f;
-            const float xb = state == ST_FIN ? x : x - h / 2.0f;
-            // For 2^-20 <= x <= 2^100 both points are at least 4.5e-7, so
-            // tau^3 stays within the reciprocal's exact range.
-            float ca, cb;
-            if (x >= 0x1p-20f && x <= 0x1p100f) {
-                ca = cost_eval_with(c, xa, RecipNewton{});
-                cb = cost_eval_with(c, xb, RecipNewton{});
-            } else {
-                ca = cost_eval(c, xa);
-                cb = cost_eval(c, xb);
-            }
-            if (state == ST_FIN) {
-                ot[oi] = topt;
-                oc[oi] = ca;
-                my = -1;
-            } else {
-                // dcost = (ca - cb) / h (2pBVP.cu:109-115) enters only
-                // through its sign, which is that of dc, and through
-                // |dcost| > 0.0001, which is |dc| >= kDcostBig
-                const float dc = ca - cb;
-                if (state == ST_TMAX) {
-                    if (dc < 0.0f) {
-                        state = ST_FIN;
-                        topt = tmax;
-                    } else {
-                        state = ST_LOW;
+            while (idle) {
+                if (qh == qn) {
+                    if (pool >= pool_end) {
+                        if (!more)
+                            break;
+                        unsigned long long claimed = 0;
+                        if (lane == 0)
+                            claimed = atomicAdd(next_chunk, (unsigned long long)chunk);
+                        // every lane is active here, so the first active lane is lane 0
+                        const uint32_t lo =
+                            (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)claimed);
+                        const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane(
+                            (int)(uint32_t)(claimed >> 32));
+                        pool = n_waves * chunk + (int64_t)(((uint64_t)hi << 32) | lo);
+                        pool_end = pool + chunk < n_pairs ? pool + chunk : n_pairs;
+                        if (pool >= n_pairs) {
+                            more = false;
+                            break;
+                        }
                     }
-                } else if (state == ST_LOW) {
-                    if (dc > 0.0f && halvings < 400) {
-                        tl = tl / 2.0f;
-                        ++halvings;
-                    } else {
-                        state = ST_BIS;
-                        if (!(fabsf(dcval) >= kDcostBig && itr < 50))
-                            state = ST_FIN; // topt stays 0, as the reference returns it
+                    const int n = pool_end - pool < kSet ? (int)(pool_end - pool) : kSet;
+                    if (lane < n) {
+                        PairEntry e;
+                        DerivTerms D;
+                        BisectState B;
+                        float a[kDim], b[kDim], tmax;
+                        e.i = e.j = e.inst = 0;
+                        src.load(pool + lane, a, b, tmax, e.i, e.j, e.inst);
+                        pair_terms(e.T, D, a, b);
+                        bisect_start(D, tmax, B, steps);
+                        e.tl = B.tl;
+                        e.tu = B.tu;
+                        e.x = B.x;
+                        e.w = B.w;
+                        e.state_itr = B.state | (B.itr << 3);
+                        q[lane] = e;
                     }
-                } else {
-                    ++itr;
-                    topt = x;
-                    dcval = dc;
-                    if (dcval > 0.0f)
-                        tu = topt;
-                    else
-                        tl = topt;
-                    if (!(fabsf(dcval) >= kDcostBig && itr < 50))
-                        state = ST_FIN;
+                    pool += n;
+                    qh = 0;
+                    qn = n;
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
                 }
+                const int rank = __popcll(idle & ((1ull << lane) - 1ull));
+                const int n_idle = __popcll(idle);
+                if (S.state == ST_IDLE && rank < qn - qh) {
+                    const PairEntry e = q[qh + rank];
+                    T = e.T;
+                    S.tl = e.tl;
+                    S.tu = e.tu;
+                    S.x = e.x;
+                    S.w = e.w;
+                    S.state = e.state_itr & 7;
+                    S.itr = e.state_itr >> 3;
+                    i = e.i;
+                    j = e.j;
+                    inst = e.inst;
+                }
+                qh += n_idle < qn - qh ? n_idle : qn - qh;
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                idle = __ballot(S.state == ST_IDLE);
             }
+            if (idle == ~0ull)
+                break; // nothing left to take
+        }
+        if (S.state < ST_DONE) {
+            float xa, xb, ca, cb;
+            int skipped;
+            if (!bisect_costs(T, S, xa, xb, ca, cb)) {
+                ca = cost_at(xa);
+                cb = cost_at(xb);
+            }
+            cost = ca;
+            bisect_update(S, ca, cb, skipped);
+            steps += 1 + skipped;
         }
     }
-    if (steps_out && lane == 0)
-        atomicAdd(steps_out, steps);
+    if (steps_out) {
+        for (int off = 32; off > 0; off >>= 1)
+            steps += __shfl_xor(steps, off, 64);
+        if (lane == 0)
+            atomicAdd(steps_out, (unsigned long long)steps);
+    }
 }
 
-__global__ __launch_bounds__(256) void k_fill_pairs_persistent(
+__global__ __launch_bounds__(kPairBlock) void k_fill_pairs_persistent(
     const float *__restrict__ samples, int num, float tmax, float *__restrict__ copts,
-    float *__restrict__ topts, int64_t n_pairs, DivMagic dm,
+    float *__restrict__ topts, int64_t n_pairs, DivMagic dm, int chunk,
     unsigned long long *__restrict__ next_chunk, unsigned long long *__restrict__ steps_out)
 {
     const OnePairSource src{samples, num, tmax, copts, topts, dm};
-    pairs_persistent(src, n_pairs, next_chunk, steps_out);
+    pairs_persistent(src, n_pairs, chunk, next_chunk, steps_out);
 }
 
 // all ordered pairs of many instances in one persistent launch
-__global__ __launch_bounds__(256) void k_fill_pairs_many(const PairJob *__restrict__ jobs,
-                                                         const int64_t *__restrict__ prefix,
-                                                         int n_inst, int64_t n_pairs,
-                                                         unsigned long long *__restrict__ next_chunk)
+__global__ __launch_bounds__(kPairBlock) void k_fill_pairs_many(
+    const PairJob *__restrict__ jobs, const int64_t *__restrict__ prefix, int n_inst,
+    int64_t n_pairs, int chunk, unsigned long long *__restrict__ next_chunk)
 {
     const ManyPairSource src{jobs, prefix, n_inst};
-    pairs_persistent(src, n_pairs, next_chunk, nullptr);
+    pairs_persistent(src, n_pairs, chunk, next_chunk, nullptr);
+}
+
+// h[i] = cost(toptBisection(x_i, goal)) for i < num-1, h[num-1] = 0
+__global__ __launch_bounds__(kPairBlock) void k_heuristic(const GoalSource src, int num)
+{
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        src.h[num - 1] = 0.0f;
+    pairs_persistent(src, num - 1, kSet, nullptr, nullptr);
 }
 
 __global__ void k_zero_counter(unsigned long long *c)
 {
     if (threadIdx.x == 0)
         *c = 0ull;
-}
-
-// h[i] = cost(toptBisection(x_i, goal)) for i < num-1, h[num-1] = 0
-__global__ __launch_bounds__(256) void k_heuristic(const float *__restrict__ samples, int num,
-                                                   float g0, float g1, float g2, float g3,
-                                                   float g4, float g5, float tmax,
-                                                   float *__restrict__ h)
-{
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= num)
-        return;
-    if (i == num - 1) {
-        h[i] = 0.0f;
-        return;
-    }
-    float a[kDim], b[kDim] = {g0, g1, g2, g3, g4, g5};
-    load_state(samples, i, a);
-    CostTerms c;
-    cost_terms(c, a, b);
-    float tau = topt_bisection(c, tmax);
-    h[i] = cost_eval(c, tau);
 }
 
 // FP64 polish of a bisected arrival time: the root of
@@ -411,9 +421,44 @@ __global__ __launch_bounds__(256) void k_polish(const float *__restrict__ sample
 using namespace pump;
 
 namespace pump {
+// Launch shape of the persistent pair pass: the workgroups and the pairs per
+// claim.  A launch with at most 16 sets of 64 pairs per resident wave is
+// dealt out evenly (no claims, no counter): with so few, the claims
+// themselves, which serialise on one address at about 12 ns each, would cost
+// more than the unevenness.  Above that a wave's own first chunk is a
+// quarter of its share, at least 8 sets (claims stay below the counter's
+// rate) and at most kMaxChunk pairs.
+struct PairShape {
+    unsigned blocks;
+    int chunk;
+    bool claims;
+};
+
+static int pair_shape(int64_t n_pairs, int blocks_per_cu, PairShape &p)
+{
+    int dev = 0, cus = 256;
+    PUMP_HIP(hipGetDevice(&dev));
+    PUMP_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    const int64_t sets = (n_pairs + kSet - 1) / kSet;
+    int64_t waves = (int64_t)cus * blocks_per_cu * (kPairBlock / 64);
+    if (waves > sets)
+        waves = sets;
+    const int64_t per = (sets + waves - 1) / waves;
+    p.claims = per > 16;
+    const int64_t chunk = p.claims ? std::min<int64_t>(std::max<int64_t>(per / 4, 8) * kSet, kMaxChunk)
+                                   : per * kSet;
+    p.chunk = (int)chunk;
+    if (!p.claims) // the waves that have a chunk
+        waves = (n_pairs + chunk - 1) / chunk;
+    p.blocks = (unsigned)((waves + kPairBlock / 64 - 1) / (kPairBlock / 64));
+    return PUMP_OK;
+}
+
+constexpr int kPairBlocksPerCu = 4; // what 111 VGPRs keep resident
+
 // All ordered pairs of one instance; *steps (may be null) receives the
-// bisection steps of all pairs, 0 for a launch below 65,536 pairs (the
-// plain one-lane-per-pair kernel, which does not count them).
+// bisection steps of all pairs, 0 for a launch below 65,536 pairs (not
+// counted there).
 int fill_copts_topts(const float *d_samples, int num, float tmax, float *d_copts, float *d_topts,
                      hipStream_t s, int64_t *steps)
 {
@@ -421,9 +466,17 @@ int fill_copts_topts(const float *d_samples, int num, float tmax, float *d_copts
     const int64_t n_pairs = (int64_t)num * (num - 1);
     if (steps)
         *steps = 0;
-    if (n_pairs < (1 << 16)) {
-        hipLaunchKernelGGL(k_fill_pairs, dim3(grid_for(n_pairs, 256)), dim3(256), 0, s, d_samples,
-                           num, tmax, d_copts, d_topts, n_pairs);
+    if (n_pairs < (1 << 16))
+        steps = nullptr;
+    PairShape p;
+    const int r = pair_shape(n_pairs, kPairBlocksPerCu, p);
+    if (r != PUMP_OK)
+        return r;
+    const DivMagic dm = n_pairs < (1ll << 32) ? div_magic((uint32_t)(num - 1)) : DivMagic{0, 0, 0};
+    if (!p.claims && !steps) {
+        hipLaunchKernelGGL(k_fill_pairs_persistent, dim3(p.blocks), dim3(kPairBlock), 0, s, d_samples, num,
+                           tmax, d_copts, d_topts, n_pairs, dm, p.chunk,
+                           (unsigned long long *)nullptr, (unsigned long long *)nullptr);
         PUMP_LAUNCHED();
         return PUMP_OK;
     }
@@ -435,18 +488,9 @@ int fill_copts_topts(const float *d_samples, int num, float tmax, float *d_copts
         hipFree(counter);
         PUMP_HIP(me);
     }
-    int dev = 0, cus = 256;
-    hipGetDevice(&dev);
-    hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    // 8 resident 256-lane workgroups per CU
-    int64_t blocks = (int64_t)cus * 8;
-    int64_t need = (n_pairs + 255) / 256;
-    if (blocks > need)
-        blocks = need;
-    const DivMagic dm = n_pairs < (1ll << 32) ? div_magic((uint32_t)(num - 1)) : DivMagic{0, 0, 0};
-    hipLaunchKernelGGL(k_fill_pairs_persistent, dim3((unsigned)blocks), dim3(256), 0, s,
-                       d_samples, num, tmax, d_copts, d_topts, n_pairs, dm, counter,
-                       steps ? counter + 1 : nullptr);
+    hipLaunchKernelGGL(k_fill_pairs_persistent, dim3(p.blocks), dim3(kPairBlock), 0, s, d_samples,
+                       num, tmax, d_copts, d_topts, n_pairs, dm, p.chunk,
+                       p.claims ? counter : nullptr, steps ? counter + 1 : nullptr);
     hipError_t le = hipGetLastError();
     hipError_t se = hipStreamSynchronize(s);
     unsigned long long n_steps = 0;
@@ -483,9 +527,12 @@ extern "C" int pump_heuristic(const float *d_samples, int num, const float *goal
                               float *d_h, pump_stream_t stream)
 {
     PUMP_REQUIRE(d_samples && goal_host && d_h && num >= 1);
-    const float *g = goal_host;
-    hipLaunchKernelGGL(k_heuristic, dim3((num + 255) / 256), dim3(256), 0, as_stream(stream),
-                       d_samples, num, g[0], g[1], g[2], g[3], g[4], g[5], tmax, d_h);
+    GoalSource src{d_samples, {}, tmax, d_h};
+    for (int d = 0; d < kDim; ++d)
+        src.goal[d] = goal_host[d];
+    // a set of 64 samples per wave
+    hipLaunchKernelGGL(k_heuristic, dim3((num + kPairBlock - 1) / kPairBlock), dim3(kPairBlock), 0,
+                       as_stream(stream), src, num);
     PUMP_LAUNCHED();
     return PUMP_OK;
 }
@@ -501,17 +548,16 @@ int fill_pairs_many(const PairJob *d_jobs, const int64_t *d_prefix, int n_inst, 
                  blocks_per_cu > 0);
     if (n_pairs == 0)
         return PUMP_OK;
-    int dev = 0, cus = 256;
-    PUMP_HIP(hipGetDevice(&dev));
-    PUMP_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    int64_t blocks = (int64_t)cus * blocks_per_cu;
-    const int64_t need = (n_pairs + 255) / 256;
-    if (blocks > need)
-        blocks = need;
-    hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(64), 0, s, d_counter);
-    PUMP_LAUNCHED();
-    hipLaunchKernelGGL(k_fill_pairs_many, dim3((unsigned)blocks), dim3(256), 0, s, d_jobs,
-                       d_prefix, n_inst, n_pairs, d_counter);
+    PairShape p;
+    const int r = pair_shape(n_pairs, blocks_per_cu, p);
+    if (r != PUMP_OK)
+        return r;
+    if (p.claims) {
+        hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(64), 0, s, d_counter);
+        PUMP_LAUNCHED();
+    }
+    hipLaunchKernelGGL(k_fill_pairs_many, dim3(p.blocks), dim3(kPairBlock), 0, s, d_jobs,
+                       d_prefix, n_inst, n_pairs, p.chunk, p.claims ? d_counter : nullptr);
     PUMP_LAUNCHED();
     return PUMP_OK;
 }

@@ -648,6 +648,36 @@ extern "C" float pump_host_topt(const float *x0, const float *x1, float tmax)
     return topt_bisection(c, tmax);
 }
 
+extern "C" void pump_host_pair(const float *x0, const float *x1, float tmax, float *topt,
+                               float *cost, int *steps)
+{
+    PairTerms T;
+    DerivTerms D;
+    BisectState S;
+    CostTerms c;
+    cost_terms(c, x0, x1);
+    pair_terms(T, D, x0, x1);
+    int n[3] = {0, 0, 0};
+    bisect_start(D, tmax, S, n[0]);
+    float ca = 0, cb = 0, xa, xb;
+    while (S.state != ST_DONE) {
+        ++n[0];
+        ++n[1];
+        int skipped;
+        if (!bisect_costs(T, S, xa, xb, ca, cb)) {
+            ++n[2];
+            ca = cost_eval(c, xa);
+            cb = cost_eval(c, xb);
+        }
+        bisect_update(S, ca, cb, skipped);
+        n[0] += skipped;
+    }
+    *cost = ca != 0.0f ? ca : cost_eval(c, S.x);
+    *topt = S.x;
+    if (steps)
+        std::memcpy(steps, n, sizeof(n));
+}
+
 extern "C" float pump_host_cost(float tau, const float *x0, const float *x1)
 {
     CostTerms c;

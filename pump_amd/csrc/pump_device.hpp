@@ -79,32 +79,7 @@ __host__ __device__ __forceinline__ void cost_terms(CostTerms &c, const float *a
     c.f30c = a[5] + b[5];
 }
 
-// 1/x by IEEE division (any x)
-struct RecipDiv {
-    __host__ __device__ double operator()(double x) const { return 1.0 / x; }
-};
-
-// 1/x for 2^-100 <= |x| <= 2^400, bit-identical to RecipDiv there.  The
-// compiler's FP64 division n/d is: d' and n' from v_div_scale, r = rcp(d'),
-// two Newton steps r1 = fma(r, fma(-d', r, 1), r) and r2 = fma(r1,
-// fma(-d', r1, 1), r1), q = n' r2, then v_div_fmas(fma(-d', q, n'), r2, q)
-// and v_div_fixup.  For n = 1 and such d the scale steps return their
-// operands unchanged (they act only for subnormal or near-overflow operands
-// and quotients, or exponent gaps of 768 and more), v_div_fmas is a plain
-// fma and v_div_fixup changes only zeros, infinities and NaNs.  What is left
-// is the sequence below, with q = r2 exactly.
-struct RecipNewton {
-    __device__ double operator()(double x) const
-    {
-        const double r0 = __builtin_amdgcn_rcp(x);
-        const double r1 = fma(r0, fma(-x, r0, 1.0), r0);
-        const double r2 = fma(r1, fma(-x, r1, 1.0), r1);
-        return fma(fma(-x, r2, 1.0), r2, r2);
-    }
-};
-
-template <class Recip>
-__host__ __device__ __forceinline__ float cost_eval_with(const CostTerms &c, float tau, Recip recip)
+__host__ __device__ __forceinline__ float cost_eval(const CostTerms &c, float tau)
 {
     const double g2 = (double)kGravity * (double)kGravity;
     const double t = (double)tau;
@@ -135,12 +110,7 @@ __host__ __device__ __forceinline__ float cost_eval_with(const CostTerms &c, flo
     s = s + g2 * t4;
     s = s + (double)(c.f29a * (c.f29b + c.f29c * tau));
     s = s + (double)(c.f30a * (c.f30b + c.f30c * tau));
-    return (float)(recip(t3) * s);
-}
-
-__host__ __device__ __forceinline__ float cost_eval(const CostTerms &c, float tau)
-{
-    return cost_eval_with(c, tau, RecipDiv{});
+    return (float)(1.0 / t3 * s);
 }
 
 // |RN(d / 1e-6f)| > 0.0001 exactly when |d| >= kDcostBig, for every float d
@@ -185,6 +155,312 @@ __host__ __device__ __forceinline__ float topt_bisection(const CostTerms &c, flo
             tl = topt;
     }
     return topt;
+}
+
+// ---------------------------------------------------------------------------
+// The same bisection with few full cost evaluations.
+//
+// toptBisection only uses the sign of dc = cost(xa) - cost(xb), xa = x + h/2
+// and xb = x - h/2 rounded to float, and whether |dc| >= kDcostBig.  Far from
+// the root both follow from the derivative, so most steps need no cost
+// evaluation (deriv_sign); near it the cost is evaluated by a shorter FP64
+// expression whose rounding to float is proven, case by case, to be that of
+// cost_eval (cost_certified), which runs itself where the proof fails.
+//
+// Notation: u = 2^-24, t the evaluation point, and with the float products of
+// CostTerms kept as they are, the numerator of the cost before the last
+// division is s(t) = s7 + sum_i fl(l_i t) + fl(a29 fl(b29 + fl(c29 t))) +
+// fl(a30 fl(b30 + fl(c30 t))) + n2 t^2 + n3 t^3 + k4 t^4, each fl one float
+// rounding.  Without those roundings it is p(t) = n0 + n1 t + n2 t^2 + n3 t^3
+// + k4 t^4, and C(t) = p(t) / t^3 has C'(t) = q(t) / t^4 with
+// q(t) = k4 t^4 - n2 t^2 - 2 n1 t - 3 n0.
+// MP(t) = |n0| + |n1| t + |n2| t^2 + |n3| t^3 + k4 t^4.
+// ---------------------------------------------------------------------------
+struct PairTerms {
+    float l[8];                   // f8..f15 with the sign of their term
+    float a29, b29, c29, a30, b30, c30;
+    double s7, n2, n3;
+};
+
+// deriv_sign's constants of a pair
+struct DerivTerms {
+    float n0x3, n1x2, n2; // 3 n0, 2 n1, n2
+    float n0, n1, n3;     // signed, for p and MP
+    float k0, k1;         // bound of the float roundings at both points: (k0 + k1 t) / t^3
+};
+
+constexpr float kK4 = 1.0f + kGravity * kGravity;
+constexpr float kTMin = 0x1p-7f, kTMax = 0x1p7f; // where deriv_sure holds
+constexpr float kFastMin = 0x1p-10f;             // cost_fast's bound holds from here to kTMax
+
+__host__ __device__ __forceinline__ void pair_terms(PairTerms &T, DerivTerms &D, const float *a,
+                                                    const float *b)
+{
+    CostTerms c;
+    cost_terms(c, a, b);
+    T.l[0] = c.f8;
+    T.l[1] = c.f9;
+    T.l[2] = -c.f10;
+    T.l[3] = -c.f11;
+    T.l[4] = -c.f12;
+    T.l[5] = -c.f13;
+    T.l[6] = -c.f14;
+    T.l[7] = -c.f15;
+    T.a29 = c.f29a;
+    T.b29 = c.f29b;
+    T.c29 = c.f29c;
+    T.a30 = c.f30a;
+    T.b30 = c.f30b;
+    T.c30 = c.f30c;
+    T.s7 = c.s7;
+    T.n2 = ((c.d16 + c.d17) + (c.d18 + c.f19)) + ((c.d20 + c.f21) + (c.d22 + c.f23)) + c.d24;
+    T.n3 = c.f25 - c.f26;
+    const double ab29 = (double)T.a29 * T.b29, ab30 = (double)T.a30 * T.b30;
+    const double ac29 = (double)T.a29 * T.c29, ac30 = (double)T.a30 * T.c30;
+    double n1 = ac29 + ac30;
+    float F = 0.0f;
+    for (int i = 0; i < 8; ++i) {
+        n1 = n1 + (double)T.l[i];
+        F = F + fabsf(T.l[i]);
+    }
+    const double n0 = (T.s7 + ab29) + ab30;
+    D.n0 = (float)n0;
+    D.n0x3 = (float)(3.0 * n0);
+    D.n1 = (float)n1;
+    D.n1x2 = 2.0f * D.n1;
+    D.n2 = (float)T.n2;
+    D.n3 = (float)T.n3;
+    // fl(l t) is off by u |l| t, and fl(a fl(b + fl(c t))) by
+    // |a| (2u (|b| + |c| t) + u |c| t); twice that for the two points
+    D.k0 = 0x1p-22f * ((float)fabs(ab29) + (float)fabs(ab30));
+    D.k1 = 0x1p-23f * (F + 3.0f * ((float)fabs(ac29) + (float)fabs(ac30)));
+}
+
+__host__ __device__ __forceinline__ float pair_mp(const DerivTerms &D, float t)
+{
+    return fmaf(fmaf(fmaf(fmaf(kK4, t, fabsf(D.n3)), t, fabsf(D.n2)), t, fabsf(D.n1)), t,
+                fabsf(D.n0));
+}
+
+// The sign of dc at x: kPos (dc >= kDcostBig for certain), kNeg
+// (dc <= -kDcostBig for certain), kZero (dc = 0 for certain) or kUnsure.
+// With d = xa - xb (exact: both lie within a factor of two of each other):
+//   * d = 0 makes both points equal, dc = 0.
+//   * C(xa) - C(xb) = d C'(y) for a y in [xb, xa], and |C'(y) - C'(x)| <=
+//     d max |C''| <= d 12 MP(x) / x^5 (1 + 1e-3) (|C''| <= 4 (k4 t^4 + n2 t^2
+//     + 2 |n1| t + 3 |n0|) / t^5, and d/x <= 2^-12.8 for x >= 2^-7).
+//   * cost_eval's float roundings before the final one move s by at most
+//     (k0 + k1 t) / 2 at either point; its FP64 roundings by 2^-47 A(t), A the
+//     sum of all terms' magnitudes (s7 as one).  A <= |n0| + (k0 + k1 t) 2^23
+//     + 4.1 n2 t^2 + 2 k4 t^4 <= 5 MP + (k0 + k1 t) 2^23: s7 is n0 less ab29
+//     and ab30; the velocity terms of n2 are in magnitude at most three times
+//     n2; and 2|g| (|vz0| + |vz1|) t^3 <= n2 t^2 + k4 t^4.
+//   * The final roundings add at most u |C| each (2^-150 for a subnormal, far
+//     inside the slack of the kDcostBig term), with |C| t^3 <=
+//     |p| + 2^-10 MP for p as evaluated here (rounding, and t within d).
+// So the sign is sure, and |dc| >= kDcostBig, when
+//   d |q| > x (k0 + k1 x + 2^-23 (|p| + 2^-10 MP)) + x^4 kDcostBig
+//           + d MP (q's own rounding, 18u, and 12 d / x).
+// Both sides are multiplied by x below, with the constants rounded up; the
+// FP32 evaluation of the right side (positive terms) is covered by 1.002.
+// A NaN or an infinity fails the comparison.
+enum : int { kUnsure = 0, kPos = 1, kNeg = 2, kZero = 3 };
+
+// The test above at x (within [kTMin, kTMax]), and q(x)
+__host__ __device__ __forceinline__ bool deriv_sure(const DerivTerms &D, float x, float &q)
+{
+    const float h = 0.000001f;
+    const float d = (x + h / 2.0f) - (x - h / 2.0f);
+    const float x2 = x * x;
+    q = fmaf(fmaf(fmaf(kK4, x2, -D.n2), x, -D.n1x2), x, -D.n0x3);
+    const float p = fmaf(fmaf(fmaf(fmaf(kK4, x, D.n3), x, D.n2), x, D.n1), x, D.n0);
+    const float mp = pair_mp(D, x);
+    const float e = fmaf(D.k1, x, D.k0) + 0x1p-23f * fmaf(0x1p-10f, mp, fabsf(p));
+    const float bound = fmaf(x2, fmaf(x2 * x, 1.1e-10f, e),
+                             d * mp * fmaf(32.0f * 0x1p-24f, x, 24.0f * d));
+    return d * fabsf(q) * x > 1.002f * bound;
+}
+
+__host__ __device__ __forceinline__ int deriv_sign(const DerivTerms &D, float x)
+{
+    const float h = 0.000001f;
+    if (x + h / 2.0f == x - h / 2.0f)
+        return kZero;
+    float q;
+    const bool sure = deriv_sure(D, x, q);
+    if (!(x >= kTMin && x <= kTMax && sure))
+        return kUnsure;
+    return q > 0.0f ? kPos : kNeg;
+}
+
+// Approximations of 1/a and 1/b within 2^-51 relative, for b within 2^-8.3
+// of a (the cubes of two points h apart, x >= kFastMin).
+__host__ __device__ __forceinline__ void recip_near(double a, double b, double &ra, double &rb)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    const double r0 = __builtin_amdgcn_rcp(a);
+    const double r1 = fma(r0, fma(-a, r0, 1.0), r0);
+    ra = fma(r1, fma(-a, r1, 1.0), r1);
+#else
+    ra = 1.0 / a;
+#endif
+    // e = 1 - b ra: ra (1 + e + e^2) is within e^3 < 2^-24.9 of 1/b,
+    // relative, and one Newton step squares that
+    const double e = fma(-b, ra, 1.0);
+    const double r = fma(ra, fma(e, e, e), ra);
+    rb = fma(r, fma(-b, r, 1.0), r);
+}
+
+// The cost at x before its rounding to float, within 2^-47 A(x) / x^3 of
+// cost_eval's: the float products are cost_eval's own; the other terms are
+// summed by their common power.  In units of 2^-53 A / x^3: cost_eval's
+// roundings on s after s7 are at most 25 (23 sums; the products and powers
+// together 2), this form's 23 (the sum n2 8, n3 and k4 2, the Horner steps 3,
+// the other sums 10), and t^3, reciprocal and final product 3 there and 7
+// here: 58, and the rest to 64 covers the bound's FP32 evaluation, its value at
+// the midpoint for both points, and its division by one's cube (the cubes
+// differ by 0.3% at most).  r3: recip_near's 1/x^3.
+__host__ __device__ __forceinline__ double cost_fast(const PairTerms &T, float x, double r3)
+{
+    const double k4 = 1.0 + (double)kGravity * (double)kGravity;
+    const double t = (double)x;
+    const double s0 = (double)(T.l[0] * x) + (double)(T.l[1] * x);
+    const double s1 = (double)(T.l[2] * x) + (double)(T.l[3] * x);
+    const double s2 = (double)(T.l[4] * x) + (double)(T.l[5] * x);
+    const double s3 = (double)(T.l[6] * x) + (double)(T.l[7] * x);
+    const double s4 = (double)(T.a29 * (T.b29 + T.c29 * x)) +
+                      (double)(T.a30 * (T.b30 + T.c30 * x));
+    const double lin = ((s0 + s1) + (s2 + s3)) + (s4 + T.s7);
+    const double s = fma(t * t, fma(t, fma(t, k4, T.n3), T.n2), lin);
+    return s * r3;
+}
+
+// cost_eval's result from cost_fast's C and the bound w of its distance:
+// every value within w of C rounds to the same float.  False where that is
+// not so (once in 10^4 evaluations) and for NaNs.  The sign of a zero is not
+// settled.
+__host__ __device__ __forceinline__ bool cost_certified(double C, double w, float &out)
+{
+    const float lo = (float)(C - w);
+    out = (float)(C + w);
+    return out == lo;
+}
+
+// A pair's place in toptBisection.  x is the next point: tmax (ST_TMAX), tl
+// (ST_LOW), the bracket's midpoint (ST_BIS), the result, whose cost is still
+// to be evaluated (ST_FIN) or has been (ST_DONE).
+enum : int { ST_TMAX = 0, ST_LOW = 1, ST_BIS = 2, ST_FIN = 3, ST_DONE = 4, ST_IDLE = 5 };
+
+// w (1 + x^4) / x^3 bounds |cost_fast - cost_eval| (w is infinite where that
+// is not known, so that every cost comes from cost_eval).
+struct BisectState {
+    float tl, tu, x, w;
+    int state, itr; // itr: bisection steps (ST_BIS), halvings (ST_LOW)
+};
+
+// The leading steps of toptBisection(tmax) that deriv_sign decides; steps
+// is incremented by their number.  With tl >= kTMin and tu <= kTMax the
+// bracket reaches neighbouring floats in fewer than 40 halvings, so no
+// 50-step limit binds here; the loop's own limit only ends it should every
+// sign be sure down to there, and the remaining steps follow one by one.
+__host__ __device__ __forceinline__ void bisect_start(const DerivTerms &D, float tmax,
+                                                      BisectState &S, int &steps)
+{
+    S.tl = 0.01f;
+    S.tu = tmax;
+    S.x = tmax;
+    S.itr = 0;
+    S.state = ST_TMAX;
+    const int up = deriv_sign(D, tmax);
+    if (up != kUnsure) {
+        ++steps;
+        S.state = up == kNeg ? ST_FIN : ST_LOW;
+        S.tl = up == kNeg ? tmax : 0.01f;
+        S.x = S.tl;
+    }
+    if (S.state == ST_LOW) {
+        const int low = deriv_sign(D, S.tl);
+        if (low == kNeg || low == kZero) {
+            ++steps;
+            S.state = ST_BIS;
+            S.x = (S.tu + S.tl) / 2.0f;
+        }
+    }
+    bool go = S.state == ST_BIS && S.tu <= kTMax;
+    for (int k = 0; k < 40 && go; ++k) {
+        float q;
+        go = deriv_sure(D, S.x, q);
+        if (go) {
+            S.tu = q > 0.0f ? S.x : S.tu;
+            S.tl = q > 0.0f ? S.tl : S.x;
+            S.x = (S.tu + S.tl) / 2.0f;
+            ++S.itr;
+        }
+    }
+    steps += S.itr;
+    // 2^-47 A(t) <= w (1 + t^4), as t <= 0.57 (1 + t^4) and t^2 <= 0.5 (1 + t^4)
+    const float mid = fmaf(0x1p23f * 0.57f, D.k1, 2.05f * D.n2);
+    const float w = 0x1p-47f * (mid + fmaxf(fmaf(0x1p23f, D.k0, fabsf(D.n0)), 2.0f * kK4));
+    S.w = (S.x >= kFastMin && S.tl >= kFastMin && S.tu <= kTMax) ? w : INFINITY;
+}
+
+// One further step from the costs ca, cb at the step's two points (ca alone
+// in ST_FIN).  dcost = (ca - cb) / h (2pBVP.cu:109-115) enters only through
+// its sign, which is that of dc = ca - cb, and through |dcost| > 0.0001,
+// which is |dc| >= kDcostBig.
+// A midpoint that leaves the bracket as it was is a fixed point: every later
+// step would evaluate the same x and do the same, up to the 50th, so the
+// bisection ends there with the same result; skipped is their number.
+__host__ __device__ __forceinline__ void bisect_update(BisectState &S, float ca, float cb,
+                                                       int &skipped)
+{
+    const float dc = ca - cb;
+    const bool pos = dc > 0.0f;
+    skipped = 0;
+    if (S.state == ST_BIS) {
+        const float tu = pos ? S.x : S.tu, tl = pos ? S.tl : S.x;
+        ++S.itr;
+        const bool go_on = fabsf(dc) >= kDcostBig && S.itr < 50;
+        const bool fixed = tu == S.tu && tl == S.tl;
+        skipped = go_on && fixed ? 50 - S.itr : 0;
+        S.tu = tu;
+        S.tl = tl;
+        S.state = go_on && !fixed ? ST_BIS : ST_FIN;
+        S.x = go_on && !fixed ? (tu + tl) / 2.0f : S.x;
+    } else if (S.state == ST_FIN) {
+        S.state = ST_DONE;
+    } else if (S.state == ST_TMAX) {
+        S.state = dc < 0.0f ? ST_FIN : ST_LOW;
+        S.x = dc < 0.0f ? S.x : S.tl;
+    } else if (pos && S.itr < 400) {
+        S.tl = S.tl / 2.0f;
+        S.x = S.tl;
+        ++S.itr;
+        if (!(S.tl >= kFastMin))
+            S.w = INFINITY;
+    } else {
+        S.state = ST_BIS;
+        S.itr = 0;
+        S.x = (S.tu + S.tl) / 2.0f;
+    }
+}
+
+// The step's two points and costs; false where a rounding is not settled
+// (the costs are cost_eval's at xa and xb then).
+__host__ __device__ __forceinline__ bool bisect_costs(const PairTerms &T, const BisectState &S,
+                                                      float &xa, float &xb, float &ca, float &cb)
+{
+    const float h = S.state == ST_FIN ? 0.0f : 0.000001f / 2.0f;
+    xa = S.x + h;
+    xb = S.x - h;
+    const double a = (double)xa, b = (double)xb;
+    double ra, rb;
+    recip_near(a * a * a, b * b * b, ra, rb);
+    const float x2 = S.x * S.x;
+    const double w = (double)fmaf(S.w, x2 * x2, S.w) * ra;
+    const bool oka = cost_certified(cost_fast(T, xa, ra), w, ca);
+    const bool okb = cost_certified(cost_fast(T, xb, rb), w, cb);
+    return oka && okb;
 }
 
 // ---------------------------------------------------------------------------

@@ -137,6 +137,54 @@ def test_host_bvp_arithmetic_matches_oracle():
     assert diff_t <= n * 1e-3 and diff_c <= n * 1e-3, (diff_t, diff_c)
 
 
+@pytest.mark.parametrize("kind", ["uniform", "close", "same", "large", "at_rest", "tmax", "zeros",
+                                  "coasting", "magnitudes", "non_finite"])
+def test_pair_bisection_matches_the_plain_one(kind):
+    """The pair pass's bisection (leading steps from the derivative's sign,
+    the rest from certified cost evaluations, fixed points cut short) gives
+    toptBisection's result and the cost bit for bit, also where its shortcuts
+    do not apply."""
+    rng = np.random.default_rng(11)
+    n, evals, plain = 4000, 0, 0
+    out, cost, steps = np.zeros(1, np.float32), np.zeros(1, np.float32), np.zeros(3, np.int32)
+    for _ in range(n):
+        a = np.concatenate([rng.uniform(0, 1, 3), rng.uniform(-0.5, 0.5, 3)]).astype(np.float32)
+        b = np.concatenate([rng.uniform(0, 1, 3), rng.uniform(-0.5, 0.5, 3)]).astype(np.float32)
+        tmax = np.float32(5)
+        if kind == "close":
+            b[:3] = a[:3] + rng.uniform(-1, 1, 3) * 10.0 ** rng.uniform(-6, -1)
+        elif kind == "same":
+            b = a.copy()
+        elif kind == "large":
+            a, b = a * np.float32(60) - 30, b * np.float32(60) - 30
+        elif kind == "at_rest":
+            a[3:] = b[3:] = 0
+        elif kind == "tmax":
+            tmax = np.float32(rng.choice([0.0, -1.0, 0.004, 0.01, 0.3, 16.0, 130.0, 1e9, np.inf,
+                                          np.nan, np.exp(rng.uniform(-6, 6))]))
+        elif kind == "zeros":
+            a[rng.random(6) < 0.5] = 0
+            b[rng.random(6) < 0.5] = -0.0
+        elif kind == "coasting":
+            b[:3] = a[:3] + a[3:] * np.float32(0.3)
+            b[3:] = a[3:] + rng.uniform(-1e-4, 1e-4, 3)
+        elif kind == "magnitudes":
+            a = np.ldexp(a, rng.integers(-40, 40, 6)).astype(np.float32)
+            b = np.ldexp(b, rng.integers(-40, 40, 6)).astype(np.float32)
+        elif kind == "non_finite":
+            a[rng.integers(6)] = rng.choice([np.inf, -np.inf, np.nan, 3e38, 1e-45])
+        P.lib.pump_host_pair(P.fp(a), P.fp(b), tmax, P.fp(out), P.fp(cost), P.ip(steps))
+        t = np.float32(P.lib.pump_host_topt(P.fp(a), P.fp(b), tmax))
+        c = np.float32(P.lib.pump_host_cost(t, P.fp(a), P.fp(b)))
+        same = [x.tobytes() == y.tobytes() or (np.isnan(x) and np.isnan(y))
+                for x, y in ((out[0], t), (cost[0], c))]
+        assert all(same), (kind, a, b, tmax, out, t, cost, c)
+        evals, plain = evals + steps[1], plain + steps[2]
+    if kind == "uniform":
+        # 12.3 steps with the final cost, about half of them evaluated
+        assert 5 * n < evals < 7 * n and plain < 0.01 * evals
+
+
 def test_host_find_optimal_path_matches_golden(golden_dir):
     g = np.load(os.path.join(golden_dir, "bvp_optimal_path.npz"))
     exact = 0
