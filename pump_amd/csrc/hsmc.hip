@@ -11,9 +11,9 @@
 // propagate + CP comes in three forms, all with the reference's particle
 // decisions (float order of PUMP.cu:645-651, no contraction; the AND over
 // (waypoint, half-space) pairs is order-independent), hence identical rows:
-//   * one wave per new path (the drop-in entry point and small wavefronts);
-//   * one workgroup per new path with the path's (waypoint, half-space)
-//     pairs staged in LDS (selected with PUMP_HSMC_KERNEL=block);
+//   * one workgroup per new path with the path's half-spaces staged in LDS
+//     (small wavefronts, and all with PUMP_HSMC_KERNEL=block);
+//   * 64 paths per wave (large wavefronts without a workspace);
 //   * the batched form for large wavefronts: classify, copy, and the
 //     time-binned half-space pass of hsmc_bins.hip.
 #include <algorithm>
@@ -344,115 +344,6 @@ __global__ __launch_bounds__(256) void k_setup_valid(uint8_t *__restrict__ valid
     }
 }
 
-// one (waypoint, half-space) entry of a path's edge
-struct HsEntry {
-    float a0, a1, a2, b;
-    int ti;
-};
-
-// Gather the entries of waypoints [i0, i1) of edge e into LDS; returns count.
-// Also counts time indices clamped into [0, tmax_steps).
-__device__ __forceinline__ int gather_entries(HsEntry *list, int *cnt, int i0, int i1, int64_t g0,
-                                              int max_hs, const float *__restrict__ as,
-                                              const float *__restrict__ bs, float tbase,
-                                              float dtl, float dt, int tmax_steps,
-                                              unsigned long long *clamped)
-{
-    if (threadIdx.x == 0)
-        *cnt = 0;
-    __syncthreads();
-    for (int i = i0 + (int)threadIdx.x; i < i1; i += blockDim.x) {
-        float time = tbase + (float)i * dtl;
-        int ti = (int)(time / dt);
-        bool any = false;
-        const int64_t head = (g0 + i) * (int64_t)max_hs;
-        for (int h = 0; h < max_hs; ++h) {
-            float b = bs[head + h];
-            if (b >= 1000.0f)
-                continue;
-            if (!any) {
-                any = true;
-                if (ti < 0 || ti >= tmax_steps) {
-                    if (clamped)
-                        atomicAdd(clamped, 1ull);
-                    ti = ti < 0 ? 0 : tmax_steps - 1;
-                }
-            }
-            int slot = atomicAdd(cnt, 1);
-            HsEntry en;
-            en.a0 = as[(head + h) * 3 + 0];
-            en.a1 = as[(head + h) * 3 + 1];
-            en.a2 = as[(head + h) * 3 + 2];
-            en.b = b;
-            en.ti = ti;
-            list[slot] = en;
-        }
-    }
-    __syncthreads();
-    return *cnt;
-}
-
-__device__ __forceinline__ bool particle_passes(const HsEntry &en, const float *__restrict__ off,
-                                                int n_mc, int p, float om)
-{
-    const float *o = off + ((int64_t)en.ti * n_mc + p) * 3;
-    return hs_pass(o[0], o[1], o[2], en.a0, en.a1, en.a2, om, en.b);
-}
-
-// Byte-validity propagate (+ optional fused CP).  Reads parent rows of
-// valid_src, writes child row dst_base+w of valid_dst.
-__global__ __launch_bounds__(256) void k_propagate(
-    int n_new, const int64_t *__restrict__ wp_offsets, int w_fixed,
-    const int *__restrict__ wf_edge, const int *__restrict__ wf_prev,
-    const float *__restrict__ as, const float *__restrict__ bs, const float *__restrict__ times,
-    const float *__restrict__ topts, float dt, int max_hs, const float *__restrict__ offsets_time,
-    int tmax_steps, float om, int n_mc, const uint8_t *__restrict__ valid_src,
-    uint8_t *__restrict__ valid_dst, int64_t dst_base, int n_p, float *__restrict__ path_cp,
-    int64_t cp_base, unsigned long long *__restrict__ clamped)
-{
-    __shared__ HsEntry list[kListCap];
-    __shared__ int cnt;
-    __shared__ int red[4];
-    const int w = blockIdx.x;
-    const int e = wf_edge[w];
-    const int prev = wf_prev[w];
-    const int64_t g0 = wp_offsets ? wp_offsets[e] : (int64_t)e * w_fixed;
-    const int W = (int)((wp_offsets ? wp_offsets[e + 1] : g0 + w_fixed) - g0);
-    const float dtl = topts[e] / (float)(W - 1);
-    const float tbase = times[prev];
-    const uint8_t *src = valid_src + (int64_t)prev * n_p;
-    uint8_t *dst = valid_dst + (dst_base + w) * (int64_t)n_p;
-    const int chunk = max_hs > 0 ? (kListCap / max_hs) : W;
-
-    int invalid = 0;
-    for (int i0 = 0; i0 < W; i0 += chunk) {
-        const int i1 = i0 + chunk < W ? i0 + chunk : W;
-        const int n = gather_entries(list, &cnt, i0, i1, g0, max_hs, as, bs, tbase, dtl, dt,
-                                     tmax_steps, clamped);
-        const bool last = i1 >= W;
-        const uint8_t *in = (i0 == 0) ? src : dst;
-        for (int p = threadIdx.x; p < n_p; p += blockDim.x) {
-            bool v = in[p] != 0;
-            for (int q = 0; q < n && v; ++q)
-                v = particle_passes(list[q], offsets_time, n_mc, p, om);
-            dst[p] = v ? 1 : 0;
-            if (last)
-                invalid += v ? 0 : 1;
-        }
-        __syncthreads();
-    }
-    if (path_cp) {
-        for (int off = 32; off > 0; off >>= 1)
-            invalid += __shfl_down(invalid, off, 64);
-        if ((threadIdx.x & 63) == 0)
-            red[threadIdx.x >> 6] = invalid;
-        __syncthreads();
-        if (threadIdx.x == 0)
-            path_cp[cp_base + w] = ((float)(red[0] + red[1] + red[2] + red[3])) / (float)n_p;
-    }
-}
-
-// calculateCP_HSMC: one workgroup per path
 // calculateCP_HSMC: one wave per path (grid-stride), 16-byte loads
 __global__ __launch_bounds__(256) void k_cp(int n_new, int64_t base, float *__restrict__ cp,
                                             const uint8_t *__restrict__ valid, int n_p)
@@ -488,71 +379,6 @@ __global__ __launch_bounds__(256) void k_gather_rows(const uint8_t *__restrict__
 }
 
 // ---------------------------------------------------------------------------
-// Bit-mask validity (chosen form): one wave handles 64 particles per step;
-// the parent word is a uniform load and the child word is the ballot of the
-// lanes' decisions.
-__global__ __launch_bounds__(256) void k_propagate_bits(
-    int n_new, const int64_t *__restrict__ wp_offsets, int w_fixed,
-    const int *__restrict__ wf_edge, const int *__restrict__ wf_prev,
-    const float *__restrict__ as, const float *__restrict__ bs, const float *__restrict__ times,
-    const float *__restrict__ topts, float dt, int max_hs, const float *__restrict__ offsets_time,
-    int tmax_steps, float om, int n_mc, const uint64_t *__restrict__ valid_src,
-    uint64_t *__restrict__ valid_dst, int64_t dst_base, int n_p, float *__restrict__ path_cp,
-    int64_t cp_base, unsigned long long *__restrict__ clamped)
-{
-    __shared__ HsEntry list[kListCap];
-    __shared__ int cnt;
-    __shared__ int red[4];
-    const int w = blockIdx.x;
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const int e = wf_edge[w];
-    const int prev = wf_prev[w];
-    const int64_t g0 = wp_offsets ? wp_offsets[e] : (int64_t)e * w_fixed;
-    const int W = (int)((wp_offsets ? wp_offsets[e + 1] : g0 + w_fixed) - g0);
-    const float dtl = topts[e] / (float)(W - 1);
-    const float tbase = times[prev];
-    const int nwords = (n_p + 63) / 64;
-    const uint64_t *src = valid_src + (int64_t)prev * nwords;
-    uint64_t *dst = valid_dst + (dst_base + w) * (int64_t)nwords;
-    const int chunk = max_hs > 0 ? (kListCap / max_hs) : W;
-
-    int valid_count = 0;
-    for (int i0 = 0; i0 < W; i0 += chunk) {
-        const int i1 = i0 + chunk < W ? i0 + chunk : W;
-        const int n = gather_entries(list, &cnt, i0, i1, g0, max_hs, as, bs, tbase, dtl, dt,
-                                     tmax_steps, clamped);
-        const bool last = i1 >= W;
-        const uint64_t *in = (i0 == 0) ? src : dst;
-        for (int wd = wid; wd < nwords; wd += 4) {
-            const uint64_t word = in[wd];
-            const int p = wd * 64 + lane;
-            bool v = (p < n_p) && ((word >> lane) & 1ull);
-            if (__ballot(v) != 0ull) {
-                for (int q = 0; q < n; ++q) {
-                    if (v)
-                        v = particle_passes(list[q], offsets_time, n_mc, p, om);
-                }
-            }
-            const uint64_t out = __ballot(v);
-            if (lane == 0)
-                dst[wd] = out;
-            if (last)
-                valid_count += (lane == 0) ? __popcll(out) : 0;
-        }
-        __syncthreads();
-    }
-    if (path_cp) {
-        if (lane == 0)
-            red[wid] = valid_count;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            int valid_all = red[0] + red[1] + red[2] + red[3];
-            path_cp[cp_base + w] = ((float)(n_p - valid_all)) / (float)n_p;
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------
 // Wave-level forms of propagate + CP.  A wave first marks, per group of 64
 // waypoints, the waypoints that hold at least one stored half-space (b <
 // 1000): from the edge's waypoint mask when one is given (bit k: waypoint k,
@@ -560,9 +386,7 @@ __global__ __launch_bounds__(256) void k_propagate_bits(
 // streamed 64 at a time (lane = particle) and tested only against those
 // waypoints' half-spaces, whose data are wave-uniform loads.  Decisions use
 // the reference's float order.  No LDS, no workgroup barriers.
-// One wave per new path (single launch; small wavefronts).
-// One path's propagate + CP by one wave (the body of the wave-per-path
-// forms): marked waypoints from the edge's summary or from bs, particles 64 at
+// One path's propagate + CP by one wave (64 paths per wave, the listed ones): marked waypoints from the edge's summary or from bs, particles 64 at
 // a time, the child row written in full, the CP from its final count.
 template <bool kBits>
 __device__ __forceinline__ void propagate_path(
@@ -687,29 +511,6 @@ __device__ __forceinline__ void propagate_path(
     if (path_cp && lane == 0) {
         const int invalid = kBits ? n_p - count : count;
         path_cp[cp_base + w] = ((float)invalid) / (float)n_p;
-    }
-}
-
-// One wave per new path (single launch; small wavefronts).
-template <bool kBits>
-__global__ __launch_bounds__(256) void k_propagate_wave(
-    int n_new, const int64_t *__restrict__ wp_offsets, int w_fixed,
-    const int *__restrict__ wf_edge, const int *__restrict__ wf_prev,
-    const float *__restrict__ as, const float *__restrict__ bs,
-    const uint64_t *__restrict__ edge_mask, const float *__restrict__ times,
-    const float *__restrict__ topts, float dt, int max_hs, const float *__restrict__ offsets_time,
-    int tmax_steps, float om, int n_mc, const void *__restrict__ valid_src,
-    void *__restrict__ valid_dst, int64_t dst_base, int n_p, float *__restrict__ path_cp,
-    int64_t cp_base, unsigned long long *__restrict__ clamped)
-{
-    const int64_t n_waves = (int64_t)gridDim.x * (blockDim.x >> 6);
-    for (int64_t w = wave_index(); w < n_new; w += n_waves) {
-        const int e = wf_edge[w];
-        const int prev = wf_prev[w];
-        const PathInfo pi = path_info(e, prev, wp_offsets, w_fixed, topts, times);
-        propagate_path<kBits>(w, e, prev, pi, as, bs, edge_mask, dt, max_hs, offsets_time,
-                              tmax_steps, om, n_mc, valid_src, valid_dst, dst_base, n_p, path_cp,
-                              cp_base, clamped);
     }
 }
 
@@ -940,6 +741,195 @@ __global__ __launch_bounds__(256) void k_copy_rows(int n_new, const int *__restr
                 const int invalid = kBits ? n_p - count[r] : count[r];
                 path_cp[cp_base + w[r]] = ((float)invalid) / (float)n_p;
             }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// One workgroup per new path (small wavefronts, and PUMP_HSMC_KERNEL=block).
+// With few paths the chip has waves to spare and what counts is the length
+// of a path's dependent loads, so the path's edge is read by all lanes at once
+// (a slot each: the live half-spaces go to an LDS list in slot order) and its
+// particles are spread over the waves, kWalk groups of 64 each; a wave takes
+// the list kBatch half-spaces at a time, all their offsets in flight
+// together.  Against 64 paths per wave one after another: 207 paths of 2000
+// particles (bit rows) in a cluttered world 116 -> 9 us, 778 of 1195 (byte
+// rows, no edge summary, with the CP count) 250 -> 16 us.
+// ---------------------------------------------------------------------------
+constexpr int kWalk = 4;
+constexpr int kBatch = 4;
+constexpr int kPathBlock = 256; // 512 is no faster below 1000 paths and twice as slow at 16384
+
+template <bool kBits>
+__global__ __launch_bounds__(kPathBlock) void k_propagate_path(
+    const int64_t *__restrict__ wp_offsets, int w_fixed, const int *__restrict__ wf_edge,
+    const int *__restrict__ wf_prev, const float *__restrict__ as, const float *__restrict__ bs,
+    const uint64_t *__restrict__ edge_mask, const float *__restrict__ times,
+    const float *__restrict__ topts, float dt, int max_hs, const float *__restrict__ offsets_time,
+    int tmax_steps, float om, int n_mc, const void *valid_src, void *valid_dst, int64_t dst_base,
+    int n_p, float *__restrict__ path_cp, int64_t cp_base,
+    unsigned long long *__restrict__ clamped, int *__restrict__ row_src)
+{
+    constexpr int kWaves = kPathBlock / 64;
+    __shared__ float4 list[kListCap]; // a, b
+    __shared__ int list_ti[kListCap];
+    __shared__ int wave_cnt[kWaves], red[kWaves];
+    const int w = blockIdx.x;
+    const int t = threadIdx.x, lane = t & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int e = wf_edge[w], prev = wf_prev[w];
+    const uint64_t em = edge_mask ? edge_mask[e] : ~0ull;
+    const PathInfo pi = path_info(e, prev, wp_offsets, w_fixed, topts, times);
+    const bool exact = edge_mask && mask_exact(em, pi.W);
+    const int n_groups = (n_p + 63) >> 6;
+    const int64_t row_bytes = kBits ? (int64_t)n_groups * 8 : (int64_t)n_p;
+    const uint8_t *src = (const uint8_t *)valid_src + prev * row_bytes;
+    uint8_t *dst = (uint8_t *)valid_dst + (dst_base + w) * row_bytes;
+    // waypoints per pass: their slots fit the list (max_hs <= kListCap)
+    const int chunk = max_hs > 0 ? kListCap / max_hs : pi.W;
+    int count = 0; // valid (bits) or invalid (bytes) particles, per lane
+    for (int i0 = 0; i0 < pi.W; i0 += chunk) {
+        const int i1 = i0 + chunk < pi.W ? i0 + chunk : pi.W;
+        const bool last = i1 >= pi.W;
+        const uint8_t *in = i0 == 0 ? src : dst;
+        const int64_t head = (pi.g0 + i0) * max_hs; // slot 0 of waypoint i0
+        int n = 0;
+        const auto marked = [&](int i) { return !exact || (i < 64 && ((em >> i) & 1ull)); };
+        const int s_end = exact && mask_bits(em, pi.W) == 0ull ? 0 : (i1 - i0) * max_hs;
+        for (int s0 = 0; s0 < s_end; s0 += kPathBlock) {
+            const int sl = s0 + t;
+            const int i = i0 + sl / max_hs;
+            float b = 1111.0f, a0 = 0.0f, a1 = 0.0f, a2 = 0.0f;
+            if (sl < s_end && marked(i)) {
+                b = bs[head + sl];
+                a0 = as[(head + sl) * 3 + 0];
+                a1 = as[(head + sl) * 3 + 1];
+                a2 = as[(head + sl) * 3 + 2];
+            }
+            // the reference skips slots with b >= 1000 (PUMP.cu:642)
+            const bool live = !(b >= 1000.0f);
+            const uint64_t m = __ballot(live);
+            if (lane == 0)
+                wave_cnt[wid] = __popcll(m);
+            __syncthreads();
+            int at = n + __popcll(m & ((1ull << lane) - 1ull));
+            for (int k = 0; k < kWaves; ++k) {
+                at += k < wid ? wave_cnt[k] : 0;
+                n += wave_cnt[k];
+            }
+            if (live) {
+                list[at] = make_float4(a0, a1, a2, b);
+                list_ti[at] = clamp_time(time_index(pi, i, dt), tmax_steps);
+            }
+            __syncthreads();
+        }
+        // waypoints that store a half-space and whose time index is clamped
+        if (clamped)
+            for (int i = i0 + t; i < i1; i += kPathBlock)
+                if (time_clamped(pi, i, dt, tmax_steps) && marked(i) &&
+                    waypoint_has_hs(bs, (pi.g0 + i) * (int64_t)max_hs, max_hs))
+                    atomicAdd(clamped, 1ull);
+        if (n == 0) {
+            // a copy of the parent's row
+            const bool wide = (row_bytes & 15) == 0 &&
+                              ((((uintptr_t)in) | ((uintptr_t)dst)) & 15) == 0;
+            if (wide) {
+                const uint4 *s16 = (const uint4 *)in;
+                uint4 *d16 = (uint4 *)dst;
+                for (int q = t; q < (int)(row_bytes >> 4); q += kPathBlock) {
+                    uint4 x = s16[q];
+                    const int c = copy_count<kBits>(x);
+                    if (i0 == 0)
+                        d16[q] = x;
+                    count += last ? c : 0;
+                }
+            } else if (kBits) {
+                for (int q = t; q < n_groups; q += kPathBlock) {
+                    uint64_t x = ((const uint64_t *)in)[q];
+                    if (i0 == 0)
+                        ((uint64_t *)dst)[q] = x;
+                    count += last ? __popcll(x) : 0;
+                }
+            } else {
+                for (int q = t; q < n_p; q += kPathBlock) {
+                    const uint8_t x = in[q] ? 1 : 0;
+                    if (i0 == 0)
+                        dst[q] = x;
+                    count += last ? 1 - x : 0;
+                }
+            }
+        } else {
+            for (int g0 = wid * kWalk; g0 < n_groups; g0 += kWaves * kWalk) {
+                bool v[kWalk];
+                int p[kWalk];
+#pragma unroll
+                for (int q = 0; q < kWalk; ++q) {
+                    p[q] = (g0 + q) * 64 + lane;
+                    if (kBits) {
+                        const uint64_t word =
+                            g0 + q < n_groups ? ((const uint64_t *)in)[g0 + q] : 0ull;
+                        v[q] = p[q] < n_p && ((word >> lane) & 1ull);
+                    } else {
+                        v[q] = p[q] < n_p && in[p[q]] != 0;
+                    }
+                }
+                for (int k = 0; k < n; k += kBatch) {
+                    float o[kBatch][kWalk][3];
+                    float4 h[kBatch];
+#pragma unroll
+                    for (int u = 0; u < kBatch; ++u) {
+                        // past the end: the last entry again
+                        const int at = k + u < n ? k + u : n - 1;
+                        h[u] = list[at];
+                        const float *row = offsets_time + (int64_t)list_ti[at] * n_mc * 3;
+#pragma unroll
+                        for (int q = 0; q < kWalk; ++q) {
+                            // n_p <= n_mc: in bounds whatever the particle's validity
+                            const float *op = row + (p[q] < n_p ? p[q] : 0) * 3;
+                            o[u][q][0] = op[0];
+                            o[u][q][1] = op[1];
+                            o[u][q][2] = op[2];
+                        }
+                    }
+#pragma unroll
+                    for (int u = 0; u < kBatch; ++u)
+#pragma unroll
+                        for (int q = 0; q < kWalk; ++q)
+                            v[q] = hs_pass(o[u][q][0], o[u][q][1], o[u][q][2], h[u].x, h[u].y,
+                                           h[u].z, om, h[u].w) &&
+                                   v[q];
+                }
+#pragma unroll
+                for (int q = 0; q < kWalk; ++q) {
+                    if (kBits) {
+                        const uint64_t out = __ballot(v[q]);
+                        if (lane == q && g0 + q < n_groups) {
+                            ((uint64_t *)dst)[g0 + q] = out;
+                            count += last ? __popcll(out) : 0;
+                        }
+                    } else if (p[q] < n_p) {
+                        dst[p[q]] = v[q] ? 1 : 0;
+                        count += last && !v[q] ? 1 : 0;
+                    }
+                }
+            }
+        }
+        if (!last)
+            __syncthreads(); // the row is read back and the list reused
+    }
+    if (row_src && t == 0)
+        row_src[w] = w;
+    if (path_cp) {
+        count = wave_sum(count);
+        if (lane == 0)
+            red[wid] = count;
+        __syncthreads();
+        if (t == 0) {
+            int total = 0;
+            for (int k = 0; k < kWaves; ++k)
+                total += red[k];
+            const int invalid = kBits ? n_p - total : total;
+            path_cp[cp_base + w] = ((float)invalid) / (float)n_p;
         }
     }
 }
@@ -1302,9 +1292,7 @@ extern "C" int pump_setup_valid_particles(uint8_t *d_valid, int n_p, int64_t max
     return PUMP_OK;
 }
 
-// Propagate kernel selection: the wave-per-path kernel (default) or the
-// workgroup-per-path kernel with an LDS list (PUMP_HSMC_KERNEL=block), which
-// suits edges that store many half-spaces.
+// PUMP_HSMC_KERNEL=block selects the workgroup-per-path form for every size.
 static bool use_block_kernel()
 {
     static int v = -1;
@@ -1347,6 +1335,31 @@ static unsigned wave_blocks_for(int64_t waves)
     const int64_t blocks = (waves + 3) / 4;
     return (unsigned)(blocks < 1 ? 1 : (blocks < cap ? blocks : cap));
 }
+
+template <bool kBits>
+static int launch_path(int n_new, const int64_t *wp_offsets, int W_fixed, const int *wf_edge,
+                       const int *wf_prev, const float *as, const float *bs,
+                       const uint64_t *edge_mask, const float *times, const float *topts, float dt,
+                       int max_hs, const float *offsets_time, int tmax_steps, float om, int n_mc,
+                       const void *src, void *dst, int64_t dst_base, int n_p, float *path_cp,
+                       int64_t cp_base, unsigned long long *clamped, int *row_src, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_propagate_path<kBits>, dim3(n_new), dim3(kPathBlock), 0, s, wp_offsets,
+                       W_fixed, wf_edge, wf_prev, as, bs, edge_mask, times, topts, dt, max_hs,
+                       offsets_time, tmax_steps, om, n_mc, src, dst, dst_base, n_p, path_cp,
+                       cp_base, clamped, row_src);
+    PUMP_LAUNCHED();
+    return PUMP_OK;
+}
+
+// The batched form runs from kBatchedMin paths on where it has a workspace.
+// Otherwise a workgroup per path below kPathFormMax paths and 64 paths per
+// wave above: 2000 particles in bit rows take 8 against 70-107 us at 500
+// paths, 40-46 against 78-264 at 16384 and 72-87 against 87-300 at 32768 (few
+// and many boxes), where the launch of the workgroups (2 ns each) decides;
+// at 65536 paths few boxes favour the waves.
+constexpr int kPathFormMax = 32768;
+constexpr int kBatchedMin = 4096;
 
 // The 64-paths-per-wave propagate: its copy unit and grid
 template <bool kBits>
@@ -1397,7 +1410,7 @@ extern "C" int pump_propagate_valid_particles(
     PUMP_REQUIRE(d_wf_edge && d_wf_prev && d_as && d_bs && d_times && d_topts && d_offsets_time &&
                  d_valid);
     hipStream_t s = as_stream(stream);
-    if (num_new_paths >= 4096 && !use_block_kernel()) {
+    if (num_new_paths >= kBatchedMin && !use_block_kernel()) {
         // A large wavefront runs the batched form in place (classify, row
         // copies, time-binned half-space tests) with a workspace from the
         // stream-ordered pool, released on the same stream; the reference
@@ -1420,21 +1433,18 @@ extern "C" int pump_propagate_valid_particles(
         }
         (void)hipGetLastError(); // the failed request is not an error of this call
     }
-    if (use_block_kernel())
-        hipLaunchKernelGGL(k_propagate, dim3(num_new_paths), dim3(256), 0, as_stream(stream),
-                           num_new_paths, d_wp_offsets, waypoints_count, d_wf_edge, d_wf_prev,
-                           d_as, d_bs, d_times, d_topts, dt, max_hs, d_offsets_time, tmax_steps,
-                           offset_mult, num_mc_particles, d_valid, d_valid, path_base, n_p,
-                           (float *)nullptr, (int64_t)0, d_clamped);
-    else
-        return launch_b64<false>(num_new_paths, d_wp_offsets, waypoints_count, d_wf_edge,
-                                 d_wf_prev, d_as, d_bs, (const uint64_t *)nullptr, d_times,
-                                 d_topts, dt, max_hs, d_offsets_time, tmax_steps, offset_mult,
-                                 num_mc_particles, (const void *)d_valid, (void *)d_valid,
-                                 path_base, n_p, (float *)nullptr, (int64_t)0, d_clamped,
-                                 as_stream(stream));
-    PUMP_LAUNCHED();
-    return PUMP_OK;
+    if (num_new_paths < kPathFormMax || use_block_kernel())
+        return launch_path<false>(num_new_paths, d_wp_offsets, waypoints_count, d_wf_edge,
+                                  d_wf_prev, d_as, d_bs, (const uint64_t *)nullptr, d_times,
+                                  d_topts, dt, max_hs, d_offsets_time, tmax_steps, offset_mult,
+                                  num_mc_particles, (const void *)d_valid, (void *)d_valid,
+                                  path_base, n_p, (float *)nullptr, (int64_t)0, d_clamped,
+                                  (int *)nullptr, s);
+    return launch_b64<false>(num_new_paths, d_wp_offsets, waypoints_count, d_wf_edge, d_wf_prev,
+                             d_as, d_bs, (const uint64_t *)nullptr, d_times, d_topts, dt, max_hs,
+                             d_offsets_time, tmax_steps, offset_mult, num_mc_particles,
+                             (const void *)d_valid, (void *)d_valid, path_base, n_p,
+                             (float *)nullptr, (int64_t)0, d_clamped, s);
 }
 
 extern "C" int pump_calculate_cp_hsmc(int num_new_paths, int64_t path_base, float *d_path_cp,
@@ -1548,8 +1558,8 @@ static int ppw_groups(bool bits, bool split, int n_p, int max_hs)
 }
 
 // Launches the propagate + CP step for a wavefront: the batched form when a
-// workspace is given and the wavefront is large, else one wave-per-path (or,
-// on request, workgroup-per-path) launch.
+// workspace is given and the wavefront is large, else the workgroup-per-path
+// or the 64-paths-per-wave form.
 template <bool kBits>
 static int launch_propagate(int n_new, int W_fixed, const int64_t *wp_offsets, const int *wf_edge,
                             const int *wf_prev, const float *as, const float *bs,
@@ -1563,7 +1573,7 @@ static int launch_propagate(int n_new, int W_fixed, const int64_t *wp_offsets, c
 {
     const int64_t row_bytes = kBits ? (int64_t)((n_p + 63) / 64) * 8 : (int64_t)n_p;
     const BatchLayout L = BatchLayout::fill(n_new, tmax_steps, ws ? ws_bytes : 0);
-    if (ws && ws_bytes >= L.total && n_new >= 4096 && !use_block_kernel()) {
+    if (ws && ws_bytes >= L.total && n_new >= kBatchedMin && !use_block_kernel()) {
         uint8_t *base = reinterpret_cast<uint8_t *>(ws);
         int *ctl = reinterpret_cast<int *>(base);
         int *hist = reinterpret_cast<int *>(base + L.hist);
@@ -1671,25 +1681,15 @@ static int launch_propagate(int n_new, int W_fixed, const int64_t *wp_offsets, c
         PUMP_LAUNCHED();
         return bins_finish(B, kBits, s);
     }
-    if (use_block_kernel()) {
-        if (kBits)
-            hipLaunchKernelGGL(k_propagate_bits, dim3(n_new), dim3(256), 0, s, n_new, wp_offsets,
-                               W_fixed, wf_edge, wf_prev, as, bs, times, topts, dt, max_hs,
-                               offsets_time, tmax_steps, om, n_mc, (const uint64_t *)src,
-                               (uint64_t *)dst, dst_base, n_p, path_cp, cp_base, clamped);
-        else
-            hipLaunchKernelGGL(k_propagate, dim3(n_new), dim3(256), 0, s, n_new, wp_offsets,
-                               W_fixed, wf_edge, wf_prev, as, bs, times, topts, dt, max_hs,
-                               offsets_time, tmax_steps, om, n_mc, (const uint8_t *)src,
-                               (uint8_t *)dst, dst_base, n_p, path_cp, cp_base, clamped);
-        PUMP_LAUNCHED();
-    } else {
-        int r = launch_b64<kBits>(n_new, wp_offsets, W_fixed, wf_edge, wf_prev, as, bs, edge_mask,
+    if (n_new < kPathFormMax || use_block_kernel())
+        return launch_path<kBits>(n_new, wp_offsets, W_fixed, wf_edge, wf_prev, as, bs, edge_mask,
                                   times, topts, dt, max_hs, offsets_time, tmax_steps, om, n_mc,
-                                  src, dst, dst_base, n_p, path_cp, cp_base, clamped, s);
-        if (r)
-            return r;
-    }
+                                  src, dst, dst_base, n_p, path_cp, cp_base, clamped, row_src, s);
+    int r = launch_b64<kBits>(n_new, wp_offsets, W_fixed, wf_edge, wf_prev, as, bs, edge_mask,
+                              times, topts, dt, max_hs, offsets_time, tmax_steps, om, n_mc, src,
+                              dst, dst_base, n_p, path_cp, cp_base, clamped, s);
+    if (r)
+        return r;
     if (row_src) { // every child row was written
         hipLaunchKernelGGL(k_row_src_iota, dim3(grid_for(n_new, 256, 4096)), dim3(256), 0, s, n_new,
                            row_src);

@@ -1,0 +1,66 @@
+"""The workgroup-per-path form of the HSMC step (small wavefronts) against the
+oracle at the edges of its loops: particle counts around the groups of 64 and
+the waves' share, edges longer than a 64-bit summary, slot counts that need
+several passes of the half-space list, rows with and without half-spaces."""
+import numpy as np
+import pytest
+
+import pump_amd as P
+
+from test_gpu_parity import (dev, edge_mask_host, host, oracle_propagate, pack_bits, ptr,
+                             random_hsmc_inputs, unpack_bits)
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n_p,w_range,max_hs,n_new", [
+    (1, (2, 6), 1, 40), (63, (2, 40), 5, 40), (64, (2, 40), 5, 40), (65, (2, 40), 5, 40),
+    (1024, (2, 20), 5, 40), (1025, (2, 20), 5, 300), (2000, (60, 70), 5, 40),
+    (130, (64, 65), 3, 40), (320, (200, 230), 5, 20), (96, (2, 9), 700, 12),
+    (96, (2, 9), 1024, 12), (272, (3, 4), 5, 4095)])
+def test_path_form_against_oracle(n_p, w_range, max_hs, n_new):
+    d = random_hsmc_inputs(n_p + max_hs, n_edges=80, max_hs=max_hs, n_p=n_p, n_mc=n_p + 3, T=70,
+                           n_new=n_new, n_parent=9, variable=True, w_range=w_range)
+    # a third of the edges store nothing, some only in their last waypoint
+    for e in range(0, 80, 3):
+        lo, hi = d["off"][e] * max_hs, d["off"][e + 1] * max_hs
+        d["bs"][lo: hi - (max_hs if e % 2 else 0)] = 1111
+    # a NaN slot is a stored half-space that no particle passes; the oracle's
+    # clamp (b < 1000) leaves it out, so its edge is kept inside the table
+    d["bs"][5] = np.nan
+    nan_edge = int(np.searchsorted(d["off"] * max_hs, 5, side="right")) - 1
+    d["wf_edge"][0] = nan_edge
+    d["times"][0] = 0.5
+    d["wf_prev"][d["wf_edge"] == nan_edge] = 0
+    ref_v, ref_cp, ref_cl = oracle_propagate(d)
+    npar = d["n_parent"]
+    g = {k: dev(d[k]) for k in ("off", "as_", "bs", "offs", "topts", "times", "wf_edge",
+                                 "wf_prev")}
+    g_mask = dev(edge_mask_host(d["off"], d["bs"], max_hs))
+    edges = (n_new, 0, ptr(g["off"]), ptr(g["wf_edge"]), ptr(g["wf_prev"]))
+    table = (ptr(g["times"]), ptr(g["topts"]), d["dt"], max_hs, ptr(g["offs"]), d["T"], d["om"],
+             d["n_mc"])
+    print("path form", n_p, w_range, max_hs, n_new, flush=True)
+    # the drop-in call, children after their parents in one array
+    valid, clamp = dev(d["valid"]), dev(np.zeros(1, np.uint64))
+    P.check("propagate", P.lib.pump_propagate_valid_particles(
+        *edges, npar, ptr(g["as_"]), ptr(g["bs"]), None, *table, ptr(valid), n_p, ptr(clamp),
+        None))
+    assert np.array_equal(host(valid), ref_v) and int(host(clamp)[0]) == ref_cl
+    for bits in (0, 1):
+        width = (n_p + 63) // 64 * 8 if bits else n_p
+        src = dev(pack_bits(d["valid"][:npar], n_p) if bits else d["valid"][:npar])
+        for mask in (None, g_mask.p):
+            dst = dev(np.full((n_new + 1, width), 0x5a, np.uint8))
+            cp, clamp = dev(np.zeros(n_new + 2, np.float32)), dev(np.zeros(1, np.uint64))
+            row_src, pcp = dev(np.full(n_new, -7, np.int32)), dev(np.zeros(npar, np.float32))
+            P.check("propagate_cp_cow", P.lib.pump_propagate_cp_cow(
+                bits, *edges, ptr(g["as_"]), ptr(g["bs"]), mask, *table, ptr(src), ptr(pcp),
+                ptr(dst), 1, ptr(row_src), n_p, ptr(cp), 2, 0, None, None, ptr(clamp), None, 0,
+                None))
+            rows = host(dst)
+            assert (rows[0] == 0x5a).all() and int(host(clamp)[0]) == ref_cl
+            got = unpack_bits(rows[1:].copy().view(np.uint64), n_p) if bits else rows[1:]
+            assert np.array_equal(got, ref_v[npar:]), (bits, mask is None)
+            assert np.array_equal(host(cp)[2:], ref_cp[npar:])
+            assert np.array_equal(host(row_src), np.arange(n_new))
