@@ -2,12 +2,17 @@
 // collisionProbability + MCCP, collisionProbability.cu:4-92).
 //
 // The reference runs one thread per particle in 32 workgroups of 64 and walks
-// the path's segments serially.  Here one wave owns one particle and its 64
-// lanes test 64 consecutive segments at once (the particle's noise row is
-// contiguous in t, so the loads coalesce); a wave ballot ends the particle at
-// the first blocked segment.  Obstacles are staged in LDS, and each lane
-// tests only the boxes that meet the union of the wave's 64 segment boxes.  Paths of a batch
-// are the grid's y dimension, so many candidate paths share one launch.
+// the path's segments serially.  Here a workgroup owns 64 particles of one
+// path, one per lane of each of its waves, and the waves share the path's
+// segments.  At one segment the 64 particles lie within the noise of one
+// another, so few boxes meet the union of their segment boxes and only those
+// are tested lane by lane; the boxes are tested against the union 64 at a
+// time, from registers.  (Lanes over the segments of one particle had the
+// whole path's extent as union, and idle lanes past its end: 64 paths of 4096
+// particles among 200 walls, 43 segments each, took 197 us, 5.7e10
+// segment-checks/s, and take 40 us, 2.8e11.)  Bound: VALU issue, about a
+// third of it the bounds' reductions; the noise rows are read a lane each,
+// uncoalesced, from L2.  Paths of a batch are the grid's y dimension.
 #include "pump_device.hpp"
 #include "pump_internal.hpp"
 
@@ -16,20 +21,27 @@
 namespace pump {
 namespace {
 
-__global__ __launch_bounds__(256) void k_mccp(const float *__restrict__ obstacles, int n_obs,
-                                              const float *__restrict__ xcomb, int tmax_steps,
-                                              int n_mc, float om, const float *__restrict__ paths,
-                                              int64_t stride_rows, const int *__restrict__ Ts,
-                                              int *__restrict__ hits)
+constexpr int kMaxWaves = 16; // waves of a workgroup at most
+// Waves of a launch, where the path count and particles leave fewer: 4096,
+// 8192, 16384, 32768 give 60, 57, 54, 60 us for 64 paths of 4096 particles
+// among 200 walls and about the same elsewhere.
+constexpr int kTargetWaves = 16384;
+
+// kBoxes: boxes per lane held in registers (0: any count, from LDS or global
+// memory).
+template <int kBoxes>
+__global__ __launch_bounds__(64 * kMaxWaves) void k_mccp(
+    const float *__restrict__ obstacles, int n_obs, const float *__restrict__ xcomb,
+    int tmax_steps, int n_mc, float om, const float *__restrict__ paths, int64_t stride_rows,
+    const int *__restrict__ Ts, int *__restrict__ hits)
 {
-    __shared__ ObsLds o;
-    stage_obstacles(o, obstacles, n_obs);
-    __syncthreads();
+    __shared__ unsigned long long hit_mask[kMaxWaves];
     const int k = blockIdx.y;
     const int lane = threadIdx.x & 63;
-    const int p = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (p >= n_mc)
-        return;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n_waves = blockDim.x >> 6;
+    const int first = blockIdx.x * 64;
+    const int p = first + lane < n_mc ? first + lane : n_mc - 1; // idle lanes repeat the last
     const float *path = paths + (int64_t)k * stride_rows * kDim;
     // segments t < T-2 (the reference skips the final segment); bounded by
     // the noise table and the path buffer
@@ -38,53 +50,119 @@ __global__ __launch_bounds__(256) void k_mccp(const float *__restrict__ obstacle
         nseg = tmax_steps - 1;
     if (nseg > (int)stride_rows - 1)
         nseg = (int)stride_rows - 1;
-    const float *xc = xcomb + (int64_t)p * 3 * tmax_steps;
-    for (int t0 = 0; t0 < nseg; t0 += 64) {
-        const int t = t0 + lane;
-        const bool act = t < nseg;
-        float v[3] = {0, 0, 0}, w[3] = {0, 0, 0};
-        float bmin[3] = {INFINITY, INFINITY, INFINITY}, bmax[3] = {-INFINITY, -INFINITY, -INFINITY};
-        if (act) {
+    const int chunk = (nseg + n_waves - 1) / n_waves;
+    const int t0 = wid * chunk, t1 = t0 + chunk < nseg ? t0 + chunk : nseg;
+    // this lane's boxes: lane, lane + 64, ...
+    constexpr int kRegs = kBoxes > 0 ? kBoxes : 1;
+    float blo[kRegs][3], bhi[kRegs][3];
+    if (kBoxes > 0) {
+#pragma unroll
+        for (int c = 0; c < kRegs; ++c) {
+            const int b = c * 64 + lane;
             for (int d = 0; d < 3; ++d) {
-                v[d] = path[t * kDim + d] + xc[t * 3 + d] * om;
-                w[d] = path[(t + 1) * kDim + d] + xc[(t + 1) * 3 + d] * om;
+                blo[c][d] = b < n_obs ? obstacles[b * 12 + d] : INFINITY;
+                bhi[c][d] = b < n_obs ? obstacles[b * 12 + 6 + d] : -INFINITY;
             }
-            seg_bbox(v, w, bmin, bmax);
         }
-        // Only boxes that meet the union of the wave's segment boxes can be
-        // hit (the broad phase of segment_hits_box uses the same <= test,
-        // and a box separated from the union is separated from each
-        // segment's box), so each lane tests just those: lane-parallel
-        // over the boxes, 64 at a time, then the candidates one by one.
-        float umin[3], umax[3];
+    }
+    const float *xc = xcomb + (int64_t)p * 3 * tmax_steps;
+    bool hit = false;
+    if (t0 < t1) {
+        // the point at t0, and the next point's noise loaded ahead
+        float v[3], xn[3];
+        int vmin[3], vmax[3]; // bounds over the wave, as ordered integers
         for (int d = 0; d < 3; ++d) {
-            umin[d] = wave_min(bmin[d]);
-            umax[d] = wave_max(bmax[d]);
+            v[d] = path[t0 * kDim + d] + xc[t0 * 3 + d] * om;
+            xn[d] = xc[(t0 + 1) * 3 + d];
         }
-        bool hit = false;
-        for (int b0 = 0; b0 < n_obs; b0 += 64) {
-            bool meets = false;
-            if (b0 + lane < n_obs) {
-                float lo[3], hi[3];
-                box_bounds(o, obstacles, b0 + lane, lo, hi);
-                meets = !((umax[0] <= lo[0]) | (hi[0] <= umin[0]) | (umax[1] <= lo[1]) |
-                          (hi[1] <= umin[1]) | (umax[2] <= lo[2]) | (hi[2] <= umin[2]));
+        for (int d = 0; d < 3; ++d) {
+            const int i = ordered_int(__float_as_int(v[d]));
+            vmin[d] = wave_min_i(i);
+            vmax[d] = wave_max_i(i);
+        }
+        for (int t = t0; t < t1; ++t) {
+            float w[3];
+            int wmin[3], wmax[3];
+            for (int d = 0; d < 3; ++d)
+                w[d] = path[(t + 1) * kDim + d] + xn[d] * om;
+            if (t + 1 < t1)
+                for (int d = 0; d < 3; ++d)
+                    xn[d] = xc[(t + 2) * 3 + d];
+            // The union of the particles' segment boxes: a box separated from
+            // it (the broad phase's own <= test) is separated from each.
+            float umin[3], umax[3];
+            for (int d = 0; d < 3; ++d) {
+                const int i = ordered_int(__float_as_int(w[d]));
+                wmin[d] = wave_min_i(i);
+                wmax[d] = wave_max_i(i);
+                umin[d] = __int_as_float(ordered_int(min(vmin[d], wmin[d])));
+                umax[d] = __int_as_float(ordered_int(max(vmax[d], wmax[d])));
             }
-            unsigned long long cand = __ballot(meets);
-            while (cand) {
-                const int b = b0 + __builtin_ctzll(cand);
-                cand &= cand - 1;
-                float lo[3], hi[3];
-                box_bounds(o, obstacles, b, lo, hi);
-                if (act && !hit)
-                    hit = segment_hits_box(v, w, bmin, bmax, lo, hi);
+            float bmin[3], bmax[3];
+            seg_bbox(v, w, bmin, bmax);
+            const auto meets = [&](const float *lo, const float *hi) {
+                return !((umax[0] <= lo[0]) | (hi[0] <= umin[0]) | (umax[1] <= lo[1]) |
+                         (hi[1] <= umin[1]) | (umax[2] <= lo[2]) | (hi[2] <= umin[2]));
+            };
+            if (kBoxes > 0) {
+#pragma unroll
+                for (int c = 0; c < kRegs; ++c) {
+                    unsigned long long cand = __ballot(meets(blo[c], bhi[c]));
+                    while (cand) {
+                        const int l = __builtin_ctzll(cand);
+                        cand &= cand - 1;
+                        float lo[3], hi[3];
+                        for (int d = 0; d < 3; ++d) {
+                            lo[d] = read_lane(blo[c][d], l);
+                            hi[d] = read_lane(bhi[c][d], l);
+                        }
+                        if (!hit)
+                            hit = segment_hits_box(v, w, bmin, bmax, lo, hi);
+                    }
+                }
+            } else {
+                for (int b0 = 0; b0 < n_obs; b0 += 64) {
+                    const int b = b0 + lane;
+                    float lo[3] = {INFINITY, INFINITY, INFINITY};
+                    float hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+                    if (b < n_obs)
+                        for (int d = 0; d < 3; ++d) {
+                            lo[d] = obstacles[(int64_t)b * 12 + d];
+                            hi[d] = obstacles[(int64_t)b * 12 + 6 + d];
+                        }
+                    unsigned long long cand = __ballot(b < n_obs && meets(lo, hi));
+                    while (cand) {
+                        const int l = __builtin_ctzll(cand);
+                        cand &= cand - 1;
+                        float clo[3], chi[3];
+                        for (int d = 0; d < 3; ++d) {
+                            clo[d] = read_lane(lo[d], l);
+                            chi[d] = read_lane(hi[d], l);
+                        }
+                        if (!hit)
+                            hit = segment_hits_box(v, w, bmin, bmax, clo, chi);
+                    }
+                }
+            }
+            if (__ballot(hit) == ~0ull)
+                break;
+            for (int d = 0; d < 3; ++d) {
+                v[d] = w[d];
+                vmin[d] = wmin[d];
+                vmax[d] = wmax[d];
             }
         }
-        if (__ballot(hit) != 0ull) {
-            if (lane == 0)
-                atomicAdd(&hits[k], 1);
-            break;
-        }
+    }
+    const unsigned long long m = __ballot(hit && first + lane < n_mc);
+    if (lane == 0)
+        hit_mask[wid] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned long long all = 0;
+        for (int i = 0; i < n_waves; ++i)
+            all |= hit_mask[i];
+        if (all)
+            atomicAdd(&hits[k], __popcll(all));
     }
 }
 
@@ -118,9 +196,24 @@ extern "C" int pump_collision_probability_many(const float *d_obstacles, int n_o
         hipLaunchKernelGGL(k_zero_hits, dim3(1), dim3(256), 0, s, d_hits, n_paths);
         PUMP_LAUNCHED();
     }
-    dim3 grid((unsigned)((n_mc + 3) / 4), (unsigned)n_paths);
-    hipLaunchKernelGGL(k_mccp, grid, dim3(256), 0, s, d_obstacles, n_obs, d_xcomb, tmax_steps, n_mc,
-                       offset_mult, d_paths, path_stride_rows, d_T, d_hits);
+    // waves per workgroup: enough that the launch has kTargetWaves of them
+    const unsigned groups = (unsigned)((n_mc + 63) / 64);
+    int waves = 1;
+    while (waves < kMaxWaves && (int64_t)groups * n_paths * waves < kTargetWaves)
+        waves *= 2;
+    const dim3 grid(groups, (unsigned)n_paths), block(64 * waves);
+    const auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, block, 0, s, d_obstacles, n_obs, d_xcomb, tmax_steps,
+                           n_mc, offset_mult, d_paths, path_stride_rows, d_T, d_hits);
+    };
+    if (n_obs <= 64)
+        launch(k_mccp<1>);
+    else if (n_obs <= 128)
+        launch(k_mccp<2>);
+    else if (n_obs <= 256)
+        launch(k_mccp<4>);
+    else
+        launch(k_mccp<0>);
     PUMP_LAUNCHED();
     return PUMP_OK;
 }

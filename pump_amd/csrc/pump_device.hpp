@@ -838,24 +838,49 @@ __device__ __forceinline__ float read_lane(float x, int l)
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l));
 }
 
-// min / max over the 64 lanes of a wave (all lanes active): rotations
-// within each row of 16, then the four row results
+// Min / max over the 64 lanes of a wave (all lanes active): rotations within
+// each row of 16, then the four row results.  They work on integers in the
+// floats' order (x -> ordered_int(x), its own inverse): an integer min takes
+// the rotation as its DPP operand, one instruction per step, and combines
+// the row results on the scalar unit, where a float min needs a separate
+// move and a canonicalisation per step.  A NaN orders beyond the infinity of
+// its sign, so a union of bounds that holds one compares false with
+// everything: nothing counts as separated from it.
+__device__ __forceinline__ int ordered_int(int i) { return i ^ ((i >> 31) & 0x7fffffff); }
+
+template <int kCtrl> __device__ __forceinline__ int dpp_rotate(int x)
+{
+    return __builtin_amdgcn_update_dpp(0, x, kCtrl, 0xf, 0xf, true);
+}
+
+__device__ __forceinline__ int wave_min_i(int x)
+{
+    x = min(x, dpp_rotate<0x121>(x));
+    x = min(x, dpp_rotate<0x122>(x));
+    x = min(x, dpp_rotate<0x124>(x));
+    x = min(x, dpp_rotate<0x128>(x));
+    return min(min(__builtin_amdgcn_readlane(x, 0), __builtin_amdgcn_readlane(x, 16)),
+               min(__builtin_amdgcn_readlane(x, 32), __builtin_amdgcn_readlane(x, 48)));
+}
+
+__device__ __forceinline__ int wave_max_i(int x)
+{
+    x = max(x, dpp_rotate<0x121>(x));
+    x = max(x, dpp_rotate<0x122>(x));
+    x = max(x, dpp_rotate<0x124>(x));
+    x = max(x, dpp_rotate<0x128>(x));
+    return max(max(__builtin_amdgcn_readlane(x, 0), __builtin_amdgcn_readlane(x, 16)),
+               max(__builtin_amdgcn_readlane(x, 32), __builtin_amdgcn_readlane(x, 48)));
+}
+
 __device__ __forceinline__ float wave_min(float x)
 {
-    x = fminf(x, dpp_move<0x121>(x));
-    x = fminf(x, dpp_move<0x122>(x));
-    x = fminf(x, dpp_move<0x124>(x));
-    x = fminf(x, dpp_move<0x128>(x));
-    return fminf(fminf(read_lane(x, 0), read_lane(x, 16)), fminf(read_lane(x, 32), read_lane(x, 48)));
+    return __int_as_float(ordered_int(wave_min_i(ordered_int(__float_as_int(x)))));
 }
 
 __device__ __forceinline__ float wave_max(float x)
 {
-    x = fmaxf(x, dpp_move<0x121>(x));
-    x = fmaxf(x, dpp_move<0x122>(x));
-    x = fmaxf(x, dpp_move<0x124>(x));
-    x = fmaxf(x, dpp_move<0x128>(x));
-    return fmaxf(fmaxf(read_lane(x, 0), read_lane(x, 16)), fmaxf(read_lane(x, 32), read_lane(x, 48)));
+    return __int_as_float(ordered_int(wave_max_i(ordered_int(__float_as_int(x)))));
 }
 
 } // namespace pump
