@@ -527,8 +527,16 @@ __device__ __forceinline__ void propagate_path(
 //      pairs and ANDs the results into their rows, then finishes their CP.
 // When the pairs overflow the workspace, (4) is replaced by the group form:
 // one wave per (listed path, 512 particles).
-constexpr int kClassifyBlock = 1024;
+// Workgroups of 1024 paths take one atomic on the list's end each, which at
+// a million paths is what the pass waits for with smaller ones; below
+// kClassifyWide paths those leave compute units without one.  Where the
+// edges' summaries are not given, 16 waves read the slots of 256 paths
+// (kSlots) and the first four go on: 60000 paths of 20 waypoints 83 us with
+// each lane reading its own path's, 16 us so.
+constexpr int kClassifyBlock = 1024, kClassifySmall = 256;
+constexpr int kClassifyWide = 1 << 18;
 
+template <int kBlock, bool kSlots>
 __device__ __forceinline__ void classify_body(
     int n_new, const int64_t *__restrict__ wp_offsets, int w_fixed,
     const int *__restrict__ wf_edge, const int *__restrict__ wf_prev,
@@ -540,39 +548,68 @@ __device__ __forceinline__ void classify_body(
     const float *__restrict__ parent_cp, float *__restrict__ path_cp, int64_t cp_base,
     const VGrid &G)
 {
-    __shared__ int wcount[kClassifyBlock / 64];
+    constexpr int kPaths = kSlots ? kBlock / 64 * kSlotPaths : kBlock; // per pass
+    __shared__ int wcount[kPaths / 64];
     __shared__ int block_base;
+    __shared__ int64_t s_g0[kSlots ? kPaths : 1];
+    __shared__ int s_W[kSlots ? kPaths : 1];
+    __shared__ uint64_t s_mask[kSlots ? kPaths : 1];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    const int64_t stride = G.nb * kClassifyBlock;
+    const int64_t stride = G.nb * kPaths;
     // workgroup-uniform trip count: every thread reaches the barriers below
-    for (int64_t base = G.bid * kClassifyBlock; base < n_new; base += stride) {
-        const int64_t w = base + threadIdx.x;
+    for (int64_t base = G.bid * kPaths; base < n_new; base += stride) {
+        const int64_t w = threadIdx.x < kPaths ? base + threadIdx.x : n_new;
         bool has = false;
         int n_clamped = 0;
         HsPath r;
+        PathInfo pi{0, 0, 0.0f, 0.0f};
+        bool look = false;
+        uint64_t em0 = ~0ull;
         if (w < n_new) {
             const int e = wf_edge[w];
             // an all-clear summary settles the path with one load
-            const uint64_t em0 = edge_mask ? edge_mask[e] : ~0ull;
-            if (em0 != 0ull) {
+            if (!kSlots)
+                em0 = edge_mask[e];
+            look = em0 != 0ull;
+            if (look) {
                 r.prev = wf_prev[w];
-                const PathInfo pi = path_info(e, r.prev, wp_offsets, w_fixed, topts, times);
-                r.emask = edge_mask ? mask_bits(em0, pi.W) : 0ull;
-                for_each_marked(pi, edge_mask != nullptr, r.emask, bs, max_hs, [&](int i) {
-                    has = true;
-                    const int ti = time_index(pi, i, dt);
-                    const int tc = clamp_time(ti, tmax_steps);
-                    n_clamped += ti != tc ? 1 : 0;
-                    if (hist)
-                        atomicAdd(&hist[tc * kSubBins + (int)(w & (kSubBins - 1))], 1);
-                });
-                r.g0 = pi.g0;
-                r.W = pi.W;
-                r.dtl = pi.dtl;
-                r.tbase = pi.tbase;
-                r.w = (int)w;
-                r.pad = 0;
+                pi = path_info(e, r.prev, wp_offsets, w_fixed, topts, times);
             }
+        }
+        bool known = true;
+        if constexpr (kSlots) {
+            known = pi.W <= 64;
+            if (threadIdx.x < kPaths) {
+                s_g0[threadIdx.x] = pi.g0;
+                s_W[threadIdx.x] = known ? pi.W : 0;
+            }
+            __syncthreads();
+            const int at = wid * kSlotPaths;
+            slot_summaries(s_g0 + at, s_W + at, s_mask + at, bs, max_hs);
+            __syncthreads();
+            if (look && known) {
+                em0 = s_mask[threadIdx.x];
+                look = em0 != 0ull;
+            }
+        }
+        if (look) {
+            r.known = known ? 1 : 0;
+            r.emask = known ? mask_bits(em0, pi.W) : 0ull;
+            for_each_marked(pi, known, r.emask, bs, max_hs, [&](int i) {
+                has = true;
+                const int ti = time_index(pi, i, dt);
+                const int tc = clamp_time(ti, tmax_steps);
+                n_clamped += ti != tc ? 1 : 0;
+                if (hist)
+                    atomicAdd(&hist[tc * kSubBins + (int)(w & (kSubBins - 1))], 1);
+            });
+            r.g0 = pi.g0;
+            r.W = pi.W;
+            r.dtl = pi.dtl;
+            r.tbase = pi.tbase;
+            r.w = (int)w;
+        }
+        if (w < n_new) {
             has_hs[w] = has ? 1 : 0;
             // copy-on-write: a path that meets no half-space keeps its
             // parent's row and CP (the same count, the same float)
@@ -590,12 +627,12 @@ __device__ __forceinline__ void classify_body(
         if (n_clamped && clamped)
             atomicAdd(clamped, (unsigned long long)n_clamped);
         const uint64_t m = __ballot(has);
-        if (lane == 0)
+        if (lane == 0 && wid < kPaths / 64)
             wcount[wid] = __popcll(m);
         __syncthreads();
         if (threadIdx.x == 0) {
             int total = 0;
-            for (int k = 0; k < kClassifyBlock / 64; ++k) {
+            for (int k = 0; k < kPaths / 64; ++k) {
                 const int c = wcount[k];
                 wcount[k] = total;
                 total += c;
@@ -612,7 +649,8 @@ __device__ __forceinline__ void classify_body(
     }
 }
 
-__global__ __launch_bounds__(kClassifyBlock) void k_classify(
+template <int kBlock, bool kSlots>
+__global__ __launch_bounds__(kBlock) void k_classify(
     int n_new, const int64_t *__restrict__ wp_offsets, int w_fixed,
     const int *__restrict__ wf_edge, const int *__restrict__ wf_prev,
     const float *__restrict__ bs, const uint64_t *__restrict__ edge_mask, int max_hs,
@@ -622,9 +660,9 @@ __global__ __launch_bounds__(kClassifyBlock) void k_classify(
     unsigned long long *__restrict__ clamped, int *__restrict__ row_src,
     const float *__restrict__ parent_cp, float *__restrict__ path_cp, int64_t cp_base)
 {
-    classify_body(n_new, wp_offsets, w_fixed, wf_edge, wf_prev, bs, edge_mask, max_hs, times,
-                  topts, dt, tmax_steps, has_hs, recs, ctl, hist, acc, clamped, row_src,
-                  parent_cp, path_cp, cp_base, hw_grid());
+    classify_body<kBlock, kSlots>(n_new, wp_offsets, w_fixed, wf_edge, wf_prev, bs, edge_mask, max_hs,
+                                  times, topts, dt, tmax_steps, has_hs, recs, ctl, hist, acc,
+                                  clamped, row_src, parent_cp, path_cp, cp_base, hw_grid());
 }
 
 // Copy unit per lane: 16-byte chunks (bit masks or byte rows), 8-byte words
@@ -670,7 +708,11 @@ __device__ __forceinline__ int copy_count(uint4 &x)
 template <bool kBits>
 __device__ __forceinline__ int copy_count(uint64_t &x)
 {
-    return __popcll(x); // 8-byte units are used for bit rows only
+    if (kBits)
+        return __popcll(x);
+    const uint32_t lo = nonzero_bytes01((uint32_t)x), hi = nonzero_bytes01((uint32_t)(x >> 32));
+    x = ((uint64_t)hi << 32) | lo;
+    return 8 - __popc(lo) - __popc(hi);
 }
 template <bool kBits>
 __device__ __forceinline__ int copy_count(uint32_t &x)
@@ -1136,10 +1178,10 @@ __global__ __launch_bounds__(kClassifyBlock) void k_classify_many(
     VGrid G;
     const McJob J = global_job(mc_job(jobs, map, kMcClassify, G));
     const BinArgs &a = J.B;
-    classify_body(a.n_new, J.wp_offsets, 0, J.wf_edge, J.wf_prev, a.bs, J.edge_mask, a.max_hs,
-                  J.times, J.topts, a.dt, a.tmax_steps, J.has, const_cast<HsPath *>(a.recs),
-                  a.ctl, a.hist, a.acc, J.clamped, J.row_src, J.parent_cp, a.path_cp, a.cp_base,
-                  G);
+    classify_body<kClassifyBlock, false>(
+        a.n_new, J.wp_offsets, 0, J.wf_edge, J.wf_prev, a.bs, J.edge_mask, a.max_hs, J.times,
+        J.topts, a.dt, a.tmax_steps, J.has, const_cast<HsPath *>(a.recs), a.ctl, a.hist, a.acc,
+        J.clamped, J.row_src, J.parent_cp, a.path_cp, a.cp_base, G);
 }
 
 __global__ __launch_bounds__(256) void k_copy_listed_many(const McJob *__restrict__ jobs,
@@ -1360,6 +1402,10 @@ static int launch_path(int n_new, const int64_t *wp_offsets, int W_fixed, const 
 // at 65536 paths few boxes favour the waves.
 constexpr int kPathFormMax = 32768;
 constexpr int kBatchedMin = 4096;
+// The drop-in call, whose batched form also allocates its workspace: a
+// workgroup per path takes 48-62 against 63-75 us at 16384 paths (500 and
+// 2000 particles, few and many boxes) and 87-120 against 70-87 at 32768.
+constexpr int kDropInBatchedMin = 20480;
 
 // The 64-paths-per-wave propagate: its copy unit and grid
 template <bool kBits>
@@ -1410,7 +1456,7 @@ extern "C" int pump_propagate_valid_particles(
     PUMP_REQUIRE(d_wf_edge && d_wf_prev && d_as && d_bs && d_times && d_topts && d_offsets_time &&
                  d_valid);
     hipStream_t s = as_stream(stream);
-    if (num_new_paths >= kBatchedMin && !use_block_kernel()) {
+    if (num_new_paths >= kDropInBatchedMin && !use_block_kernel()) {
         // A large wavefront runs the batched form in place (classify, row
         // copies, time-binned half-space tests) with a workspace from the
         // stream-ordered pool, released on the same stream; the reference
@@ -1586,7 +1632,6 @@ static int launch_propagate(int n_new, int W_fixed, const int64_t *wp_offsets, c
         B.n_mc = n_mc;
         B.tmax_steps = tmax_steps;
         B.max_hs = max_hs;
-        B.known = edge_mask ? 1 : 0;
         B.dt = dt;
         B.om = om;
         B.as = as;
@@ -1616,10 +1661,19 @@ static int launch_propagate(int n_new, int W_fixed, const int64_t *wp_offsets, c
         hipLaunchKernelGGL(k_zero_words, dim3(grid_for(n_zero, 256, 1024)), dim3(256), 0, s, ctl,
                            n_zero);
         PUMP_LAUNCHED();
-        hipLaunchKernelGGL(k_classify, dim3(grid_for(n_new, kClassifyBlock, 2048)),
-                           dim3(kClassifyBlock), 0, s, n_new, wp_offsets, W_fixed, wf_edge,
-                           wf_prev, bs, edge_mask, max_hs, times, topts, dt, tmax_steps, has,
-                           recs, ctl, hist, acc, clamped, row_src, parent_cp, path_cp, cp_base);
+        const auto classify = [&](auto kernel, int block, int paths) {
+            hipLaunchKernelGGL(kernel, dim3(grid_for(n_new, paths, 2048)), dim3(block), 0, s,
+                               n_new, wp_offsets, W_fixed, wf_edge, wf_prev, bs, edge_mask,
+                               max_hs, times, topts, dt, tmax_steps, has, recs, ctl, hist, acc,
+                               clamped, row_src, parent_cp, path_cp, cp_base);
+        };
+        if (!edge_mask)
+            classify(k_classify<kClassifyBlock, true>, kClassifyBlock,
+                     kClassifyBlock / 64 * kSlotPaths);
+        else if (n_new < kClassifyWide)
+            classify(k_classify<kClassifySmall, false>, kClassifySmall, kClassifySmall);
+        else
+            classify(k_classify<kClassifyBlock, false>, kClassifyBlock, kClassifyBlock);
         PUMP_LAUNCHED();
         int r = bins_scan(B, s);
         if (r)
@@ -1645,7 +1699,7 @@ static int launch_propagate(int n_new, int W_fixed, const int64_t *wp_offsets, c
         int unit = 1;
         if (row_bytes % 16 == 0 && (al & 15) == 0)
             unit = 16;
-        else if (kBits)
+        else if (kBits || (row_bytes % 8 == 0 && (al & 7) == 0))
             unit = 8;
         else if (row_bytes % 4 == 0 && (al & 3) == 0)
             unit = 4;
@@ -1668,6 +1722,10 @@ static int launch_propagate(int n_new, int W_fixed, const int64_t *wp_offsets, c
                                cp_base);
         else if (unit == 16)
             hipLaunchKernelGGL((k_copy_rows<16, false>), dim3(grid), dim3(256), 0, s, n_new,
+                               wf_prev, has, cc, sb, db, dst_base, row_bytes, n_p, seg, path_cp,
+                               cp_base);
+        else if (unit == 8)
+            hipLaunchKernelGGL((k_copy_rows<8, false>), dim3(grid), dim3(256), 0, s, n_new,
                                wf_prev, has, cc, sb, db, dst_base, row_bytes, n_p, seg, path_cp,
                                cp_base);
         else if (unit == 4)
@@ -1708,8 +1766,8 @@ int pump::mc_cow_job(McJob &J, int n_new, const int64_t *wp_offsets, const int *
                      const void *src, const float *parent_cp, void *dst, int *row_src, int n_p,
                      float *path_cp, void *ws, size_t ws_bytes)
 {
-    if (n_new < 1 || n_p < 1 || !wp_offsets || !ws || !src || !dst || !row_src || !path_cp ||
-        !parent_cp)
+    if (n_new < 1 || n_p < 1 || !wp_offsets || !edge_mask || !ws || !src || !dst || !row_src ||
+        !path_cp || !parent_cp)
         return PUMP_E_INVALID;
     const BatchLayout L = BatchLayout::fill(n_new, tmax_steps, ws_bytes);
     const int64_t row_bytes = (int64_t)((n_p + 63) / 64) * 8;
@@ -1724,7 +1782,6 @@ int pump::mc_cow_job(McJob &J, int n_new, const int64_t *wp_offsets, const int *
     B.n_mc = n_mc;
     B.tmax_steps = tmax_steps;
     B.max_hs = max_hs;
-    B.known = edge_mask ? 1 : 0;
     B.dt = dt;
     B.om = om;
     B.as = as;

@@ -148,7 +148,7 @@ __global__ __launch_bounds__(kScanBlock) void k_bin_scan(int T, const int *__res
 // lane = listed path: its (waypoint, time index) pairs into the sorted array
 // at tstart[ti] + (pairs of lower sub-bins) + (rank within the sub-bin)
 __device__ __forceinline__ void bin_emit_body(const HsPath *__restrict__ recs,
-                                              const int *__restrict__ ctl, int known,
+                                              const int *__restrict__ ctl,
                                               const float *__restrict__ bs, int max_hs, float dt,
                                               int tmax_steps, const int *__restrict__ hist,
                                               const int *__restrict__ tstart,
@@ -167,7 +167,7 @@ __device__ __forceinline__ void bin_emit_body(const HsPath *__restrict__ recs,
         pi.dtl = r.dtl;
         pi.tbase = r.tbase;
         const int sub = r.w & (kSubBins - 1);
-        for_each_marked(pi, known != 0, r.emask, bs, max_hs, [&](int i) {
+        for_each_marked(pi, r.known != 0, r.emask, bs, max_hs, [&](int i) {
             const int ti = clamp_time(time_index(pi, i, dt), tmax_steps);
             int below;
             time_total(hist, ti, sub, &below);
@@ -183,7 +183,7 @@ __device__ __forceinline__ void bin_emit_body(const HsPath *__restrict__ recs,
 }
 
 __global__ __launch_bounds__(256) void k_bin_emit(const HsPath *__restrict__ recs,
-                                                  const int *__restrict__ ctl, int known,
+                                                  const int *__restrict__ ctl,
                                                   const float *__restrict__ bs, int max_hs,
                                                   float dt, int tmax_steps,
                                                   const int *__restrict__ hist,
@@ -191,7 +191,7 @@ __global__ __launch_bounds__(256) void k_bin_emit(const HsPath *__restrict__ rec
                                                   int *__restrict__ cursor,
                                                   BinEntry *__restrict__ entries)
 {
-    bin_emit_body(recs, ctl, known, bs, max_hs, dt, tmax_steps, hist, tstart, cursor, entries,
+    bin_emit_body(recs, ctl, bs, max_hs, dt, tmax_steps, hist, tstart, cursor, entries,
                   hw_grid());
 }
 
@@ -573,7 +573,7 @@ __device__ __forceinline__ void group_pass(const BinArgs &a, int64_t n_listed, c
         }
         for (int i0 = 0; i0 < pi.W; i0 += 256) {
             uint64_t masks[4];
-            const uint64_t any = hs_masks(masks, pi, i0, a.known != 0, r.emask, a.max_hs, a.bs,
+            const uint64_t any = hs_masks(masks, pi, i0, r.known != 0, r.emask, a.max_hs, a.bs,
                                           a.dt, a.tmax_steps, (unsigned long long *)nullptr);
             uint64_t alive = 0;
 #pragma unroll
@@ -729,7 +729,7 @@ __global__ __launch_bounds__(256) void k_bin_emit_many(const McJob *__restrict__
 {
     VGrid G;
     const BinArgs a = global_args(mc_job(jobs, map, kMcEmit, G).B);
-    bin_emit_body(a.recs, a.ctl, a.known, a.bs, a.max_hs, a.dt, a.tmax_steps, a.hist, a.tstart,
+    bin_emit_body(a.recs, a.ctl, a.bs, a.max_hs, a.dt, a.tmax_steps, a.hist, a.tstart,
                   a.cursor, a.entries, G);
 }
 
@@ -826,7 +826,7 @@ int bins_finish(const BinArgs &a, bool bits, hipStream_t s)
 {
     // device-side counts; the grids are sized for their upper bounds
     hipLaunchKernelGGL(k_bin_emit, dim3(grid_for(a.n_new, 256, 4096)), dim3(256), 0, s, a.recs,
-                       (const int *)a.ctl, a.known, a.bs, a.max_hs, a.dt, a.tmax_steps,
+                       (const int *)a.ctl, a.bs, a.max_hs, a.dt, a.tmax_steps,
                        (const int *)a.hist, (const int *)a.tstart, a.cursor, a.entries);
     PUMP_LAUNCHED();
     const int64_t groups = (a.n_p + 63) / 64;

@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "pump_device.hpp"
 #include "pump_internal.hpp"
 
 #pragma clang fp contract(off)
@@ -108,6 +109,58 @@ __device__ __forceinline__ void for_each_marked(const PathInfo &pi, bool known, 
     for (int i = scan_from; i < pi.W; ++i)
         if (waypoint_has_hs(bs, (pi.g0 + i) * (int64_t)max_hs, max_hs))
             f(i);
+}
+
+// Waypoint summaries from the slots themselves, for kSlotPaths paths of a
+// wave whose first waypoints and waypoint counts lie in g0[] and W[] (W = 0:
+// not looked at; at most 64 otherwise): mask[l] for each.  Called by whole
+// waves.  2^lg lanes take one path, a waypoint each, so that a path's slots
+// are read side by side, with kAhead paths' first kSlots slots in flight per
+// lane: a lane reading its own path's slots one waypoint after another waits
+// for every one of them.
+constexpr int kSlotPaths = 16;
+__device__ __forceinline__ void slot_summaries(const int64_t *g0, const int *W, uint64_t *mask,
+                                               const float *__restrict__ bs, int max_hs)
+{
+    constexpr int kAhead = 4, kSlots = 8;
+    const int lane = threadIdx.x & 63;
+    const int longest = wave_max_i(W[lane & (kSlotPaths - 1)]);
+    int lg = 2;
+    while ((1 << lg) < longest)
+        ++lg;
+    const int per = 64 >> lg; // paths per ballot, at most kSlotPaths
+    const int i = lane & ((1 << lg) - 1), sub = lane >> lg;
+    for (int l0 = 0; l0 < kSlotPaths; l0 += per * kAhead) {
+        const float *b[kAhead];
+        bool in[kAhead], has[kAhead];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            const int l = l0 + u * per + sub;
+            in[u] = l < kSlotPaths && i < W[l & (kSlotPaths - 1)];
+            b[u] = bs + (g0[l & (kSlotPaths - 1)] + i) * (int64_t)max_hs;
+            has[u] = false;
+        }
+        for (int h0 = 0; h0 < max_hs; h0 += kSlots) {
+            float x[kAhead][kSlots];
+#pragma unroll
+            for (int h = 0; h < kSlots; ++h)
+#pragma unroll
+                for (int u = 0; u < kAhead; ++u)
+                    x[u][h] = in[u] && h0 + h < max_hs ? b[u][h0 + h] : 1111.0f;
+#pragma unroll
+            for (int h = 0; h < kSlots; ++h)
+#pragma unroll
+                for (int u = 0; u < kAhead; ++u)
+                    has[u] = has[u] || !(x[u][h] >= 1000.0f);
+        }
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            const uint64_t m = __ballot(has[u]) >> (sub << lg);
+            const int l = l0 + u * per + sub;
+            if (i == 0 && l < kSlotPaths)
+                mask[l] = lg == 6 ? m : m & ((1ull << (1 << lg)) - 1ull);
+        }
+    }
 }
 
 // masks[c] bit l: waypoint i0+c*64+l holds a stored half-space (i0..i0+255),
@@ -238,6 +291,12 @@ __device__ __forceinline__ int invalid_bytes(const uint8_t *__restrict__ r, int 
             count += 16 - __popc(nonzero_bytes01(x.x)) - __popc(nonzero_bytes01(x.y)) -
                      __popc(nonzero_bytes01(x.z)) - __popc(nonzero_bytes01(x.w));
         }
+    } else if (((n_p & 7) == 0) && (((uintptr_t)r) & 7) == 0) {
+        const uint2 *r8 = reinterpret_cast<const uint2 *>(r);
+        for (int k = lane; k < (n_p >> 3); k += 64) {
+            const uint2 x = r8[k];
+            count += 8 - __popc(nonzero_bytes01(x.x)) - __popc(nonzero_bytes01(x.y));
+        }
     } else if (((n_p & 3) == 0) && (((uintptr_t)r) & 3) == 0) {
         const uint32_t *r4 = reinterpret_cast<const uint32_t *>(r);
         for (int k = lane; k < (n_p >> 2); k += 64)
@@ -277,9 +336,9 @@ constexpr int kHsGroups = 4;   // the same for the group form of the batched pas
 // batched classification pass.
 struct HsPath {
     int64_t g0;     // first waypoint of the edge
-    uint64_t emask; // the edge's waypoint summary (when known)
+    uint64_t emask; // the edge's waypoint summary, when known
     float dtl, tbase;
-    int W, prev, w, pad;
+    int W, prev, w, known;
 };
 
 // One (listed path, waypoint with a stored half-space) pair of the
@@ -316,7 +375,7 @@ enum : int {
 // tests them (or, on overflow, runs the group form) and writes the listed
 // paths' CP.
 struct BinArgs {
-    int n_new, n_p, n_mc, tmax_steps, max_hs, known;
+    int n_new, n_p, n_mc, tmax_steps, max_hs;
     float dt, om;
     const float *as, *bs, *offsets_time;
     const wave::HsPath *recs;

@@ -64,3 +64,44 @@ def test_path_form_against_oracle(n_p, w_range, max_hs, n_new):
             assert np.array_equal(got, ref_v[npar:]), (bits, mask is None)
             assert np.array_equal(host(cp)[2:], ref_cp[npar:])
             assert np.array_equal(host(row_src), np.arange(n_new))
+
+
+@pytest.mark.parametrize("w_range,max_hs,n_p,n_new", [
+    ((2, 4), 1, 64, 4096), ((2, 9), 5, 120, 4097), ((2, 17), 5, 200, 5000),
+    ((30, 33), 8, 72, 4100), ((33, 64), 9, 68, 4096), ((60, 70), 5, 333, 4200),
+    ((2, 20), 3, 24, 20500)])
+def test_batched_form_without_summaries(w_range, max_hs, n_p, n_new):
+    """The batched form finds the waypoints that store a half-space from the
+    slots themselves: groups of 4 to 64 lanes per path, more slots than one
+    round of loads, edges past 64 waypoints among them; byte rows of 8-, 4-
+    and 1-byte units; the drop-in call in place at its batched sizes."""
+    d = random_hsmc_inputs(max_hs + n_p, n_edges=700, max_hs=max_hs, n_p=n_p, n_mc=n_p + 1, T=90,
+                           n_new=n_new, n_parent=33, variable=True, w_range=w_range)
+    drop = np.random.default_rng(1).uniform(size=700) < 0.7
+    for e in np.nonzero(drop)[0]:
+        d["bs"][d["off"][e] * max_hs: d["off"][e + 1] * max_hs] = 1111
+    ref_v, ref_cp, ref_cl = oracle_propagate(d)
+    npar = d["n_parent"]
+    g = {k: dev(d[k]) for k in ("off", "as_", "bs", "offs", "topts", "times", "wf_edge",
+                                 "wf_prev")}
+    edges = (n_new, 0, ptr(g["off"]), ptr(g["wf_edge"]), ptr(g["wf_prev"]))
+    table = (ptr(g["times"]), ptr(g["topts"]), d["dt"], max_hs, ptr(g["offs"]), d["T"], d["om"],
+             d["n_mc"])
+    print("batched", w_range, max_hs, n_p, n_new, flush=True)
+    ws_bytes = P.lib.pump_propagate_workspace(n_new, d["T"])
+    ws = P.DeviceArray(shape=(ws_bytes,), dtype=np.uint8, fill=0x77)
+    src, dst = dev(d["valid"][:npar]), dev(np.full((n_new, n_p), 9, np.uint8))
+    cp, clamp = dev(np.zeros(n_new, np.float32)), dev(np.zeros(1, np.uint64))
+    P.check("propagate_cp", P.lib.pump_propagate_cp(
+        *edges, ptr(g["as_"]), ptr(g["bs"]), None, *table, ptr(src), ptr(dst), 0, n_p, ptr(cp), 0,
+        ptr(clamp), ws.p, ws_bytes, None))
+    assert np.array_equal(host(dst), ref_v[npar:]) and np.array_equal(host(cp), ref_cp[npar:])
+    assert int(host(clamp)[0]) == ref_cl
+    valid, clamp = dev(d["valid"]), dev(np.zeros(1, np.uint64))
+    P.check("propagate", P.lib.pump_propagate_valid_particles(
+        *edges, npar, ptr(g["as_"]), ptr(g["bs"]), None, *table, ptr(valid), n_p, ptr(clamp),
+        None))
+    assert np.array_equal(host(valid), ref_v) and int(host(clamp)[0]) == ref_cl
+    allcp = dev(np.zeros(npar + n_new, np.float32))
+    P.check("cp", P.lib.pump_calculate_cp_hsmc(n_new, npar, ptr(allcp), ptr(valid), n_p, None))
+    assert np.array_equal(host(allcp)[npar:], ref_cp[npar:])
