@@ -105,3 +105,64 @@ def test_batched_form_without_summaries(w_range, max_hs, n_p, n_new):
     allcp = dev(np.zeros(npar + n_new, np.float32))
     P.check("cp", P.lib.pump_calculate_cp_hsmc(n_new, npar, ptr(allcp), ptr(valid), n_p, None))
     assert np.array_equal(host(allcp)[npar:], ref_cp[npar:])
+
+
+@pytest.mark.parametrize("n_p,max_hs,scale", [(64, 1, 1.0), (300, 5, 1.0), (520, 9, 1.0),
+                                              (300, 5, 1e-14), (300, 5, 1e12)])
+def test_batched_tests_at_the_reach_of_the_particles(n_p, max_hs, scale):
+    """The batched tests leave out a half-space that no particle reaches.
+    Normals along a group's farthest particle with offsets a float above, at
+    and below that particle's product, and values that the bound cannot judge
+    (zero, tiny, infinite and NaN normals, offsets at and below zero)."""
+    n_new = 4100
+    d = random_hsmc_inputs(n_p, n_edges=300, max_hs=max_hs, n_p=n_p, n_mc=n_p, T=50, n_new=n_new,
+                           n_parent=9, variable=True, w_range=(2, 9))
+    rng = np.random.default_rng(n_p)
+    f = np.float32
+    # the same particles at every time: the products do not depend on the path
+    o = d["offs"][0] * f(scale)
+    o[: n_p // 2] *= f(0.25)  # groups of different reach
+    o[1] = 0.0
+    d["offs"][:] = o
+    far = o[np.argmax((o * o).sum(1))]
+    hs = d["bs"].size
+    d["as_"][:] = far * f(1.0 / scale) * rng.choice(np.array([0.5, 1, 2], f), (hs, 1))
+    lhs = d["as_"][:, 0] * far[0]
+    lhs = lhs + d["as_"][:, 1] * far[1]
+    lhs = (lhs + d["as_"][:, 2] * far[2]) * d["om"]
+    d["bs"][:] = lhs * rng.choice(np.array([0.9, 0.9999, 1, 1, 1.00001, 1.0001, 1.1], f), hs)
+    up = rng.integers(-1, 2, hs)
+    d["bs"][:] = np.where(up == 0, d["bs"], np.nextafter(d["bs"], np.where(up < 0, f(-np.inf), f(np.inf))))
+    d["bs"][d["bs"] >= 1000] = 999
+    odd = rng.uniform(size=hs) < 0.1
+    values = np.array([0, -0.0, 1e-45, 1e-25, 1e-8, -1e-3, 900], f)
+    d["bs"][odd] = rng.choice(values, odd.sum())
+    # a normal that fails a particle for good is kept rare
+    odd = rng.uniform(size=hs) < 0.02
+    d["as_"][odd] = rng.choice(np.array([0, 1e-38, 1e-24, 1e20, np.inf, np.nan], f),
+                               (odd.sum(), 3))
+    d["bs"][rng.uniform(size=hs) < 0.5] = 1111
+    ref_v, ref_cp, ref_cl = oracle_propagate(d)
+    npar = d["n_parent"]
+    assert 0.02 < ref_v[npar:].mean() < 0.84
+    g = {k: dev(d[k]) for k in ("off", "as_", "bs", "offs", "topts", "times", "wf_edge",
+                                 "wf_prev")}
+    g_mask = dev(edge_mask_host(d["off"], d["bs"], max_hs))
+    ws_bytes = P.lib.pump_propagate_workspace(n_new, d["T"])
+    ws = P.DeviceArray(shape=(ws_bytes,), dtype=np.uint8)
+    print("reach", n_p, max_hs, scale, flush=True)
+    for bits in (0, 1):
+        width = (n_p + 63) // 64 * 8 if bits else n_p
+        src = dev(pack_bits(d["valid"][:npar], n_p) if bits else d["valid"][:npar])
+        dst = dev(np.zeros((n_new, width), np.uint8))
+        cp, clamp = dev(np.zeros(n_new, np.float32)), dev(np.zeros(1, np.uint64))
+        fn = P.lib.pump_propagate_cp_bits if bits else P.lib.pump_propagate_cp
+        P.check("propagate_cp", fn(
+            n_new, 0, ptr(g["off"]), ptr(g["wf_edge"]), ptr(g["wf_prev"]), ptr(g["as_"]),
+            ptr(g["bs"]), g_mask.p, ptr(g["times"]), ptr(g["topts"]), d["dt"], max_hs,
+            ptr(g["offs"]), d["T"], d["om"], d["n_mc"], ptr(src), ptr(dst), 0, n_p, ptr(cp), 0,
+            *((0, None, None) if bits else ()), ptr(clamp), ws.p, ws_bytes, None))
+        rows = host(dst)
+        got = unpack_bits(rows.view(np.uint64), n_p) if bits else rows
+        assert np.array_equal(got, ref_v[npar:]), bits
+        assert np.array_equal(host(cp), ref_cp[npar:])
