@@ -1,27 +1,45 @@
 // roadmap.hip -- the roadmap glue of mainPUMP.cu:257-392 on the device:
 //   * rn = k-th smallest pair cost (thrust::sort + index, mainPUMP.cu:303-304)
-//     as a 3-pass radix select over order-preserving uint32 keys
-//     (11 + 11 + 10 bits), histograms in LDS, no host round trips between
-//     passes;
+//     over order-preserving uint32 keys: a sample brackets it, one pass over
+//     the array counts the keys below the bracket and collects those inside,
+//     and histograms of 2048 bins narrow these down to one;
 //   * edge numbering (copts < rn, row-major i then j, mainPUMP.cu:327-346):
 //     per-row counts, an exclusive scan, then an order-preserving per-row
 //     compaction with wave ballots;
 //   * maxNNSize and the padded neighbour tables (mainPUMP.cu:362-392);
 //   * waypoint offsets for a fixed or per-edge waypoint count.
 // All of this is HBM-streaming integer/compare work over the pair arrays.
+#include <algorithm>
+
 #include "pump_internal.hpp"
 
 namespace pump {
 namespace {
 
+// ---- k-th smallest key ----------------------------------------------------
 constexpr int kSelBins = 2048;
+constexpr int kSelSample = 16384; // keys of the sample, 16 per thread of one workgroup
+constexpr int kSelRun = 16;       // neighbouring keys per place of the sample: one 64-byte line
+constexpr int kSelTile = 8192;    // keys per workgroup and round of the bracket pass
+constexpr int kSelMaxRegions = 1024;
 
+// The keys still in question are those with key - lo <= span; k is the rank
+// sought among them.  The next pass bins them by (key - lo) >> shift.
 struct SelState {
-    uint32_t prefix;
-    uint32_t mask;
-    unsigned long long k; // rank still to skip inside the current prefix
+    unsigned long long k;
+    unsigned long long below;  // keys under lo (bracket pass)
+    unsigned long long n_cand; // keys inside the bracket (bracket pass)
+    uint32_t full;             // regions whose keys did not fit (bracket pass)
+    uint32_t lo, span, shift;
+    int counted; // k is a rank among the keys in question (not before the first pick)
+    int done;    // result holds the answer
+    int missed;  // the bracket does not hold rank k, or its keys did not fit
     float result;
-    uint32_t pad;
+
+    __device__ bool bracket_holds() const
+    {
+        return k >= below && k - below < n_cand && full == 0;
+    }
 };
 
 __device__ __forceinline__ uint32_t order_key(float f)
@@ -36,107 +54,344 @@ __device__ __forceinline__ float key_float(uint32_t k)
     return __uint_as_float(u);
 }
 
+// the bins of a span of keys: 2048 at most
+__device__ __forceinline__ uint32_t sel_shift(uint32_t span)
+{
+    return (uint32_t)max(0, 32 - 11 - (int)__clz((int)(span | 1u)));
+}
+
+// every key is in question
+__device__ __forceinline__ void sel_whole_range(SelState *st)
+{
+    st->lo = 0;
+    st->span = 0xffffffffu;
+    st->shift = sel_shift(st->span);
+}
+
+// inclusive scan of v over the workgroup; sh: one entry per wave
+template <typename T>
+__device__ __forceinline__ T block_scan(T v, T *sh)
+{
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    for (int off = 1; off < 64; off <<= 1) {
+        const T y = __shfl_up(v, off, 64);
+        if (lane >= off)
+            v += y;
+    }
+    __syncthreads(); // sh may be in use
+    if (lane == 63)
+        sh[wid] = v;
+    __syncthreads();
+    for (int w = 0; w < wid; ++w)
+        v += sh[w];
+    return v;
+}
+
 __global__ __launch_bounds__(256) void k_sel_init(SelState *st, unsigned long long *hist,
                                                   unsigned long long k)
 {
     for (int b = threadIdx.x; b < kSelBins; b += blockDim.x)
         hist[b] = 0;
     if (threadIdx.x == 0) {
-        st->prefix = 0;
-        st->mask = 0;
+        *st = SelState{};
         st->k = k;
-        st->result = 0.0f;
+        st->counted = 1;
+        sel_whole_range(st);
     }
 }
 
-__global__ __launch_bounds__(256) void k_sel_hist(const float *__restrict__ keys, int64_t n,
-                                                  const SelState *__restrict__ st, int shift,
-                                                  uint32_t bin_mask,
-                                                  unsigned long long *__restrict__ hist)
+// One workgroup: keys that bracket rank k, from a sample (kSelRun neighbours at
+// a scattered place in each of 1024 equal stretches), after two rounds of 2048
+// bins each.  The ranks in the sample are five standard deviations to either
+// side of k's place; a bracket that misses rank k all the same is found out by
+// its counts.  With n <= kSelSample the sample is the array and the key of
+// rank k itself comes out (done).  Lines, not single keys: the scattered loads
+// of 16384 keys took 20 us more on an array of 6.4e7; bins between the
+// smallest and the largest key, not of the leading bits: costs span a few
+// binary orders, whose handful of counters took another 10 us.
+__global__ __launch_bounds__(1024) void k_sel_sample(const float *__restrict__ keys, int64_t n,
+                                                     unsigned long long k, SelState *st,
+                                                     unsigned long long *hist)
+{
+    constexpr int kPer = kSelSample / 1024;
+    __shared__ uint32_t h[2][kSelBins];
+    __shared__ uint32_t sh[16];
+    __shared__ uint32_t least, most;
+    __shared__ uint32_t bin[2], before[2];
+    const int t = threadIdx.x;
+    const bool whole = n <= kSelSample;
+    const int m = whole ? (int)n : kSelSample;
+    uint32_t key[kPer];
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        int64_t at = q * 1024 + t;
+        if (!whole) {
+            constexpr int kPlaces = kSelSample / kSelRun;
+            const int j = (q * 1024 + t) / kSelRun;
+            const int64_t step = n / kPlaces; // >= kSelRun
+            at = j * step + (int64_t)(((uint32_t)j * 2654435769u) >> 7) % (step - kSelRun + 1) +
+                 t % kSelRun;
+        }
+        key[q] = q * 1024 + t < m ? order_key(keys[at]) : 0u;
+    }
+    if (t == 0) {
+        least = 0xffffffffu;
+        most = 0u;
+    }
+    for (int b = t; b < kSelBins; b += 1024)
+        hist[b] = 0;
+    uint32_t lo_key = 0xffffffffu, hi_key = 0u;
+#pragma unroll
+    for (int q = 0; q < kPer; ++q)
+        if (q * 1024 + t < m) {
+            lo_key = min(lo_key, key[q]);
+            hi_key = max(hi_key, key[q]);
+        }
+    for (int off = 32; off > 0; off >>= 1) {
+        lo_key = min(lo_key, (uint32_t)__shfl_xor((int)lo_key, off, 64));
+        hi_key = max(hi_key, (uint32_t)__shfl_xor((int)hi_key, off, 64));
+    }
+    __syncthreads();
+    if ((t & 63) == 0) {
+        atomicMin(&least, lo_key);
+        atomicMax(&most, hi_key);
+    }
+    const float place = (float)k / (float)n * (float)m;
+    const int margin = (int)(5.0f * sqrtf(fminf(place, (float)m - place) + 1.0f)) + 4;
+    const bool open_lo = !whole && (int)place - margin <= 0;
+    const bool open_hi = !whole && (int)place + margin >= m - 1;
+    uint32_t rank[2], lo[2], span[2], shift[2];
+    rank[0] = whole ? (uint32_t)k : (uint32_t)max(0, (int)place - margin);
+    rank[1] = whole ? (uint32_t)k : (uint32_t)min(m - 1, (int)place + margin);
+    __syncthreads();
+    for (int e = 0; e < 2; ++e) {
+        lo[e] = least;
+        span[e] = most - least;
+        shift[e] = sel_shift(span[e]);
+    }
+    for (int pass = 0; whole ? span[0] != 0 || pass == 0 : pass < 2; ++pass) {
+        for (int b = t; b < 2 * kSelBins; b += 1024)
+            (&h[0][0])[b] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < kPer; ++q) {
+            if (q * 1024 + t >= m)
+                continue;
+            if (key[q] - lo[0] <= span[0])
+                atomicAdd(&h[0][(key[q] - lo[0]) >> shift[0]], 1u);
+            if (pass > 0 && key[q] - lo[1] <= span[1])
+                atomicAdd(&h[1][(key[q] - lo[1]) >> shift[1]], 1u);
+        }
+        __syncthreads();
+        for (int e = 0; e < 2; ++e) {
+            const int from = pass > 0 ? e : 0; // the first pass is the same for both
+            const uint32_t c0 = h[from][2 * t], c1 = h[from][2 * t + 1];
+            const uint32_t c = block_scan(c0 + c1, sh) - c0 - c1;
+            if (rank[e] >= c && rank[e] < c + c0 + c1) {
+                const bool second = rank[e] >= c + c0;
+                bin[e] = 2 * t + (second ? 1 : 0);
+                before[e] = second ? c + c0 : c;
+            }
+        }
+        __syncthreads();
+        for (int e = 0; e < 2; ++e) {
+            lo[e] += bin[e] << shift[e];
+            rank[e] -= before[e];
+            span[e] = (1u << shift[e]) - 1u;
+            shift[e] = sel_shift(span[e]);
+        }
+        __syncthreads();
+    }
+    if (t == 0) {
+        *st = SelState{};
+        st->k = k;
+        if (whole) {
+            st->done = 1;
+            st->result = key_float(lo[0]);
+        } else {
+            const uint32_t hi = open_hi ? 0xffffffffu : lo[1] + span[1];
+            st->lo = open_lo ? 0u : lo[0];
+            st->span = hi - st->lo;
+            st->shift = sel_shift(st->span);
+        }
+    }
+}
+
+// One pass over all keys: counts those below the bracket and collects those
+// inside it (a percent or so) in cand, each workgroup in a region of its own
+// (region_cap keys; its count in counts).  Bound by the read of the array:
+// 6.4e7 keys in 60 us (4.3 TB/s); the selection 225 -> 107 us against three
+// histogram passes over the array, 5 launches for 7.  (Turning the counts into
+// the next state in the workgroup that ends last cost 100 us: every wave's
+// device-scope release writes its L2 back.  A launch costs 5.)
+__global__ __launch_bounds__(256) void k_sel_bracket(const float *__restrict__ keys, int64_t n,
+                                                     SelState *st, float *__restrict__ cand,
+                                                     uint32_t *__restrict__ counts,
+                                                     uint32_t region_cap)
+{
+    __shared__ uint32_t held;
+    __shared__ unsigned long long sh[4];
+    constexpr int kVec = kSelTile / 4 / 256;
+    const uint32_t lo = st->lo, span = st->span;
+    const int lane = threadIdx.x & 63;
+    const uint64_t lower = (1ull << lane) - 1ull;
+    float *region = cand + (int64_t)blockIdx.x * region_cap;
+    // 16-byte loads from the first aligned key on; up to 3 keys before and after
+    const int64_t head = min((int64_t)((16 - ((uintptr_t)keys & 15)) & 15) / 4, n);
+    const float4 *vec = reinterpret_cast<const float4 *>(keys + head);
+    const int64_t n4 = (n - head) / 4;
+    uint32_t below = 0;
+    if (threadIdx.x == 0)
+        held = 0;
+    __syncthreads();
+    const auto keep = [&](float f, uint32_t pos) {
+        if (pos < region_cap)
+            region[pos] = f;
+    };
+    if (blockIdx.x == 0 && threadIdx.x < 8) {
+        const int64_t i = threadIdx.x < 4 ? (int64_t)threadIdx.x : head + 4 * n4 + threadIdx.x - 4;
+        if (threadIdx.x < 4 ? i < head : i < n) {
+            const uint32_t key = order_key(keys[i]);
+            below += key < lo;
+            if (key - lo <= span)
+                keep(keys[i], atomicAdd(&held, 1u));
+        }
+    }
+    for (int64_t q0 = (int64_t)blockIdx.x * (256 * kVec); q0 < n4;
+         q0 += (int64_t)gridDim.x * (256 * kVec)) {
+        float4 v[kVec];
+#pragma unroll
+        for (int j = 0; j < kVec; ++j) {
+            const int64_t q = q0 + j * 256 + threadIdx.x;
+            v[j] = vec[q < n4 ? q : n4 - 1];
+        }
+#pragma unroll
+        for (int j = 0; j < kVec; ++j) {
+            const bool have = q0 + j * 256 + threadIdx.x < n4;
+            const float f[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
+            uint64_t in[4], any = 0ull;
+            uint32_t c = 0;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const uint32_t key = order_key(f[e]);
+                below += have && key < lo;
+                in[e] = __ballot(have && key - lo <= span);
+                any |= in[e];
+                c += __popcll(in[e]);
+            }
+            if (any == 0ull)
+                continue;
+            uint32_t pos = 0;
+            if (lane == 0)
+                pos = atomicAdd(&held, c);
+            pos = __builtin_amdgcn_readfirstlane(pos);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if ((in[e] >> lane) & 1ull)
+                    keep(f[e], pos + __popcll(in[e] & lower));
+                pos += __popcll(in[e]);
+            }
+        }
+    }
+    const unsigned long long total = block_scan((unsigned long long)below, sh);
+    if (threadIdx.x == 255) {
+        const uint32_t c = held;
+        counts[blockIdx.x] = c;
+        atomicAdd(&st->below, total);
+        atomicAdd(&st->n_cand, (unsigned long long)c);
+        if (c > region_cap)
+            atomicAdd(&st->full, 1u);
+    }
+}
+
+// Histogram of the keys in question in 2048 bins.  keys == nullptr: the
+// collected keys, a wave per region; few workgroups then, since each adds up
+// to 2048 counters to the device's.
+__global__ __launch_bounds__(1024) void k_sel_pass(const float *__restrict__ keys, int64_t n,
+                                                   const float *__restrict__ cand,
+                                                   const uint32_t *__restrict__ counts,
+                                                   int regions, uint32_t region_cap,
+                                                   const SelState *__restrict__ st,
+                                                   unsigned long long *__restrict__ hist)
 {
     __shared__ uint32_t h[kSelBins];
-    for (int b = threadIdx.x; b < kSelBins; b += blockDim.x)
+    if (st->done || (!keys && (st->missed || (!st->counted && !st->bracket_holds()))))
+        return;
+    const uint32_t lo = st->lo, span = st->span, shift = st->shift;
+    for (int b = threadIdx.x; b < kSelBins; b += 1024)
         h[b] = 0;
     __syncthreads();
-    const uint32_t prefix = st->prefix, mask = st->mask;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    // 4-wide unrolled stream
-    for (; i + 3 * stride < n; i += 4 * stride) {
-        uint32_t u0 = order_key(keys[i]);
-        uint32_t u1 = order_key(keys[i + stride]);
-        uint32_t u2 = order_key(keys[i + 2 * stride]);
-        uint32_t u3 = order_key(keys[i + 3 * stride]);
-        if ((u0 & mask) == prefix)
-            atomicAdd(&h[(u0 >> shift) & bin_mask], 1u);
-        if ((u1 & mask) == prefix)
-            atomicAdd(&h[(u1 >> shift) & bin_mask], 1u);
-        if ((u2 & mask) == prefix)
-            atomicAdd(&h[(u2 >> shift) & bin_mask], 1u);
-        if ((u3 & mask) == prefix)
-            atomicAdd(&h[(u3 >> shift) & bin_mask], 1u);
-    }
-    for (; i < n; i += stride) {
-        uint32_t u = order_key(keys[i]);
-        if ((u & mask) == prefix)
-            atomicAdd(&h[(u >> shift) & bin_mask], 1u);
+    const auto add = [&](float f) {
+        const uint32_t t = order_key(f) - lo;
+        if (t <= span)
+            atomicAdd(&h[t >> shift], 1u);
+    };
+    // four loads in flight
+    const auto stream = [&](const float *src, int64_t first, int64_t stride, int64_t count) {
+        int64_t i = first;
+        for (; i + 3 * stride < count; i += 4 * stride) {
+            const float f0 = src[i], f1 = src[i + stride], f2 = src[i + 2 * stride],
+                        f3 = src[i + 3 * stride];
+            add(f0);
+            add(f1);
+            add(f2);
+            add(f3);
+        }
+        for (; i < count; i += stride)
+            add(src[i]);
+    };
+    if (keys) {
+        stream(keys, (int64_t)blockIdx.x * 1024 + threadIdx.x, (int64_t)gridDim.x * 1024, n);
+    } else {
+        const int wave = blockIdx.x * 16 + (threadIdx.x >> 6);
+        for (int r = wave; r < regions; r += gridDim.x * 16)
+            stream(cand + (int64_t)r * region_cap, threadIdx.x & 63, 64, counts[r]);
     }
     __syncthreads();
-    for (int b = threadIdx.x; b < kSelBins; b += blockDim.x)
+    for (int b = threadIdx.x; b < kSelBins; b += 1024)
         if (h[b])
             atomicAdd(&hist[b], (unsigned long long)h[b]);
 }
 
-// one block: find the bin holding rank k, narrow the prefix, clear the
-// histogram for the next pass
-__global__ __launch_bounds__(256) void k_sel_pick(SelState *st, unsigned long long *hist,
-                                                  int shift, uint32_t bin_mask, int last)
+// One workgroup: narrows the keys in question to the bin of rank k (2 or 3
+// passes leave one key) and clears the histogram.
+__global__ __launch_bounds__(1024) void k_sel_pick(SelState *st, unsigned long long *hist,
+                                                   bool whole)
 {
-    __shared__ unsigned long long part[256];
-    __shared__ int found_bin;
-    __shared__ unsigned long long found_before;
-    const int per = kSelBins / 256; // 8 bins per thread
-    unsigned long long local[8];
-    unsigned long long sum = 0;
-    for (int q = 0; q < per; ++q) {
-        local[q] = hist[threadIdx.x * per + q];
-        sum += local[q];
-    }
-    part[threadIdx.x] = sum;
+    __shared__ unsigned long long sh[16];
+    SelState now = *st;
     __syncthreads();
-    // exclusive scan (Hillis-Steele on 256 entries)
-    for (int off = 1; off < 256; off <<= 1) {
-        unsigned long long v = threadIdx.x >= off ? part[threadIdx.x - off] : 0;
-        __syncthreads();
-        part[threadIdx.x] += v;
-        __syncthreads();
-    }
-    unsigned long long before = part[threadIdx.x] - sum;
-    const unsigned long long k = st->k;
-    if (threadIdx.x == 0)
-        found_bin = -1;
-    __syncthreads();
-    if (k >= before && k < before + sum) {
-        unsigned long long c = before;
-        for (int q = 0; q < per; ++q) {
-            if (k < c + local[q]) {
-                found_bin = threadIdx.x * per + q;
-                found_before = c;
-                break;
+    if (now.done || (now.missed && !whole)) // whole: the pass was over the array
+        return;
+    if (!now.counted) {
+        if (!now.bracket_holds()) {
+            if (threadIdx.x == 0) {
+                st->missed = st->counted = 1;
+                sel_whole_range(st);
             }
-            c += local[q];
+            return;
         }
+        now.k -= now.below;
     }
-    __syncthreads();
-    for (int q = 0; q < per; ++q)
-        hist[threadIdx.x * per + q] = 0;
-    if (threadIdx.x == 0 && found_bin >= 0) {
-        st->prefix |= ((uint32_t)found_bin & bin_mask) << shift;
-        st->mask |= bin_mask << shift;
-        st->k = k - found_before;
-        if (last)
-            st->result = key_float(st->prefix);
+    const int b0 = 2 * threadIdx.x;
+    const unsigned long long c0 = hist[b0], c1 = hist[b0 + 1];
+    hist[b0] = 0;
+    hist[b0 + 1] = 0;
+    const unsigned long long c = block_scan(c0 + c1, sh) - c0 - c1;
+    if (now.k < c || now.k >= c + c0 + c1)
+        return;
+    // one thread: rank k lies in one of its two bins
+    const bool second = now.k >= c + c0;
+    now.lo += (uint32_t)(b0 + (second ? 1 : 0)) << now.shift;
+    now.span = (1u << now.shift) - 1u;
+    now.k -= second ? c + c0 : c;
+    now.counted = 1;
+    if (now.shift == 0) {
+        now.result = key_float(now.lo);
+        now.done = 1;
     }
+    now.shift = sel_shift(now.span);
+    *st = now;
 }
 
 // ---- exclusive scan of int64 (in place, total appended at a[n]) ---------
@@ -244,15 +499,53 @@ __global__ __launch_bounds__(1024) void k_scan_apply(int64_t *__restrict__ a, in
 }
 
 // ---- edges ----------------------------------------------------------------
+// A row of the pair arrays in 16-byte units: rows start at any float, so unit
+// u covers the row's elements 4u - shift .. 4u - shift + 3, loaded as one
+// vector unless it runs over the row's ends.
+struct RowUnits {
+    const float *row;
+    int len, shift;
+
+    __device__ RowUnits(const float *r, int n) : row(r), len(n)
+    {
+        shift = (int)(((uintptr_t)r >> 2) & 3);
+    }
+    __device__ int units() const { return (len + shift + 3) >> 2; }
+    // elements outside the row read as +inf, below no threshold
+    __device__ float4 load(int u) const
+    {
+        const int k = 4 * u - shift;
+        if (k >= 0 && k + 4 <= len)
+            return *reinterpret_cast<const float4 *>(row + k);
+        const float none = INFINITY;
+        return make_float4(k >= 0 && k < len ? row[k] : none,
+                           k + 1 >= 0 && k + 1 < len ? row[k + 1] : none,
+                           k + 2 >= 0 && k + 2 < len ? row[k + 2] : none,
+                           k + 3 >= 0 && k + 3 < len ? row[k + 3] : none);
+    }
+};
+
+constexpr int kRowUnits = 8; // 16-byte units in flight per thread
+
+// Bound by the read: 256 MB in 38 us, 53 with 4-byte loads one at a time.
+
 __global__ __launch_bounds__(256) void k_count_rows(const float *__restrict__ copts, int num,
                                                     float rn, int64_t *__restrict__ counts)
 {
     __shared__ int sh[4];
     const int i = blockIdx.x;
-    const float *row = copts + (int64_t)i * (num - 1);
+    const RowUnits R(copts + (int64_t)i * (num - 1), num - 1);
+    const int n = R.units();
     int c = 0;
-    for (int k = threadIdx.x; k < num - 1; k += blockDim.x)
-        c += row[k] < rn;
+    for (int u0 = 0; u0 < n; u0 += 256 * kRowUnits) {
+        float4 v[kRowUnits];
+#pragma unroll
+        for (int j = 0; j < kRowUnits; ++j)
+            v[j] = R.load(u0 + j * 256 + threadIdx.x);
+#pragma unroll
+        for (int j = 0; j < kRowUnits; ++j)
+            c += (v[j].x < rn) + (v[j].y < rn) + (v[j].z < rn) + (v[j].w < rn);
+    }
     for (int off = 32; off > 0; off >>= 1)
         c += __shfl_down(c, off, 64);
     if ((threadIdx.x & 63) == 0)
@@ -262,6 +555,14 @@ __global__ __launch_bounds__(256) void k_count_rows(const float *__restrict__ co
         counts[i] = (int64_t)(sh[0] + sh[1] + sh[2] + sh[3]);
 }
 
+// Order-preserving compaction of one row: a thread's units come in strips of
+// 256, so the order is strip, then thread, then element.  A wave's place in a
+// strip comes from ballots, the strips' and waves' places from one scan of
+// their 4 * kRowUnits counts.  The kept elements' indexes go to LDS first, so
+// that the gathers of the two values are in flight together and the four
+// stores are coalesced.  Bound by the read of the costs and one line of topts
+// per edge; 8000 rows with 6 of 1000 kept: 131 us with 256 elements and two
+// barriers at a time, 67 us with the stores made by the element's lane, 55 us so.
 __global__ __launch_bounds__(256) void k_fill_rows(const float *__restrict__ copts,
                                                    const float *__restrict__ topts, int num,
                                                    float rn, const int64_t *__restrict__ row_start,
@@ -270,37 +571,63 @@ __global__ __launch_bounds__(256) void k_fill_rows(const float *__restrict__ cop
                                                    float *__restrict__ copts_edge,
                                                    float *__restrict__ topts_edge)
 {
-    __shared__ int wave_cnt[4];
+    __shared__ int cnt[kRowUnits * 4];
+    __shared__ uint16_t kept[kRowUnits * 256 * 4];
     const int i = blockIdx.x;
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     const int64_t rbase = (int64_t)i * (num - 1);
+    const RowUnits R(copts + rbase, num - 1);
+    const int n = R.units();
+    const uint64_t lower = (1ull << lane) - 1ull;
     int64_t out = row_start[i];
-    for (int k0 = 0; k0 < num - 1; k0 += 256) {
-        int k = k0 + threadIdx.x;
-        float c = 0.0f;
-        bool keep = false;
-        if (k < num - 1) {
-            c = copts[rbase + k];
-            keep = c < rn;
+    for (int u0 = 0; u0 < n; u0 += 256 * kRowUnits) {
+        int before[kRowUnits]; // kept elements of lower lanes in the strip
+        uint32_t mine = 0;     // 4 bits per strip
+        float4 v[kRowUnits];
+#pragma unroll
+        for (int j = 0; j < kRowUnits; ++j)
+            v[j] = R.load(u0 + j * 256 + threadIdx.x);
+#pragma unroll
+        for (int j = 0; j < kRowUnits; ++j) {
+            const uint64_t m0 = __ballot(v[j].x < rn), m1 = __ballot(v[j].y < rn),
+                           m2 = __ballot(v[j].z < rn), m3 = __ballot(v[j].w < rn);
+            before[j] = __popcll(m0 & lower) + __popcll(m1 & lower) + __popcll(m2 & lower) +
+                        __popcll(m3 & lower);
+            mine |= (uint32_t)((v[j].x < rn) | (v[j].y < rn) << 1 | (v[j].z < rn) << 2 |
+                               (v[j].w < rn) << 3)
+                    << (4 * j);
+            if (lane == 0)
+                cnt[j * 4 + wid] = __popcll(m0) + __popcll(m1) + __popcll(m2) + __popcll(m3);
         }
-        unsigned long long m = __ballot(keep);
-        int before_in_wave = __popcll(m & ((1ull << lane) - 1ull));
-        if (lane == 0)
-            wave_cnt[wid] = __popcll(m);
         __syncthreads();
-        int wave_before = 0;
-        for (int w = 0; w < wid; ++w)
-            wave_before += wave_cnt[w];
-        int chunk_total = wave_cnt[0] + wave_cnt[1] + wave_cnt[2] + wave_cnt[3];
-        if (keep) {
-            int64_t e = out + wave_before + before_in_wave;
-            int j = k + (k >= i ? 1 : 0);
-            edge_src[e] = i;
-            edge_dst[e] = j;
-            copts_edge[e] = c;
-            topts_edge[e] = topts[rbase + k];
+        int incl = lane < 4 * kRowUnits ? cnt[lane] : 0;
+        const int own = incl;
+        for (int off = 1; off < 4 * kRowUnits; off <<= 1) {
+            const int y = __shfl_up(incl, off, 64);
+            if (lane >= off)
+                incl += y;
         }
-        out += chunk_total;
+        const int excl = incl - own;
+#pragma unroll
+        for (int j = 0; j < kRowUnits; ++j) {
+            int e = __shfl(excl, j * 4 + wid, 64) + before[j];
+            uint32_t bits = (mine >> (4 * j)) & 15u;
+            while (bits) {
+                kept[e++] = (uint16_t)(4 * (j * 256 + (int)threadIdx.x) + __builtin_ctz(bits));
+                bits &= bits - 1u;
+            }
+        }
+        const int total = __shfl(incl, 4 * kRowUnits - 1, 64);
+        __syncthreads();
+        for (int q = threadIdx.x; q < total; q += 256) {
+            const int k = 4 * u0 - R.shift + kept[q];
+            const float c = R.row[k], t = topts[rbase + k];
+            edge_src[out + q] = i;
+            edge_dst[out + q] = k + (k >= i ? 1 : 0);
+            copts_edge[out + q] = c;
+            topts_edge[out + q] = t;
+        }
+        out += total;
         __syncthreads();
     }
 }
@@ -319,30 +646,66 @@ __global__ __launch_bounds__(256) void k_fill_i32(int *__restrict__ a, int64_t n
         a[i] = v;
 }
 
-__global__ __launch_bounds__(256) void k_in_degree(const int *__restrict__ edge_dst, int64_t n,
-                                                   int *__restrict__ indeg)
+// In-degrees, counted in LDS first: a workgroup takes a share of the edges
+// (blockIdx.x) and kDegTile destinations (blockIdx.y).  Bound by the device's
+// counters, 12 additions per ns: 4e5 edges into 8000 took 33 us one by one and
+// take 6 us with kDegShares workgroups that add 8000 counters each.
+constexpr int kDegTile = 16384;
+constexpr int kDegShares = 16;
+
+__global__ __launch_bounds__(1024) void k_in_degree(const int *__restrict__ edge_dst, int64_t n,
+                                                    int num, int *__restrict__ indeg)
 {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += stride)
-        atomicAdd(&indeg[edge_dst[e]], 1);
+    extern __shared__ int deg[];
+    const int d0 = blockIdx.y * kDegTile;
+    const int nd = min(num - d0, kDegTile);
+    for (int d = threadIdx.x; d < nd; d += 1024)
+        deg[d] = 0;
+    __syncthreads();
+    const int64_t stride = (int64_t)gridDim.x * 1024;
+    int64_t e = (int64_t)blockIdx.x * 1024 + threadIdx.x;
+    const auto add = [&](int dst) {
+        if ((unsigned)(dst - d0) < (unsigned)nd)
+            atomicAdd(&deg[dst - d0], 1);
+    };
+    for (; e + 7 * stride < n; e += 8 * stride) {
+        int dst[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            dst[j] = edge_dst[e + j * stride];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            add(dst[j]);
+    }
+    for (; e < n; e += stride)
+        add(edge_dst[e]);
+    __syncthreads();
+    for (int d = threadIdx.x; d < nd; d += 1024)
+        if (deg[d])
+            atomicAdd(&indeg[d0 + d], deg[d]);
 }
 
-__global__ __launch_bounds__(256) void k_max_deg(const int64_t *__restrict__ row_start,
-                                                 const int *__restrict__ indeg, int num,
-                                                 int *__restrict__ out)
+// one workgroup: the largest degree
+__global__ __launch_bounds__(1024) void k_max_deg(const int64_t *__restrict__ row_start,
+                                                  const int *__restrict__ indeg, int num,
+                                                  int *__restrict__ out)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ int sh[16];
     int m = 0;
-    if (i < num) {
-        int go = (int)(row_start[i + 1] - row_start[i]);
-        m = go > indeg[i] ? go : indeg[i];
+    for (int i = threadIdx.x; i < num; i += 1024) {
+        const int go = (int)(row_start[i + 1] - row_start[i]);
+        m = max(m, max(go, indeg[i]));
     }
-    for (int off = 32; off > 0; off >>= 1) {
-        int o = __shfl_down(m, off, 64);
-        m = o > m ? o : m;
-    }
+    for (int off = 32; off > 0; off >>= 1)
+        m = max(m, __shfl_xor(m, off, 64));
     if ((threadIdx.x & 63) == 0)
-        atomicMax(out, m);
+        sh[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 16; ++w)
+            m = max(m, sh[w]);
+        *out = m;
+    }
 }
 
 __global__ __launch_bounds__(256) void k_nn_go(const int64_t *__restrict__ row_start,
@@ -470,42 +833,81 @@ extern "C" int64_t pump_rn_index(int64_t num, float rn_perc)
     return (int64_t)prod;
 }
 
-extern "C" size_t pump_select_rn_workspace(int64_t)
+// state and histogram; the bracket's keys follow when the workspace holds them
+constexpr size_t kSelHist = 280;
+static_assert(sizeof(SelState) <= kSelHist && kSelHist % 8 == 0, "layout of the selection");
+static size_t select_rn_base() { return kSelHist + kSelBins * sizeof(unsigned long long); }
+
+// room for the bracket's keys, 10 sqrt(16384 p) + 8 of 16384 (at most 4%) when
+// a share p or 1 - p of the keys lies below, in equal regions
+static int64_t select_rn_cand(int64_t n) { return n <= kSelSample ? 0 : n / 16 + 131072; }
+
+extern "C" size_t pump_select_rn_workspace(int64_t n_pairs)
 {
-    return sizeof(SelState) + 256 + kSelBins * sizeof(unsigned long long);
+    return select_rn_base() + kSelMaxRegions * sizeof(uint32_t) +
+           (size_t)select_rn_cand(n_pairs) * sizeof(float);
 }
 
 extern "C" int pump_select_rn(const float *d_copts, int64_t n_pairs, int64_t rn_idx, float *rn_host,
                               void *d_ws, size_t ws_bytes, pump_stream_t stream)
 {
     PUMP_REQUIRE(d_copts && rn_host && n_pairs > 0 && rn_idx >= 0 && rn_idx < n_pairs);
-    if (!d_ws || ws_bytes < pump_select_rn_workspace(n_pairs))
+    if (!d_ws || ws_bytes < select_rn_base())
         return PUMP_E_CAPACITY;
     hipStream_t s = as_stream(stream);
     SelState *st = reinterpret_cast<SelState *>(d_ws);
     unsigned long long *hist =
-        reinterpret_cast<unsigned long long *>(reinterpret_cast<char *>(d_ws) + sizeof(SelState) + 256);
-    hipLaunchKernelGGL(k_sel_init, dim3(1), dim3(256), 0, s, st, hist,
-                       (unsigned long long)rn_idx);
-    PUMP_LAUNCHED();
-    const int shifts[3] = {21, 10, 0};
-    const uint32_t masks[3] = {0x7ffu, 0x7ffu, 0x3ffu};
+        reinterpret_cast<unsigned long long *>(reinterpret_cast<char *>(d_ws) + kSelHist);
+    uint32_t *counts = reinterpret_cast<uint32_t *>(hist + kSelBins);
+    float *cand = reinterpret_cast<float *>(counts + kSelMaxRegions);
+    const unsigned long long k = (unsigned long long)rn_idx;
     int dev = 0, cus = 256;
     hipGetDevice(&dev);
     hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    unsigned blocks = grid_for(n_pairs / 4 + 1, 256, (int64_t)cus * 8);
-    for (int p = 0; p < 3; ++p) {
-        hipLaunchKernelGGL(k_sel_hist, dim3(blocks), dim3(256), 0, s, d_copts, n_pairs, st,
-                           shifts[p], masks[p], hist);
+    const int regions = (int)grid_for(n_pairs, kSelTile, std::min(cus * 4, kSelMaxRegions));
+    const uint32_t region_cap = (uint32_t)(select_rn_cand(n_pairs) / regions);
+    const auto pass = [&](const float *keys) {
+        const unsigned blocks = keys ? grid_for(n_pairs / 4 + 1, 1024, (int64_t)cus * 2) : 16u;
+        hipLaunchKernelGGL(k_sel_pass, dim3(blocks), dim3(1024), 0, s, keys, n_pairs, cand, counts,
+                           regions, region_cap, st, hist);
+        hipLaunchKernelGGL(k_sel_pick, dim3(1), dim3(1024), 0, s, st, hist,
+                           keys != nullptr);
+    };
+    const bool bracket = ws_bytes >= pump_select_rn_workspace(n_pairs);
+    if (bracket) {
+        hipLaunchKernelGGL(k_sel_sample, dim3(1), dim3(1024), 0, s, d_copts, n_pairs, k, st, hist);
         PUMP_LAUNCHED();
-        hipLaunchKernelGGL(k_sel_pick, dim3(1), dim3(256), 0, s, st, hist, shifts[p], masks[p],
-                           p == 2 ? 1 : 0);
+        if (n_pairs > kSelSample) {
+            hipLaunchKernelGGL(k_sel_bracket, dim3(regions), dim3(256), 0, s, d_copts, n_pairs, st,
+                               cand, counts, region_cap);
+            PUMP_LAUNCHED();
+            pass(nullptr);
+            PUMP_LAUNCHED();
+            pass(nullptr);
+            PUMP_LAUNCHED();
+        }
+    } else {
+        hipLaunchKernelGGL(k_sel_init, dim3(1), dim3(256), 0, s, st, hist, k);
         PUMP_LAUNCHED();
+        for (int p = 0; p < 3; ++p) {
+            pass(d_copts);
+            PUMP_LAUNCHED();
+        }
     }
-    float rn = 0.0f;
-    PUMP_HIP(hipMemcpyAsync(&rn, &st->result, sizeof(float), hipMemcpyDeviceToHost, s));
+    SelState got;
+    PUMP_HIP(hipMemcpyAsync(&got, st, sizeof(got), hipMemcpyDeviceToHost, s));
     PUMP_HIP(hipStreamSynchronize(s));
-    *rn_host = rn;
+    if (!got.done) {
+        // a bracket of more than 22 bits needs one more pass over its keys; one
+        // that missed rank k needs three over the array
+        for (int p = 0; p < (got.missed ? 3 : 1); ++p) {
+            pass(got.missed ? d_copts : nullptr);
+            PUMP_LAUNCHED();
+        }
+        PUMP_HIP(hipMemcpyAsync(&got, st, sizeof(got), hipMemcpyDeviceToHost, s));
+        PUMP_HIP(hipStreamSynchronize(s));
+    }
+    *rn_host = got.result;
     return PUMP_OK;
 }
 
@@ -554,12 +956,13 @@ extern "C" int pump_max_nn_size(const int64_t *d_row_start, const int *d_edge_ds
     PUMP_HIP(hipMalloc((void **)&d_max, sizeof(int)));
     hipLaunchKernelGGL(k_zero_i32, dim3(grid_for(num + 1, 256)), dim3(256), 0, s, d_in_degree,
                        (int64_t)num);
-    hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(64), 0, s, d_max, (int64_t)1);
     if (n_edges > 0)
-        hipLaunchKernelGGL(k_in_degree, dim3(grid_for(n_edges, 256)), dim3(256), 0, s, d_edge_dst,
-                           n_edges, d_in_degree);
-    hipLaunchKernelGGL(k_max_deg, dim3((num + 255) / 256), dim3(256), 0, s, d_row_start,
-                       d_in_degree, num, d_max);
+        hipLaunchKernelGGL(k_in_degree,
+                           dim3(grid_for(n_edges, 4096, kDegShares),
+                                (unsigned)((num + kDegTile - 1) / kDegTile)),
+                           dim3(1024), sizeof(int) * (size_t)std::min(num, kDegTile), s,
+                           d_edge_dst, n_edges, num, d_in_degree);
+    hipLaunchKernelGGL(k_max_deg, dim3(1), dim3(1024), 0, s, d_row_start, d_in_degree, num, d_max);
     hipError_t le = hipGetLastError();
     int m = 0;
     hipError_t ce = hipMemcpyAsync(&m, d_max, sizeof(int), hipMemcpyDeviceToHost, s);
