@@ -24,10 +24,12 @@ namespace pump {
 namespace {
 
 constexpr int kEdgesPerBlock = 128;
+constexpr int kEdges32PerBlock = 128;
 constexpr int kTile = 256;
 
 constexpr int kEdgeObs = 256;                  // boxes staged in LDS by the edge pass
 constexpr int kEdgeMaskWords = kEdgeObs / 64;  // candidate-mask words per edge
+constexpr int kSlabs = 16;                     // slabs per axis of the slab table
 constexpr int kMapCap = 2016;                  // block waypoints mapped to their edge in LDS
 
 // Per-edge record of an edge-pass workgroup in LDS: everything a lane needs
@@ -233,7 +235,7 @@ constexpr int kRetestCap = 512;
 
 __host__ __device__ inline EdgeLds edge_lds(int epb, int obs_cap, int words_cap,
                                             int rec_bytes = (int)sizeof(EdgeRec),
-                                            int retest_cap = 0)
+                                            int retest_cap = 0, bool slab = false)
 {
     EdgeLds L{};
     int o = 0;
@@ -245,7 +247,7 @@ __host__ __device__ inline EdgeLds edge_lds(int epb, int obs_cap, int words_cap,
     };
     L.recs = take(epb * rec_bytes, 16);
     L.obs = take(obs_cap * (int)sizeof(BoxRec), 16);
-    L.emask = take(epb * words_cap * 8, 8);
+    L.emask = take((slab ? 6 * kSlabs : epb) * words_cap * 8, 8); // masks or slab table
     L.loff = take((epb + 1) * 4, 4);
     L.ok = take(epb, 4);
     L.wmap = take(kMapCap, 4);
@@ -332,18 +334,124 @@ __device__ __forceinline__ void candidate_masks(bool own, const float *x0, const
     }
 }
 
+// Slab table (many boxes): which staged boxes a segment can meet, looked up
+// per segment instead of kept per edge.  The boxes' extent is cut into kSlabs
+// slabs per axis; row (2 d, s) holds the boxes not separated by
+// bbMax_d <= lo_d from some box of segments with bbMax_d in slab s counted
+// from the top, row (2 d + 1, s) those not separated by hi_d <= bbMin_d with
+// bbMin_d in slab s from the bottom.  The AND of a segment's six rows holds
+// every box that the reference's broad phase (collisionCheck.cu:104-112) does
+// not reject: lo_d < bbMax_d gives top - lo_d >= top - bbMax_d, and the
+// subtraction, the product with inv >= 0 and the truncation are monotone, so
+// the box's slab is not below the segment's; the same with hi_d from below.
+// Slab 0 holds every box; NaN goes there (segment) or everywhere (box).
+struct SlabAxes {
+    float base[3], top[3], inv[3]; // lower, upper end of the extent, slabs per length
+};
+
+// slab of a distance from the extent's end, in [0, kSlabs - 1]; NaN: 0
+__device__ __forceinline__ int slab_of(float dist, float inv)
+{
+    return (int)fminf(fmaxf(dist * inv, 0.0f), (float)(kSlabs - 1));
+}
+
+// a value that is the same in every lane, in a scalar register
+__device__ __forceinline__ float uniform(float x)
+{
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x)));
+}
+
+// the extent of the first 64 staged boxes' finite bounds (whole waves, the
+// same in every lane); no finite extent: one slab.  Any extent would do: a
+// box past it is in the end slab.
+__device__ __forceinline__ SlabAxes slab_axes(const float *__restrict__ obstacles, int n_masked)
+{
+    const int b = (threadIdx.x & 63) < n_masked ? (threadIdx.x & 63) : n_masked - 1;
+    float x[6];
+    for (int d = 0; d < 3; ++d) {
+        x[d] = obstacles[b * 12 + d];
+        x[3 + d] = obstacles[b * 12 + 6 + d];
+    }
+    SlabAxes A;
+    for (int d = 0; d < 3; ++d) {
+        const bool ok = fabsf(x[d]) < INFINITY && fabsf(x[3 + d]) < INFINITY;
+        const float lo = uniform(wave_min(ok ? fminf(x[d], x[3 + d]) : INFINITY));
+        const float hi = uniform(wave_max(ok ? fmaxf(x[d], x[3 + d]) : -INFINITY));
+        const float inv = (float)kSlabs / (hi - lo);
+        const bool cut = hi > lo && inv < INFINITY; // an overflowed hi - lo gives inv = 0
+        A.base[d] = cut ? lo : 0.0f;
+        A.top[d] = cut ? hi : 0.0f;
+        A.inv[d] = cut ? inv : 0.0f;
+    }
+    return A;
+}
+
+// rows of the boxes of word wd: lane = box; entry s of a row is the ballot of
+// the boxes that slab s holds, kept by lane s
+__device__ __forceinline__ void slab_rows(const SlabAxes &A, const float *__restrict__ obstacles,
+                                          int n_masked, int n_words, int wd,
+                                          unsigned long long *__restrict__ tab)
+{
+    const int lane = threadIdx.x & 63, b = wd * 64 + lane;
+    float x[6]; // lo_d, hi_d
+    for (int row = 0; row < 6; ++row)
+        x[row] = b < n_masked ? obstacles[b * 12 + (row & 1 ? 6 : 0) + (row >> 1)] : 0.0f;
+#pragma unroll
+    for (int row = 0; row < 6; ++row) {
+        const int d = row >> 1;
+        // the last slab that holds this lane's box
+        int n = x[row] != x[row] ? kSlabs - 1
+                                 : slab_of(row & 1 ? x[row] - A.base[d] : A.top[d] - x[row],
+                                           A.inv[d]);
+        n = b < n_masked ? n : -1;
+        unsigned long long mine = 0ull;
+#pragma unroll
+        for (int s = 0; s < kSlabs; ++s) {
+            const unsigned long long m = __ballot(n >= s);
+            mine = lane == s ? m : mine;
+        }
+        if (lane < kSlabs)
+            tab[(row * kSlabs + lane) * n_words + wd] = mine;
+    }
+}
+
+// The staged boxes that a segment is tested against, 64 to a word: those of
+// its edge, or those of its own bounds in the slab table.
+struct EdgeBoxes {
+    const unsigned long long *row;
+    __device__ unsigned long long word(int wd) const { return row[wd]; }
+};
+
+struct SlabBoxes {
+    const unsigned long long *tab;
+    int at[6];
+    __device__ SlabBoxes(const unsigned long long *t, const SlabAxes &A, int n_words,
+                         const float *bmin, const float *bmax)
+        : tab(t)
+    {
+        for (int d = 0; d < 3; ++d) {
+            at[2 * d] = (2 * d * kSlabs + slab_of(A.top[d] - bmax[d], A.inv[d])) * n_words;
+            at[2 * d + 1] = ((2 * d + 1) * kSlabs + slab_of(bmin[d] - A.base[d], A.inv[d])) * n_words;
+        }
+    }
+    __device__ unsigned long long word(int wd) const
+    {
+        return (tab[at[0] + wd] & tab[at[1] + wd]) & (tab[at[2] + wd] & tab[at[3] + wd]) &
+               (tab[at[4] + wd] & tab[at[5] + wd]);
+    }
+};
+
 // Phase 1 of the FP32 form's decision for segment v -> w of an edge: true
 // when some candidate box is not separated from it by the margin-widened
 // broad phase (a few segments in a hundred).  Only those are decided further.
-__device__ __forceinline__ bool seg_near32(const float *v, const float *w, const EdgeRec32 &R,
-                                           const unsigned long long *emask_row, int n_words,
+template <typename Boxes>
+__device__ __forceinline__ bool seg_near32(const SegBox &sb, const Boxes &cand, int n_words,
                                            const BoxRec *boxes, const float *__restrict__ obstacles,
                                            int n_masked, int n_obs)
 {
-    const SegBox sb = seg_box32(v, w, R.m);
     bool near = false;
     for (int wd = 0; wd < n_words && !near; ++wd) {
-        unsigned long long mk = emask_row[wd];
+        unsigned long long mk = cand.word(wd);
         while (mk && !near) {
             const BoxRec B = boxes[wd * 64 + __builtin_ctzll(mk)];
             mk &= mk - 1;
@@ -364,15 +472,15 @@ __device__ __forceinline__ bool seg_near32(const float *v, const float *w, const
 // candidate boxes, kMiss when it surely misses all of them, else kUndecided
 // (left to the exact re-test).  Boxes separated by the widened broad phase
 // are misses; the others go through classify32.
+template <typename Boxes>
 __device__ __forceinline__ int seg_state32(const float *v, const float *w, const EdgeRec32 &R,
-                                           const unsigned long long *emask_row, int n_words,
+                                           const SegBox &sb, const Boxes &cand, int n_words,
                                            const BoxRec *boxes, const float *__restrict__ obstacles,
                                            int n_masked, int n_obs)
 {
-    const SegBox sb = seg_box32(v, w, R.m);
     int state = kMiss;
     for (int wd = 0; wd < n_words && state != kHit; ++wd) {
-        unsigned long long mk = emask_row[wd];
+        unsigned long long mk = cand.word(wd);
         while (mk && state != kHit) {
             const BoxRec B = boxes[wd * 64 + __builtin_ctzll(mk)];
             mk &= mk - 1;
@@ -398,10 +506,12 @@ __device__ __forceinline__ int seg_state32(const float *v, const float *w, const
 // FP64 waypoints k and k+1 (pathPoint, 2pBVP.cu:117-131, from the edge's
 // EdgePoly) against the edge's candidate boxes (collisionCheck.cu:65-143).
 // A hit clears the edge's flag (only zeros are written: concurrent writes
-// agree).  Out of line: it runs a few times per pass, and its FP64
+// agree).  cand holds the boxes near the segment widened by its margin, and
+// so those near the exact one.  Out of line: it runs a few times per pass, and its FP64
 // registers, and any spills, stay off the rest of the kernel.
-__device__ __noinline__ void exact32(const EdgeRec32 *recs, const int *loff,
-                                     const unsigned long long *emask_row, int n_words,
+template <typename Boxes>
+__device__ __noinline__ void exact32(const EdgeRec32 *recs, const int *loff, const Boxes cand,
+                                     int n_words,
                                      const BoxRec *boxes, const float *__restrict__ obstacles,
                                      int n_masked, int n_obs, uint8_t *ok, int le, int k)
 {
@@ -416,7 +526,7 @@ __device__ __noinline__ void exact32(const EdgeRec32 *recs, const int *loff,
     seg_bbox(ve, we, bmin, bmax);
     bool hit = false;
     for (int wd = 0; wd < n_words && !hit; ++wd) {
-        unsigned long long m = emask_row[wd];
+        unsigned long long m = cand.word(wd);
         while (m && !hit) {
             const BoxRec B = boxes[wd * 64 + __builtin_ctzll(m)];
             m &= m - 1;
@@ -436,23 +546,25 @@ __device__ __noinline__ void exact32(const EdgeRec32 *recs, const int *loff,
 // A listed segment, decided after the tiles: from its FP32 waypoints by
 // seg_state32 (a sure hit clears the edge's flag), by exact32 when
 // undecided.  Returns 1 when the exact re-test ran.
+template <typename BoxesOf>
 __device__ __forceinline__ int decide32(const EdgeRec32 *recs, const int *loff,
-                                        const unsigned long long *emask, int n_words,
+                                        const BoxesOf &boxes_of, int n_words,
                                         const BoxRec *boxes, const float *__restrict__ obstacles,
                                         int n_masked, int n_obs, uint8_t *ok, int le, int k)
 {
     const EdgeRec32 &R = recs[le];
     const int Wq = loff[le + 1] - loff[le];
-    const unsigned long long *emask_row = emask + le * n_words;
     float v[kDim], w[kDim];
     waypoint32(R, k, Wq, v);
     waypoint32(R, k + 1, Wq, w);
-    const int st = seg_state32(v, w, R, emask_row, n_words, boxes, obstacles, n_masked, n_obs);
+    const SegBox sb = seg_box32(v, w, R.m);
+    const auto cand = boxes_of(le, sb.dn, sb.up);
+    const int st = seg_state32(v, w, R, sb, cand, n_words, boxes, obstacles, n_masked, n_obs);
     if (st == kHit)
         ok[le] = 0;
     if (st != kUndecided)
         return 0;
-    exact32(recs, loff, emask_row, n_words, boxes, obstacles, n_masked, n_obs, ok, le, k);
+    exact32(recs, loff, cand, n_words, boxes, obstacles, n_masked, n_obs, ok, le, k);
     return 1;
 }
 
@@ -467,7 +579,8 @@ __device__ __forceinline__ int decide32(const EdgeRec32 *recs, const int *loff,
 // far end of its segment from the next lane (DPP), and tests the segment
 // against its edge's candidate boxes only.  An edge already known to be
 // blocked skips its remaining segments, and a lane stops at its first hit.
-template <bool kCheck, bool kWrite, int EPB, bool kF32 = false>
+// kSlab: a slab table takes the place of the edges' masks.
+template <bool kCheck, bool kWrite, int EPB, bool kF32 = false, bool kSlab = false>
 __device__ __forceinline__ void edge_block(const EdgeJob &J, int64_t e0, char *smem, int obs_cap,
                                            int words_cap,
                                            unsigned long long *__restrict__ retests = nullptr)
@@ -484,7 +597,8 @@ __device__ __forceinline__ void edge_block(const EdgeJob &J, int64_t e0, char *s
     const int n_obs = J.n_obs;
     uint8_t *__restrict__ is_free = J.is_free;
     constexpr int kWaves = kTile / 64;
-    const EdgeLds L = edge_lds(EPB, obs_cap, words_cap, (int)sizeof(Rec), kF32 ? kRetestCap : 0);
+    const EdgeLds L =
+        edge_lds(EPB, obs_cap, words_cap, (int)sizeof(Rec), kF32 ? kRetestCap : 0, kSlab);
     Rec *recs = reinterpret_cast<Rec *>(smem + L.recs);           // per-edge records
     BoxRec *boxes = reinterpret_cast<BoxRec *>(smem + L.obs);     // staged boxes
     unsigned long long *emask = reinterpret_cast<unsigned long long *>(smem + L.emask);
@@ -566,8 +680,22 @@ __device__ __forceinline__ void edge_block(const EdgeJob &J, int64_t e0, char *s
             for (int j = 0; j < W; ++j)
                 wmap[a + j] = (uint8_t)q;
     }
-    if (kCheck && n_words > 0 && part == kMaskPart)
+    SlabAxes axes{};
+    if constexpr (kCheck && kSlab) {
+        axes = slab_axes(obstacles, n_masked);
+        // one word per wave, from the waves without records on
+        for (int wd = kWaves - 1 - wid; wd < n_words; wd += kWaves)
+            slab_rows(axes, obstacles, n_masked, n_words, wd, emask);
+    } else if (kCheck && n_words > 0 && part == kMaskPart) {
         candidate_masks(own, x0, x1, tau, obstacles, n_masked, n_words, emask + q * n_words);
+    }
+    // the staged boxes for a segment of edge le with these bounds
+    const auto boxes_of = [&](int le, const float *bmin, const float *bmax) {
+        if constexpr (kSlab)
+            return SlabBoxes(emask, axes, n_words, bmin, bmax);
+        else
+            return EdgeBoxes{emask + le * n_words};
+    };
     __syncthreads();
 
     // tiles start every 63 waypoints; tile j belongs to wave j % kWaves
@@ -605,8 +733,9 @@ __device__ __forceinline__ void edge_block(const EdgeJob &J, int64_t e0, char *s
             // surely clear is listed, and decided after the tiles by the
             // whole workgroup at once
             const float v[3] = {x[0], x[1], x[2]};
-            if (seg_near32(v, w, reinterpret_cast<const EdgeRec32 *>(recs)[le],
-                           emask + le * n_words, n_words, boxes, obstacles, n_masked, n_obs)) {
+            const SegBox sb = seg_box32(v, w, reinterpret_cast<const EdgeRec32 *>(recs)[le].m);
+            if (seg_near32(sb, boxes_of(le, sb.dn, sb.up), n_words, boxes, obstacles, n_masked,
+                           n_obs)) {
                 const int i = atomicAdd(rcnt, 1);
                 if (i < kRetestCap)
                     rlist[i] = ((uint32_t)le << 24) | (uint32_t)k;
@@ -617,8 +746,9 @@ __device__ __forceinline__ void edge_block(const EdgeJob &J, int64_t e0, char *s
             float bmin[3], bmax[3];
             seg_bbox(v, w, bmin, bmax);
             bool hit = false;
+            const auto cand = boxes_of(le, bmin, bmax);
             for (int wd = 0; wd < n_words && !hit; ++wd) {
-                unsigned long long m = emask[le * n_words + wd];
+                unsigned long long m = cand.word(wd);
                 while (m && !hit) {
                     const int b = wd * 64 + __builtin_ctzll(m);
                     m &= m - 1;
@@ -649,7 +779,7 @@ __device__ __forceinline__ void edge_block(const EdgeJob &J, int64_t e0, char *s
                 const uint32_t r = rlist[i];
                 const int le = (int)(r >> 24), k = (int)(r & 0xffffffu);
                 if (ok[le])
-                    n_exact += decide32(reinterpret_cast<const EdgeRec32 *>(recs), loff, emask,
+                    n_exact += decide32(reinterpret_cast<const EdgeRec32 *>(recs), loff, boxes_of,
                                         n_words, boxes, obstacles, n_masked, n_obs, ok, le,
                                         k);
             }
@@ -666,9 +796,10 @@ __device__ __forceinline__ void edge_block(const EdgeJob &J, int64_t e0, char *s
                 float v[kDim], w[kDim];
                 waypoint32(R, k, Wq, v);
                 waypoint32(R, k + 1, Wq, w);
-                if (seg_near32(v, w, R, emask + le * n_words, n_words, boxes, obstacles, n_masked,
+                const SegBox sb = seg_box32(v, w, R.m);
+                if (seg_near32(sb, boxes_of(le, sb.dn, sb.up), n_words, boxes, obstacles, n_masked,
                                n_obs))
-                    n_exact += decide32(reinterpret_cast<const EdgeRec32 *>(recs), loff, emask,
+                    n_exact += decide32(reinterpret_cast<const EdgeRec32 *>(recs), loff, boxes_of,
                                         n_words, boxes, obstacles, n_masked, n_obs, ok, le, k);
             }
         }
@@ -683,7 +814,7 @@ __device__ __forceinline__ void edge_block(const EdgeJob &J, int64_t e0, char *s
     }
 }
 
-template <bool kCheck, bool kWrite, int EPB>
+template <bool kCheck, bool kWrite, int EPB, bool kSlab>
 __global__ __launch_bounds__(kTile) void k_edges(
     const float *__restrict__ samples, const int *__restrict__ edge_src,
     const int *__restrict__ edge_dst, const float *__restrict__ topts_edge, int64_t n_edges,
@@ -694,12 +825,13 @@ __global__ __launch_bounds__(kTile) void k_edges(
     const EdgeJob J{samples, edge_src, edge_dst, topts_edge, n_edges, wp_offsets,
                     w_fixed, obstacles, n_obs, disc, is_free};
     const int cap = kCheck ? edge_obs_cap(n_obs) : 0;
-    edge_block<kCheck, kWrite, EPB>(J, (int64_t)blockIdx.x * EPB, smem, cap, edge_words(cap));
+    edge_block<kCheck, kWrite, EPB, false, kSlab>(J, (int64_t)blockIdx.x * EPB, smem, cap,
+                                                  edge_words(cap));
 }
 
 // the fused edge pass with FP32 waypoints and exact flags (chosen form)
-template <bool kWrite, int EPB>
-__global__ __launch_bounds__(kTile, 8) void k_edges32(
+template <bool kWrite, int EPB, bool kSlab>
+__global__ __launch_bounds__(kTile, kSlab ? 7 : 8) void k_edges32(
     const float *__restrict__ samples, const int *__restrict__ edge_src,
     const int *__restrict__ edge_dst, const float *__restrict__ topts_edge, int64_t n_edges,
     const int64_t *__restrict__ wp_offsets, int w_fixed, const float *__restrict__ obstacles,
@@ -710,8 +842,8 @@ __global__ __launch_bounds__(kTile, 8) void k_edges32(
     const EdgeJob J{samples, edge_src, edge_dst, topts_edge, n_edges, wp_offsets,
                     w_fixed, obstacles, n_obs, disc, is_free};
     const int cap = edge_obs_cap(n_obs);
-    edge_block<true, kWrite, EPB, true>(J, (int64_t)blockIdx.x * EPB, smem, cap, edge_words(cap),
-                                        retests);
+    edge_block<true, kWrite, EPB, true, kSlab>(J, (int64_t)blockIdx.x * EPB, smem, cap,
+                                               edge_words(cap), retests);
 }
 
 // the fused edge pass of many instances in one launch; LDS holds obs_cap
@@ -829,22 +961,38 @@ static int edges_per_block()
     return v;
 }
 
-template <bool kCheck, bool kWrite, int EPB>
+// The slab table from this many boxes on: more than one word of them.  Its
+// rows cost every workgroup some 300 instructions per word and every segment 6
+// LDS reads per word, the edges' masks 20 instructions per box that meets a
+// wave's edges and a test per candidate and segment.  800,000 edges, random
+// boxes, masks and table: 30 boxes 56 and 61 us (FP32 waypoints 50 and 57), 64
+// boxes 71 and 64 (67 and 61), 128 boxes 118 and 79 (124 and 82); in the
+// corridor world, 1.6 million edges, 50 boxes 104 and 116 (FP32 waypoints),
+// 200 boxes 357 and 282.
+constexpr int kSlabMinObs = 65;
+
+template <bool kCheck, bool kWrite, int EPB, bool kSlab = false>
 static int launch_edges(const float *d_samples, const int *d_edge_src, const int *d_edge_dst,
                         const float *d_topts_edge, int64_t n_edges, const int64_t *d_wp_offsets,
                         int waypoints_count, const float *d_obstacles, int n_obs, float *d_disc,
                         uint8_t *d_is_free, hipStream_t s)
 {
+    if constexpr (kCheck && !kSlab)
+        if (n_obs >= kSlabMinObs)
+            return launch_edges<kCheck, kWrite, EPB, true>(
+                d_samples, d_edge_src, d_edge_dst, d_topts_edge, n_edges, d_wp_offsets,
+                waypoints_count, d_obstacles, n_obs, d_disc, d_is_free, s);
     const int64_t nb = (n_edges + EPB - 1) / EPB;
     if (nb > 0x7fffffff)
         return PUMP_E_RANGE;
     const int cap = kCheck ? edge_obs_cap(n_obs) : 0;
-    const size_t lds = (size_t)edge_lds(EPB, cap, edge_words(cap)).bytes;
-    const void *fn = reinterpret_cast<const void *>(&k_edges<kCheck, kWrite, EPB>);
+    const size_t lds =
+        (size_t)edge_lds(EPB, cap, edge_words(cap), (int)sizeof(EdgeRec), 0, kSlab).bytes;
+    const void *fn = reinterpret_cast<const void *>(&k_edges<kCheck, kWrite, EPB, kSlab>);
     const int r = allow_lds(fn, lds);
     if (r != PUMP_OK)
         return r;
-    hipLaunchKernelGGL((k_edges<kCheck, kWrite, EPB>), dim3((unsigned)nb), dim3(kTile), lds, s,
+    hipLaunchKernelGGL((k_edges<kCheck, kWrite, EPB, kSlab>), dim3((unsigned)nb), dim3(kTile), lds, s,
                        d_samples, d_edge_src, d_edge_dst, d_topts_edge, n_edges, d_wp_offsets,
                        waypoints_count, d_obstacles, n_obs, d_disc, d_is_free);
     PUMP_LAUNCHED();
@@ -928,35 +1076,29 @@ extern "C" int pump_edges_discretize_check_fp32(
     PUMP_REQUIRE(n_obs == 0 || d_obstacles);
     PUMP_REQUIRE(d_wp_offsets || waypoints_count >= 2);
     PUMP_REQUIRE(waypoints_count < kMaxWaypointsPerEdge);
-    constexpr int EPB = 128;
-    const int64_t nb = (n_edges + EPB - 1) / EPB;
-    if (nb > 0x7fffffff)
-        return PUMP_E_RANGE;
-    const int cap = edge_obs_cap(n_obs);
-    const size_t lds =
-        (size_t)edge_lds(EPB, cap, edge_words(cap), (int)sizeof(EdgeRec32), kRetestCap).bytes;
-    hipStream_t s = as_stream(stream);
-    if (d_disc_motions) {
-        const void *fn = reinterpret_cast<const void *>(&k_edges32<true, EPB>);
-        int r = allow_lds(fn, lds);
+    const bool slab = n_obs >= kSlabMinObs;
+    const auto launch = [&](auto kernel) -> int {
+        const int64_t nb = (n_edges + kEdges32PerBlock - 1) / kEdges32PerBlock;
+        if (nb > 0x7fffffff)
+            return PUMP_E_RANGE;
+        const int cap = edge_obs_cap(n_obs);
+        const size_t lds = (size_t)edge_lds(kEdges32PerBlock, cap, edge_words(cap),
+                                            (int)sizeof(EdgeRec32), kRetestCap, slab)
+                               .bytes;
+        const int r = allow_lds(reinterpret_cast<const void *>(kernel), lds);
         if (r != PUMP_OK)
             return r;
-        hipLaunchKernelGGL((k_edges32<true, EPB>), dim3((unsigned)nb), dim3(kTile), lds, s,
+        hipLaunchKernelGGL(kernel, dim3((unsigned)nb), dim3(kTile), lds, as_stream(stream),
                            d_samples, d_edge_src, d_edge_dst, d_topts_edge, n_edges, d_wp_offsets,
                            waypoints_count, d_obstacles, n_obs, d_disc_motions, d_is_free_edges,
                            d_retests);
-    } else {
-        const void *fn = reinterpret_cast<const void *>(&k_edges32<false, EPB>);
-        int r = allow_lds(fn, lds);
-        if (r != PUMP_OK)
-            return r;
-        hipLaunchKernelGGL((k_edges32<false, EPB>), dim3((unsigned)nb), dim3(kTile), lds, s,
-                           d_samples, d_edge_src, d_edge_dst, d_topts_edge, n_edges, d_wp_offsets,
-                           waypoints_count, d_obstacles, n_obs, (float *)nullptr,
-                           d_is_free_edges, d_retests);
-    }
-    PUMP_LAUNCHED();
-    return PUMP_OK;
+        PUMP_LAUNCHED();
+        return PUMP_OK;
+    };
+    constexpr int EPB = kEdges32PerBlock;
+    if (d_disc_motions)
+        return slab ? launch(&k_edges32<true, EPB, true>) : launch(&k_edges32<true, EPB, false>);
+    return slab ? launch(&k_edges32<false, EPB, true>) : launch(&k_edges32<false, EPB, false>);
 }
 
 namespace {
