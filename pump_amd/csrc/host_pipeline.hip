@@ -36,26 +36,26 @@ int rm_upload(pump_roadmap *rm, const float *samples_h, const float *obstacles_h
 {
     const int num = rm->num;
     hipStream_t s = rm->stream;
-    TRY(dalloc(&rm->samples, (size_t)num * 6));
-    TRY(dalloc(&rm->obstacles, (size_t)rm->n_obs * 12));
+    TRY(dalloc(rm->mem, &rm->samples, (size_t)num * 6));
+    TRY(dalloc(rm->mem, &rm->obstacles, (size_t)rm->n_obs * 12));
     TRYH(hipMemcpyAsync(rm->samples, samples_h, sizeof(float) * num * 6, hipMemcpyHostToDevice, s));
     if (rm->n_obs)
         TRYH(hipMemcpyAsync(rm->obstacles, obstacles_h, sizeof(float) * rm->n_obs * 12,
                             hipMemcpyHostToDevice, s));
     if (rm->owns_noise && offsets_time_h && xcomb_h && rm->n_mc > 0) {
         size_t nt = (size_t)rm->tmax_steps * rm->n_mc * 3;
-        TRY(dalloc(&rm->offsets_time, nt));
-        TRY(dalloc(&rm->xcomb, nt));
+        TRY(dalloc(rm->mem, &rm->offsets_time, nt));
+        TRY(dalloc(rm->mem, &rm->xcomb, nt));
         TRYH(hipMemcpyAsync(rm->offsets_time, offsets_time_h, sizeof(float) * nt,
                             hipMemcpyHostToDevice, s));
         TRYH(hipMemcpyAsync(rm->xcomb, xcomb_h, sizeof(float) * nt, hipMemcpyHostToDevice, s));
-        TRY(dalloc(&rm->offsets_split,
+        TRY(dalloc(rm->mem, &rm->offsets_split,
                    pump_split_offsets_bytes(rm->tmax_steps, rm->n_mc) / sizeof(uint16_t)));
         TRY(pump_split_offsets(rm->offsets_time, rm->tmax_steps, rm->n_mc, rm->offsets_split, s));
     }
     rm->n_pairs = (int64_t)num * (num - 1);
-    TRY(dalloc(&rm->copts, (size_t)rm->n_pairs));
-    TRY(dalloc(&rm->topts, (size_t)rm->n_pairs));
+    TRY(dalloc(rm->mem, &rm->copts, (size_t)rm->n_pairs));
+    TRY(dalloc(rm->mem, &rm->topts, (size_t)rm->n_pairs));
     return PUMP_OK;
 }
 
@@ -79,7 +79,7 @@ int rm_tables(pump_roadmap *rm)
     hipStream_t s = rm->stream;
     EventTimer tm(s);
     if (P.polish) {
-        TRY(dalloc(&rm->topts64, (size_t)rm->n_pairs));
+        TRY(dalloc(rm->mem, &rm->topts64, (size_t)rm->n_pairs));
         TRY(pump_polish_topts(rm->samples, num, P.tmax, rm->topts, rm->topts64, s));
     }
 
@@ -87,52 +87,53 @@ int rm_tables(pump_roadmap *rm)
     rm->rn_idx = pump_rn_index(num, P.rn_perc);
     if (rm->rn_idx < 0 || rm->rn_idx >= rm->n_pairs)
         return PUMP_E_RANGE;
-    TRY(ensure_ws(rm, std::max(pump_select_rn_workspace(rm->n_pairs), pump_scan_workspace(num + 1))));
+    TRY(ensure_ws(rm,
+                  std::max(pump_select_rn_workspace(rm->n_pairs), pump_scan_workspace(num + 1))));
     tm.start();
     TRY(pump_select_rn(rm->copts, rm->n_pairs, rm->rn_idx, &rm->rn, rm->ws, rm->ws_bytes, s));
     rm->info.ms_select = tm.stop();
 
     // edges (mainPUMP.cu:313-348)
-    TRY(dalloc(&rm->row_start, (size_t)num + 1));
+    TRY(dalloc(rm->mem, &rm->row_start, (size_t)num + 1));
     tm.start();
     TRY(pump_count_edges(rm->copts, num, rm->rn, rm->row_start, &rm->n_edges, rm->ws, rm->ws_bytes,
                          s));
     const size_t E = (size_t)rm->n_edges;
-    TRY(dalloc(&rm->edge_src, E));
-    TRY(dalloc(&rm->edge_dst, E));
-    TRY(dalloc(&rm->copts_edge, E));
-    TRY(dalloc(&rm->topts_edge, E));
+    TRY(dalloc(rm->mem, &rm->edge_src, E));
+    TRY(dalloc(rm->mem, &rm->edge_dst, E));
+    TRY(dalloc(rm->mem, &rm->copts_edge, E));
+    TRY(dalloc(rm->mem, &rm->topts_edge, E));
     TRY(pump_fill_edges(rm->copts, rm->topts, num, rm->rn, rm->row_start, rm->edge_src,
                         rm->edge_dst, rm->copts_edge, rm->topts_edge, s));
     rm->info.ms_edges_build = tm.stop();
 
     // maxNNSize and heuristic (mainPUMP.cu:350-369)
     tm.start();
-    TRY(dalloc(&rm->in_degree, (size_t)num));
+    TRY(dalloc(rm->mem, &rm->in_degree, (size_t)num));
     TRY(pump_max_nn_size(rm->row_start, rm->edge_dst, rm->n_edges, num, rm->in_degree, &rm->max_nn,
                          s));
-    TRY(dalloc(&rm->h, (size_t)num));
+    TRY(dalloc(rm->mem, &rm->h, (size_t)num));
     TRY(pump_heuristic(rm->samples, num, rm->goal, P.tmax, rm->h, s));
     rm->info.ms_nn = tm.stop();
     if (!P.keep_pairs) {
         TRYH(hipStreamSynchronize(s));
-        dfree(rm->copts);
-        dfree(rm->topts);
+        dfree(rm->mem, rm->copts);
+        dfree(rm->mem, rm->topts);
     }
 
     // sampleFree (mainPUMP.cu:429-439)
-    TRY(dalloc(&rm->is_free_samples, (size_t)num));
+    TRY(dalloc(rm->mem, &rm->is_free_samples, (size_t)num));
     tm.start();
     TRY(pump_sample_free(rm->obstacles, rm->n_obs, rm->samples, num, rm->is_free_samples, s));
     rm->info.ms_sample_free = tm.stop();
 
     // waypoint offsets (mainPUMP.cu:441-463)
-    TRY(dalloc(&rm->wp_offsets, E + 1));
+    TRY(dalloc(rm->mem, &rm->wp_offsets, E + 1));
     TRY(ensure_ws(rm, pump_scan_workspace((int64_t)E + 1)));
     TRY(pump_waypoint_offsets(rm->topts_edge, rm->n_edges, P.w_fixed, P.wp_dt, P.w_cap,
                               rm->wp_offsets, &rm->n_wp, rm->ws, rm->ws_bytes, s));
-    TRY(dalloc(&rm->disc, (size_t)rm->n_wp * 6));
-    TRY(dalloc(&rm->is_free_edges, E));
+    TRY(dalloc(rm->mem, &rm->disc, (size_t)rm->n_wp * 6));
+    TRY(dalloc(rm->mem, &rm->is_free_edges, E));
     return PUMP_OK;
 }
 
@@ -164,10 +165,10 @@ int rm_alloc_halfspaces(pump_roadmap *rm)
     rm->max_hs = rm->n_obs > P.max_hs ? P.max_hs : rm->n_obs;
     rm->maxd2 = pump_maxd2(P.offset_mult);
     const size_t hs = (size_t)rm->n_wp * (size_t)(rm->max_hs > 0 ? rm->max_hs : 1);
-    TRY(dalloc(&rm->as, hs * 3));
-    TRY(dalloc(&rm->bs, hs));
-    TRY(dalloc(&rm->count, (size_t)rm->n_wp));
-    TRY(dalloc(&rm->edge_hs_mask, (size_t)rm->n_edges));
+    TRY(dalloc(rm->mem, &rm->as, hs * 3));
+    TRY(dalloc(rm->mem, &rm->bs, hs));
+    TRY(dalloc(rm->mem, &rm->count, (size_t)rm->n_wp));
+    TRY(dalloc(rm->mem, &rm->edge_hs_mask, (size_t)rm->n_edges));
     if (rm->max_hs == 0)
         TRY(pump_setup_as_bs((int64_t)hs, rm->bs, rm->as, rm->stream));
     return PUMP_OK;
@@ -331,9 +332,10 @@ extern "C" int pump_roadmap_build(const float *samples_h, int num, const float *
 
 namespace {
 
-template <typename T> int upload_n(T **dst, const T *src, size_t n, hipStream_t s)
+template <typename T>
+int upload_n(pump_roadmap *rm, T **dst, const T *src, size_t n, hipStream_t s)
 {
-    TRY(dalloc(dst, n));
+    TRY(dalloc(rm->mem, dst, n));
     if (n)
         TRYH(hipMemcpyAsync(*dst, src, sizeof(T) * n, hipMemcpyHostToDevice, s));
     return PUMP_OK;
@@ -381,28 +383,28 @@ int from_tables(pump_roadmap *rm, const pump_roadmap_tables &t, const float *off
             }
         }
     TRY(rm_upload(rm, t.samples, t.obstacles, offsets_time_h, xcomb_h));
-    dfree(rm->copts); // no pair tables: the roadmap starts from its edges
-    dfree(rm->topts);
+    dfree(rm->mem, rm->copts); // no pair tables: the roadmap starts from its edges
+    dfree(rm->mem, rm->topts);
     rm->n_pairs = 0;
     rm->rn = t.rn;
     rm->n_edges = t.n_edges;
     rm->n_wp = n_wp;
     rm->max_hs = mh;
     rm->maxd2 = pump_maxd2(rm->prm.offset_mult);
-    TRY(upload_n(&rm->row_start, t.row_start, (size_t)num + 1, s));
-    TRY(upload_n(&rm->edge_src, (const int *)src.data(), E, s));
-    TRY(upload_n(&rm->edge_dst, t.edge_dst, E, s));
-    TRY(upload_n(&rm->copts_edge, t.copts_edge, E, s));
-    TRY(upload_n(&rm->topts_edge, t.topts_edge, E, s));
-    TRY(upload_n(&rm->h, t.h, (size_t)num, s));
-    TRY(upload_n(&rm->is_free_edges, t.is_free_edges, E, s));
-    TRY(upload_n(&rm->is_free_samples, t.is_free_samples, (size_t)num, s));
-    TRY(upload_n(&rm->wp_offsets, t.wp_offsets, E + 1, s));
-    TRY(upload_n(&rm->as, t.as, (size_t)n_wp * mh * 3, s));
-    TRY(upload_n(&rm->bs, t.bs, (size_t)n_wp * mh, s));
-    TRY(upload_n(&rm->count, (const int *)count.data(), (size_t)n_wp, s));
-    TRY(upload_n(&rm->edge_hs_mask, (const uint64_t *)mask.data(), E, s));
-    TRY(dalloc(&rm->in_degree, (size_t)num));
+    TRY(upload_n(rm, &rm->row_start, t.row_start, (size_t)num + 1, s));
+    TRY(upload_n(rm, &rm->edge_src, (const int *)src.data(), E, s));
+    TRY(upload_n(rm, &rm->edge_dst, t.edge_dst, E, s));
+    TRY(upload_n(rm, &rm->copts_edge, t.copts_edge, E, s));
+    TRY(upload_n(rm, &rm->topts_edge, t.topts_edge, E, s));
+    TRY(upload_n(rm, &rm->h, t.h, (size_t)num, s));
+    TRY(upload_n(rm, &rm->is_free_edges, t.is_free_edges, E, s));
+    TRY(upload_n(rm, &rm->is_free_samples, t.is_free_samples, (size_t)num, s));
+    TRY(upload_n(rm, &rm->wp_offsets, t.wp_offsets, E + 1, s));
+    TRY(upload_n(rm, &rm->as, t.as, (size_t)n_wp * mh * 3, s));
+    TRY(upload_n(rm, &rm->bs, t.bs, (size_t)n_wp * mh, s));
+    TRY(upload_n(rm, &rm->count, (const int *)count.data(), (size_t)n_wp, s));
+    TRY(upload_n(rm, &rm->edge_hs_mask, (const uint64_t *)mask.data(), E, s));
+    TRY(dalloc(rm->mem, &rm->in_degree, (size_t)num));
     TRY(pump_max_nn_size(rm->row_start, rm->edge_dst, rm->n_edges, num, rm->in_degree, &rm->max_nn,
                          s));
     return rm_finish(rm, t_begin);
@@ -461,32 +463,32 @@ void pump::rmb::rm_release(pump_roadmap *rm)
         return;
     if (rm->stream)
         hipStreamSynchronize(rm->stream);
-    dfree(rm->samples);
-    dfree(rm->obstacles);
-    dfree(rm->copts);
-    dfree(rm->topts);
-    dfree(rm->topts64);
-    dfree(rm->row_start);
-    dfree(rm->edge_src);
-    dfree(rm->edge_dst);
-    dfree(rm->copts_edge);
-    dfree(rm->topts_edge);
-    dfree(rm->in_degree);
-    dfree(rm->h);
-    dfree(rm->wp_offsets);
-    dfree(rm->disc);
-    dfree(rm->is_free_edges);
-    dfree(rm->is_free_samples);
-    dfree(rm->as);
-    dfree(rm->bs);
-    dfree(rm->count);
-    dfree(rm->edge_hs_mask);
+    dfree(rm->mem, rm->samples);
+    dfree(rm->mem, rm->obstacles);
+    dfree(rm->mem, rm->copts);
+    dfree(rm->mem, rm->topts);
+    dfree(rm->mem, rm->topts64);
+    dfree(rm->mem, rm->row_start);
+    dfree(rm->mem, rm->edge_src);
+    dfree(rm->mem, rm->edge_dst);
+    dfree(rm->mem, rm->copts_edge);
+    dfree(rm->mem, rm->topts_edge);
+    dfree(rm->mem, rm->in_degree);
+    dfree(rm->mem, rm->h);
+    dfree(rm->mem, rm->wp_offsets);
+    dfree(rm->mem, rm->disc);
+    dfree(rm->mem, rm->is_free_edges);
+    dfree(rm->mem, rm->is_free_samples);
+    dfree(rm->mem, rm->as);
+    dfree(rm->mem, rm->bs);
+    dfree(rm->mem, rm->count);
+    dfree(rm->mem, rm->edge_hs_mask);
     if (rm->owns_noise) {
-        dfree(rm->offsets_time);
-        dfree(rm->offsets_split);
-        dfree(rm->xcomb);
+        dfree(rm->mem, rm->offsets_time);
+        dfree(rm->mem, rm->offsets_split);
+        dfree(rm->mem, rm->xcomb);
     }
-    dfree(rm->ws);
+    dfree(rm->mem, rm->ws);
     delete rm->search_ws;
     rm->search_ws = nullptr;
     if (rm->stream && rm->owns_stream)

@@ -4,6 +4,7 @@
 #pragma once
 
 #include <chrono>
+#include <cstddef>
 #include <new>
 #include <vector>
 
@@ -13,7 +14,88 @@
 namespace pump {
 namespace rmb {
 struct SearchWs;
-}
+
+// The device memory of one roadmap: ranges cut from blocks of 8, 32 and then
+// 64 MiB, given back with the roadmap; a request past kWhole is an allocation
+// of its own and goes back when it is released.  A range is handed out once,
+// so that a buffer that grows leaves its old range to the kernels still
+// queued on it without a wait.  hipMalloc and hipFree of a buffer of 4 MiB
+// take 78 and 204 us (of 32 MiB 192 and 250): the 60 buffers of a planned
+// problem of 1000 samples took 9 of its 14 ms.  Used by one thread at a time,
+// as the roadmap is.
+class DevArena {
+public:
+    DevArena() = default;
+    DevArena(const DevArena &) = delete;
+    DevArena &operator=(const DevArena &) = delete;
+    ~DevArena()
+    {
+        for (const Block &b : blocks)
+            hipFree(b.p);
+    }
+
+    // nullptr when the device (or the host) is out of memory
+    void *alloc(size_t bytes)
+    {
+        bytes = (bytes + kAlign - 1) / kAlign * kAlign;
+        if (bytes > kWhole)
+            return add(bytes, true);
+        for (Block &b : blocks)
+            if (!b.whole && b.bytes - b.used >= bytes)
+                return take(b, bytes);
+        if (add(next, false)) {
+            next = next * 4 < kLargest ? next * 4 : kLargest;
+            return take(blocks.back(), bytes);
+        }
+        return add(bytes, true); // no room for another block
+    }
+
+    void release(void *p)
+    {
+        for (size_t i = 0; i < blocks.size(); ++i)
+            if (blocks[i].whole && blocks[i].p == p) {
+                hipFree(p);
+                blocks.erase(blocks.begin() + (std::ptrdiff_t)i);
+                return;
+            }
+    }
+
+private:
+    struct Block {
+        char *p;
+        size_t bytes, used;
+        bool whole;
+    };
+    static constexpr size_t kAlign = 256, kWhole = (size_t)16 << 20, kLargest = (size_t)64 << 20;
+    std::vector<Block> blocks;
+    size_t next = (size_t)8 << 20;
+
+    static void *take(Block &b, size_t bytes)
+    {
+        void *p = b.p + b.used;
+        b.used += bytes;
+        return p;
+    }
+
+    void *add(size_t bytes, bool whole)
+    {
+        void *p = nullptr;
+        if (hipMalloc(&p, bytes) != hipSuccess) {
+            // the failed attempt leaves its error as the thread's last error:
+            // clear it, so that a later launch check does not report it
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        try {
+            blocks.push_back(Block{static_cast<char *>(p), bytes, 0, whole});
+        } catch (const std::bad_alloc &) {
+            hipFree(p);
+            return nullptr;
+        }
+        return p;
+    }
+};
+} // namespace rmb
 } // namespace pump
 
 struct pump_roadmap {
@@ -49,6 +131,7 @@ struct pump_roadmap {
     size_t ws_bytes = 0;
     // device buffers of the search, kept between searches (allocated on first use)
     pump::rmb::SearchWs *search_ws = nullptr;
+    pump::rmb::DevArena mem; // every device buffer of the roadmap and its searches
     pump_roadmap_info info{};
     // a roadmap of a batch borrows the batch's stream and noise tables
     bool owns_stream = true, owns_noise = true;
@@ -78,23 +161,36 @@ template <typename T> inline void dfree(T *&p)
     p = nullptr;
 }
 
+template <typename T> inline int dalloc(DevArena &m, T **p, size_t n)
+{
+    *p = static_cast<T *>(m.alloc(sizeof(T) * (n ? n : 1)));
+    return *p ? PUMP_OK : PUMP_E_NOMEM;
+}
+
+template <typename T> inline void dfree(DevArena &m, T *&p)
+{
+    if (p)
+        m.release((void *)p);
+    p = nullptr;
+}
+
 inline int ensure_ws(pump_roadmap *rm, size_t bytes)
 {
     if (rm->ws_bytes >= bytes)
         return PUMP_OK;
-    dfree(rm->ws);
+    dfree(rm->mem, rm->ws);
     char *w = nullptr;
-    int r = dalloc(&w, bytes);
+    int r = dalloc(rm->mem, &w, bytes);
     rm->ws = w;
     rm->ws_bytes = r == PUMP_OK ? bytes : 0;
     return r;
 }
 
-// A device buffer that grows on demand: to twice the request, and to at least
-// 4 MiB, so that a search whose wavefront grows from a few paths to hundreds
-// of thousands reallocates each buffer a few times, not dozens (each hipFree
-// also waits for the device).
+// A device buffer of a roadmap that grows on demand, to twice the request and
+// to at least 64 KiB, so that a search whose wavefront grows from a few paths
+// to hundreds of thousands takes new memory a few times, not dozens.
 struct DevBuf {
+    DevArena *mem = nullptr;
     void *p = nullptr;
     size_t bytes = 0;
     int ensure(size_t b)
@@ -102,35 +198,24 @@ struct DevBuf {
         if (b <= bytes)
             return PUMP_OK;
         if (p)
-            hipFree(p);
-        p = nullptr;
+            mem->release(p);
         bytes = 0;
-        size_t want = b * 2 > ((size_t)4 << 20) ? b * 2 : ((size_t)4 << 20);
-        if (hipMalloc(&p, want) != hipSuccess) {
-            // the failed attempt leaves its error as the thread's last error:
-            // clear it, so that a later launch check does not report it
-            (void)hipGetLastError();
-            if (hipMalloc(&p, b) != hipSuccess) {
-                (void)hipGetLastError();
-                p = nullptr;
-                return PUMP_E_NOMEM;
-            }
+        size_t want = b * 2 > ((size_t)64 << 10) ? b * 2 : ((size_t)64 << 10);
+        p = mem->alloc(want);
+        if (!p) {
             want = b;
+            p = mem->alloc(want);
         }
+        if (!p)
+            return PUMP_E_NOMEM;
         bytes = want;
         return PUMP_OK;
-    }
-    ~DevBuf()
-    {
-        if (p)
-            hipFree(p);
     }
 };
 
 // The search's device buffers. The roadmap keeps them from one search to the
 // next: a repeated query on the same roadmap then makes no hipMalloc/hipFree
-// once the buffers have grown to its sizes (each hipFree of a grown buffer
-// also waits for the device). Every search initialises what it reads, so
+// once the buffers have grown to its sizes. Every search initialises what it reads, so
 // the contents a previous search left behind are never used. The host- and
 // device-bookkeeping searches share the buffers whose meaning is the same;
 // searches on one roadmap run one at a time (its one stream).
@@ -146,13 +231,23 @@ struct SearchWs {
     DevBuf sel_paths, sel_T, sel_hits;
     // rows of the path table (prev, node, cost, time, cpv) the last search stored
     int64_t last_num_paths = 0;
+
+    explicit SearchWs(DevArena *m)
+    {
+        for (DevBuf *b :
+             {&voff, &vedge, &scan, &prev, &node, &cost, &time, &cpv, &next, &head, &open, &valid,
+              &flags, &steps, &clamp, &cnt, &wf_prev, &wf_edge, &wf_next, &stage, &cp, &new_time,
+              &new_cost, &keep, &node_cnt, &node_cur, &grp, &surv, &src_rows, &bkt, &bflag, &prop,
+              &row_src, &sel_paths, &sel_T, &sel_hits})
+            b->mem = m;
+    }
 };
 
 // the roadmap's search buffers, created on first use (nullptr when out of host memory)
 inline SearchWs *search_ws(pump_roadmap *rm)
 {
     if (!rm->search_ws)
-        rm->search_ws = new (std::nothrow) SearchWs();
+        rm->search_ws = new (std::nothrow) SearchWs(&rm->mem);
     return rm->search_ws;
 }
 
