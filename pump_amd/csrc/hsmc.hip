@@ -674,24 +674,6 @@ __global__ __launch_bounds__(kBlock) void k_classify(
 // that pass.
 constexpr int kCopyRows = 4;
 
-template <int kUnit>
-struct CopyWord;
-template <>
-struct CopyWord<16> {
-    using T = uint4;
-};
-template <>
-struct CopyWord<8> {
-    using T = uint64_t;
-};
-template <>
-struct CopyWord<4> {
-    using T = uint32_t;
-};
-template <>
-struct CopyWord<1> {
-    using T = uint8_t;
-};
 
 // byte rows: normalise to 0/1 and count zeros; bit rows: count ones
 template <bool kBits>
@@ -1113,41 +1095,6 @@ __global__ __launch_bounds__(256) void k_propagate_b64(
                                   dst_base, n_p, path_cp, cp_base, clamped);
         }
     }
-}
-
-// Copy-on-write form: the listed paths' child rows start as their parents'
-// rows (the half-space pass ANDs into them).  One wave per listed path.
-template <int kUnit>
-__device__ __forceinline__ void copy_listed_body(const HsPath *__restrict__ recs,
-                                                 const int *__restrict__ ctl,
-                                                 const uint8_t *__restrict__ src,
-                                                 uint8_t *__restrict__ dst, int64_t dst_base,
-                                                 int64_t row_bytes, const VGrid &G)
-{
-    using T = typename CopyWord<kUnit>::T;
-    if (ctl[kCtlOverflow]) // the group form writes whole rows itself
-        return;
-    const int lane = threadIdx.x & 63;
-    const int n = ctl[kCtlListed];
-    const int units = (int)(row_bytes / kUnit);
-    const int64_t n_waves = wave_count(G);
-    for (int64_t slot = wave_index(G); slot < n; slot += n_waves) {
-        const HsPath r = recs[slot];
-        const T *sp = reinterpret_cast<const T *>(src + (int64_t)r.prev * row_bytes);
-        T *dp = reinterpret_cast<T *>(dst + (dst_base + r.w) * row_bytes);
-        for (int j = lane; j < units; j += 64)
-            dp[j] = sp[j];
-    }
-}
-
-template <int kUnit>
-__global__ __launch_bounds__(256) void k_copy_listed(const HsPath *__restrict__ recs,
-                                                     const int *__restrict__ ctl,
-                                                     const uint8_t *__restrict__ src,
-                                                     uint8_t *__restrict__ dst, int64_t dst_base,
-                                                     int64_t row_bytes)
-{
-    copy_listed_body<kUnit>(recs, ctl, src, dst, dst_base, row_bytes, hw_grid());
 }
 
 // The classification, row copies and workspace clearing of many problems'
@@ -1681,18 +1628,10 @@ static int launch_propagate(int n_new, int W_fixed, const int64_t *wp_offsets, c
         if (row_src) {
             // copy-on-write: only the listed paths' rows are written
             const uintptr_t al = ((uintptr_t)src | (uintptr_t)dst);
-            const unsigned g = wave_blocks_for(n_new);
-            if (row_bytes % 16 == 0 && (al & 15) == 0)
-                hipLaunchKernelGGL(k_copy_listed<16>, dim3(g), dim3(256), 0, s, recs, ctl,
-                                   (const uint8_t *)src, (uint8_t *)dst, dst_base, row_bytes);
-            else if (row_bytes % 8 == 0 && (al & 7) == 0)
-                hipLaunchKernelGGL(k_copy_listed<8>, dim3(g), dim3(256), 0, s, recs, ctl,
-                                   (const uint8_t *)src, (uint8_t *)dst, dst_base, row_bytes);
-            else
-                hipLaunchKernelGGL(k_copy_listed<1>, dim3(g), dim3(256), 0, s, recs, ctl,
-                                   (const uint8_t *)src, (uint8_t *)dst, dst_base, row_bytes);
-            PUMP_LAUNCHED();
-            return bins_finish(B, kBits, s);
+            const int unit = row_bytes % 16 == 0 && (al & 15) == 0 ? 16
+                             : row_bytes % 8 == 0 && (al & 7) == 0 ? 8
+                                                                   : 1;
+            return bins_finish(B, kBits, s, unit, row_bytes);
         }
         // copy unit and segment width
         const uintptr_t al = ((uintptr_t)src | (uintptr_t)dst);

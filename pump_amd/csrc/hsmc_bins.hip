@@ -89,17 +89,25 @@ __device__ __forceinline__ int time_total(const int *__restrict__ hist, int t, i
 
 // One workgroup: time-index starts, chunks, entry/chunk totals, overflow.
 // The pairs of time index t occupy [tstart[t], tstart[t+1]), sub-bin by
-// sub-bin (sub-bin k: paths with w % kSubBins == k).
+// sub-bin (sub-bin k: paths with w % kSubBins == k).  The chunks are written
+// lane = chunk, each finding its time index in the starts kept in LDS (tables
+// of up to kScanTimes; a thread per time index wrote its chunks one after
+// another before, in stores that met no other lane's: 13 us, now 9, with 3003
+// chunks).
+constexpr int kScanTimes = 4096;
+
 __device__ __forceinline__ void bin_scan_body(int T, const int *__restrict__ hist,
                                               int *__restrict__ tstart,
                                               BinChunk *__restrict__ chunks, int *__restrict__ ctl,
                                               int64_t entry_cap, int64_t chunk_cap)
 {
     __shared__ int tot_e, tot_c;
+    __shared__ int first_e[kScanTimes + 1], first_c[kScanTimes + 1];
     constexpr int kKeep = 4; // time indices per thread whose totals stay in registers
     const int per = (T + kScanBlock - 1) / kScanBlock;
     const int t0 = threadIdx.x * per;
     const int t1 = (t0 + per) < T ? (t0 + per) : T;
+    const bool in_lds = T <= kScanTimes;
     int se = 0, sc = 0, unused;
     int keep[kKeep];
 #pragma unroll
@@ -117,22 +125,40 @@ __device__ __forceinline__ void bin_scan_body(int T, const int *__restrict__ his
         const int j = t - t0;
         const int h = j < kKeep ? keep[j] : time_total(hist, t, 0, &unused);
         tstart[t] = se;
-        if (!overflow)
-            for (int j = 0; j * kBinChunk < h; ++j) {
-                BinChunk c;
-                c.ti = t;
-                c.begin = se + j * kBinChunk;
-                c.end = se + ((j + 1) * kBinChunk < h ? (j + 1) * kBinChunk : h);
-                chunks[sc + j] = c;
-            }
+        if (in_lds) {
+            first_e[t] = se;
+            first_c[t] = sc;
+        } else if (!overflow) {
+            for (int q = 0; q * kBinChunk < h; ++q)
+                chunks[sc + q] = BinChunk{t, se + q * kBinChunk, se + min((q + 1) * kBinChunk, h)};
+        }
         se += h;
         sc += (h + kBinChunk - 1) / kBinChunk;
     }
     if (threadIdx.x == 0) {
         tstart[T] = tot_e;
+        if (in_lds) {
+            first_e[T] = tot_e;
+            first_c[T] = tot_c;
+        }
         ctl[kCtlEntries] = tot_e;
         ctl[kCtlChunks] = tot_c;
         ctl[kCtlOverflow] = overflow ? 1 : 0;
+    }
+    if (!in_lds || overflow)
+        return;
+    __syncthreads();
+    for (int c = threadIdx.x; c < tot_c; c += kScanBlock) {
+        int lo = 0, hi = T; // first_c[lo] <= c < first_c[hi]
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (first_c[mid] <= c)
+                lo = mid;
+            else
+                hi = mid;
+        }
+        const int begin = first_e[lo] + (c - first_c[lo]) * kBinChunk;
+        chunks[c] = BinChunk{lo, begin, min(begin + kBinChunk, first_e[lo + 1])};
     }
 }
 
@@ -195,6 +221,23 @@ __global__ __launch_bounds__(256) void k_bin_emit(const HsPath *__restrict__ rec
                   hw_grid());
 }
 
+// The same with the row copies of the copy-on-write step (kUnit bytes at a
+// time), which need nothing of it: workgroups from emit_blocks on copy.  Two
+// launches took 13 + 8 us one after the other, the one 17.
+template <int kUnit>
+__global__ __launch_bounds__(256) void k_bin_emit_copy(const BinArgs a, int emit_blocks,
+                                                       int64_t row_bytes)
+{
+    if ((int)blockIdx.x < emit_blocks)
+        bin_emit_body(a.recs, a.ctl, a.bs, a.max_hs, a.dt, a.tmax_steps, a.hist, a.tstart,
+                      a.cursor, a.entries, VGrid{(int64_t)blockIdx.x, (int64_t)emit_blocks});
+    else
+        copy_listed_body<kUnit>(a.recs, a.ctl, (const uint8_t *)a.valid_src,
+                                (uint8_t *)a.valid_dst, a.dst_base, row_bytes,
+                                VGrid{(int64_t)blockIdx.x - emit_blocks,
+                                      (int64_t)gridDim.x - emit_blocks});
+}
+
 constexpr float kTiny = 1e-30f;
 __device__ __forceinline__ float at_least_tiny(float v) { return v < kTiny ? kTiny : v; }
 
@@ -212,8 +255,8 @@ __device__ __forceinline__ float at_least_tiny(float v) { return v < kTiny ? kTi
 // test, and the instructions that bring each half-space to it; per-lane
 // outcomes, eight live bits probed per pair and atomics issued lane by lane
 // doubled them.  Copy-on-write step of 1e6 paths, 47,705 pairs, 2000
-// particles: the pass 60 -> 38 us, the step 126 -> 109 us; 4e5 paths of 8192
-// particles at 512 per wave: 243 -> 163 us.
+// particles: the pass 60 -> 38 us; 4e5 paths of 8192 particles at 512 per
+// wave: the step 243 -> 163 us.
 template <bool kBits, int NQ>
 __device__ __forceinline__ void bin_test(const BinArgs &a, int64_t n_chunks, const VGrid &G)
 {
@@ -268,18 +311,25 @@ __device__ __forceinline__ void bin_test(const BinArgs &a, int64_t n_chunks, con
                 if (lane < ne && h0 + h < max_hs)
                     b[h] = a.bs[my_wp * max_hs + h0 + h];
             }
+            // the first slot's normals, which nearly all pairs hold, beside the
+            // offsets, those of the other slots together after them
+            float av[kSlotTile][3];
+#pragma unroll
+            for (int h = 0; h < kSlotTile; ++h) {
+                av[h][0] = av[h][1] = av[h][2] = 0.0f;
+                if (h == 0 ? lane < ne : !(b[h] >= 1000.0f)) {
+                    const int64_t k = my_wp * max_hs + h0 + h;
+                    av[h][0] = a.as[k * 3 + 0];
+                    av[h][1] = a.as[k * 3 + 1];
+                    av[h][2] = a.as[k * 3 + 2];
+                }
+            }
 #pragma unroll
             for (int h = 0; h < kSlotTile; ++h) {
                 const bool live = !(b[h] >= 1000.0f);
                 if (__ballot(live) == 0ull)
                     continue;
-                float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f;
-                if (live) {
-                    const int64_t k = my_wp * max_hs + h0 + h;
-                    a0 = a.as[k * 3 + 0];
-                    a1 = a.as[k * 3 + 1];
-                    a2 = a.as[k * 3 + 2];
-                }
+                const float a0 = av[h][0], a1 = av[h][1], a2 = av[h][2];
                 const float b2 = b[h] * b[h];
                 const bool out = b[h] > 0.0f && b2 > kTiny &&
                                  reach2 * at_least_tiny(a0 * a0 + a1 * a1 + a2 * a2) < b2;
@@ -851,12 +901,26 @@ int bins_scan(const BinArgs &a, hipStream_t s)
     return PUMP_OK;
 }
 
-int bins_finish(const BinArgs &a, bool bits, hipStream_t s)
+int bins_finish(const BinArgs &a, bool bits, hipStream_t s, int copy_unit, int64_t row_bytes)
 {
     // device-side counts; the grids are sized for their upper bounds
-    hipLaunchKernelGGL(k_bin_emit, dim3(grid_for(a.n_new, 256, 4096)), dim3(256), 0, s, a.recs,
-                       (const int *)a.ctl, a.bs, a.max_hs, a.dt, a.tmax_steps,
-                       (const int *)a.hist, (const int *)a.tstart, a.cursor, a.entries);
+    const unsigned g_em = grid_for(a.n_new, 256, 4096);
+    if (copy_unit == 0) {
+        hipLaunchKernelGGL(k_bin_emit, dim3(g_em), dim3(256), 0, s, a.recs, (const int *)a.ctl,
+                           a.bs, a.max_hs, a.dt, a.tmax_steps, (const int *)a.hist,
+                           (const int *)a.tstart, a.cursor, a.entries);
+    } else {
+        const auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(g_em + wave_blocks(a.n_new)), dim3(256), 0, s, a,
+                               (int)g_em, row_bytes);
+        };
+        if (copy_unit == 16)
+            launch(k_bin_emit_copy<16>);
+        else if (copy_unit == 8)
+            launch(k_bin_emit_copy<8>);
+        else
+            launch(k_bin_emit_copy<1>);
+    }
     PUMP_LAUNCHED();
     const int64_t groups = (a.n_p + 63) / 64;
     const int nq = (a.nq == 1 || a.nq == 2 || a.nq == 8) ? a.nq : kTestGroups;

@@ -367,6 +367,51 @@ enum : int {
     kCtlChunks = 3,   // binned chunks
 };
 
+// the word of a row copy of kUnit bytes at a time
+template <int kUnit>
+struct CopyWord;
+template <>
+struct CopyWord<16> {
+    using T = uint4;
+};
+template <>
+struct CopyWord<8> {
+    using T = uint64_t;
+};
+template <>
+struct CopyWord<4> {
+    using T = uint32_t;
+};
+template <>
+struct CopyWord<1> {
+    using T = uint8_t;
+};
+
+// Copy-on-write form: the listed paths' child rows start as their parents'
+// rows (the half-space pass ANDs into them).  One wave per listed path.
+template <int kUnit>
+__device__ __forceinline__ void copy_listed_body(const HsPath *__restrict__ recs,
+                                                 const int *__restrict__ ctl,
+                                                 const uint8_t *__restrict__ src,
+                                                 uint8_t *__restrict__ dst, int64_t dst_base,
+                                                 int64_t row_bytes, const VGrid &G)
+{
+    using T = typename CopyWord<kUnit>::T;
+    if (ctl[kCtlOverflow]) // the group form writes whole rows itself
+        return;
+    const int lane = threadIdx.x & 63;
+    const int n = ctl[kCtlListed];
+    const int units = (int)(row_bytes / kUnit);
+    const int64_t n_waves = wave_count(G);
+    for (int64_t slot = wave_index(G); slot < n; slot += n_waves) {
+        const HsPath r = recs[slot];
+        const T *sp = reinterpret_cast<const T *>(src + (int64_t)r.prev * row_bytes);
+        T *dp = reinterpret_cast<T *>(dst + (dst_base + r.w) * row_bytes);
+        for (int j = lane; j < units; j += 64)
+            dp[j] = sp[j];
+    }
+}
+
 } // namespace wave
 
 // Listed-path half-space pass of the batched form (hsmc_bins.hip).
@@ -397,7 +442,10 @@ struct BinArgs {
     int nq;
 };
 int bins_scan(const BinArgs &a, hipStream_t s);
-int bins_finish(const BinArgs &a, bool bits, hipStream_t s);
+// copy_unit != 0: the listed rows are also copied from their parents', that
+// many bytes at a time
+int bins_finish(const BinArgs &a, bool bits, hipStream_t s, int copy_unit = 0,
+                int64_t row_bytes = 0);
 
 // The copy-on-write MC step (bit validity, FP32 tests) of many problems in
 // one launch per stage.  A problem's job holds everything its stages read;

@@ -166,3 +166,39 @@ def test_batched_tests_at_the_reach_of_the_particles(n_p, max_hs, scale):
         got = unpack_bits(rows.view(np.uint64), n_p) if bits else rows
         assert np.array_equal(got, ref_v[npar:]), bits
         assert np.array_equal(host(cp), ref_cp[npar:])
+
+
+@pytest.mark.parametrize("T", [1, 1025, 4096, 4097, 5200])
+def test_batched_chunks_of_many_times(T):
+    """The chunks of tables around the scan's LDS capacity of 4096 times, most
+    of the pairs in few times and the others spread over all of them."""
+    n_new, n_p, max_hs = 6000, 64, 3
+    d = random_hsmc_inputs(T, n_edges=300, max_hs=max_hs, n_p=n_p, n_mc=n_p, T=T, n_new=n_new,
+                           n_parent=40, variable=True, w_range=(2, 9))
+    d["dt"] = np.float32(4.0 / 5200)
+    d["wf_prev"][: n_new // 2] = 0
+    d["wf_edge"][: n_new // 2] = 5
+    ref_v, ref_cp, ref_cl = oracle_propagate(d)
+    npar = d["n_parent"]
+    g = {k: dev(d[k]) for k in ("off", "as_", "bs", "offs", "topts", "times", "wf_edge",
+                                 "wf_prev")}
+    g_mask = dev(edge_mask_host(d["off"], d["bs"], max_hs))
+    ws_bytes = P.lib.pump_propagate_workspace(n_new, T)
+    ws = P.DeviceArray(shape=(ws_bytes,), dtype=np.uint8)
+    src = dev(pack_bits(d["valid"][:npar], n_p))
+    dst = dev(np.zeros((n_new, 8), np.uint8))
+    cp, clamp = dev(np.zeros(n_new, np.float32)), dev(np.zeros(1, np.uint64))
+    row_src = dev(np.zeros(n_new, np.int32))
+    pcp = dev(1 - d["valid"][:npar].mean(1, dtype=np.float32))
+    print("times", T, flush=True)
+    P.check("cow", P.lib.pump_propagate_cp_cow(
+        1, n_new, 0, ptr(g["off"]), ptr(g["wf_edge"]), ptr(g["wf_prev"]), ptr(g["as_"]),
+        ptr(g["bs"]), g_mask.p, ptr(g["times"]), ptr(g["topts"]), d["dt"], max_hs, ptr(g["offs"]),
+        T, d["om"], d["n_mc"], ptr(src), ptr(pcp), ptr(dst), 0, ptr(row_src), n_p, ptr(cp), 0, 0,
+        None, None, ptr(clamp), ws.p, ws_bytes, None))
+    own = host(row_src) >= 0
+    assert own.mean() > 0.5 and int(host(clamp)[0]) == ref_cl
+    got = unpack_bits(host(dst).view(np.uint64), n_p)
+    assert np.array_equal(got[own], ref_v[npar:][own])
+    assert np.array_equal(ref_v[npar:][~own], d["valid"][d["wf_prev"][~own]])
+    assert np.array_equal(host(cp)[own], ref_cp[npar:][own])
