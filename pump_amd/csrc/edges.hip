@@ -10,7 +10,8 @@
 // the waypoints go to discMotions (consecutive lanes write consecutive
 // 24-byte records), and segment (k, k+1) is tested by the lane holding
 // waypoint k, with the far end taken from the next lane, against the boxes
-// that are not separated from its edge's bounding box.
+// that are not separated from its edge's bounding box, or, of many boxes,
+// those that a table of slabs gives for the segment's own bounds.
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>
