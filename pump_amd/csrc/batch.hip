@@ -159,7 +159,7 @@ int new_instance(pump_batch *b, const pump_batch_instance &I, int n_mc, int tmax
     rm->offsets_time = b->offsets_time;
     rm->xcomb = b->xcomb;
     rm->offsets_split = b->offsets_split;
-    return rm_upload(rm, I.samples, I.obstacles, nullptr, nullptr);
+    return rm_upload(rm, I.samples, I.obstacles, nullptr, nullptr, true);
 }
 
 // all ordered pairs of every instance: one persistent launch

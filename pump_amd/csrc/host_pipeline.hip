@@ -31,31 +31,68 @@ using namespace pump;
 namespace pump {
 namespace rmb {
 
-int rm_upload(pump_roadmap *rm, const float *samples_h, const float *obstacles_h,
-              const float *offsets_time_h, const float *xcomb_h)
+// Room for the arrays over E edges (ends, costs, times, waypoint offsets,
+// flags, half-space masks; scratch) and over n_wp waypoints (states,
+// half-spaces in hs slots, counts).
+static void reserve_edges(pump_roadmap *rm, size_t E, size_t scratch)
 {
-    const int num = rm->num;
+    rm->mem.reserve({E * sizeof(int), E * sizeof(int), E * sizeof(float), E * sizeof(float),
+                     (E + 1) * sizeof(int64_t), E, E * sizeof(uint64_t), scratch});
+}
+
+static void reserve_waypoints(pump_roadmap *rm, size_t n_wp, size_t hs, bool states)
+{
+    rm->mem.reserve({states ? n_wp * 6 * sizeof(float) : 0, n_wp * hs * 3 * sizeof(float),
+                     n_wp * hs * sizeof(float), n_wp * sizeof(int)});
+}
+
+int rm_upload(pump_roadmap *rm, const float *samples_h, const float *obstacles_h,
+              const float *offsets_time_h, const float *xcomb_h, bool pairs)
+{
+    const size_t num = (size_t)rm->num;
     hipStream_t s = rm->stream;
+    const bool noise = rm->owns_noise && offsets_time_h && xcomb_h && rm->n_mc > 0;
+    const size_t nt = noise ? (size_t)rm->tmax_steps * rm->n_mc * 3 : 0;
+    const size_t nsplit = noise ? pump_split_offsets_bytes(rm->tmax_steps, rm->n_mc) : 0;
+    const size_t np = pairs ? num * (num - 1) : 0;
+    const size_t table = np * sizeof(float), select = pump_select_rn_workspace((int64_t)np);
+    const bool keep = pairs && rm->prm.keep_pairs;
+    // with the tables over the samples (rm_tables)
+    rm->mem.reserve({num * 6 * sizeof(float), (size_t)rm->n_obs * 12 * sizeof(float),
+                     nt * sizeof(float), nt * sizeof(float), nsplit, keep ? table : 0,
+                     keep ? table : 0, keep ? select : 0, pump_scan_workspace(rm->num + 1), (num + 1) * sizeof(int64_t),
+                     num * sizeof(int), num * sizeof(float), num});
     TRY(dalloc(rm->mem, &rm->samples, (size_t)num * 6));
     TRY(dalloc(rm->mem, &rm->obstacles, (size_t)rm->n_obs * 12));
     TRYH(hipMemcpyAsync(rm->samples, samples_h, sizeof(float) * num * 6, hipMemcpyHostToDevice, s));
     if (rm->n_obs)
         TRYH(hipMemcpyAsync(rm->obstacles, obstacles_h, sizeof(float) * rm->n_obs * 12,
                             hipMemcpyHostToDevice, s));
-    if (rm->owns_noise && offsets_time_h && xcomb_h && rm->n_mc > 0) {
-        size_t nt = (size_t)rm->tmax_steps * rm->n_mc * 3;
+    if (noise) {
         TRY(dalloc(rm->mem, &rm->offsets_time, nt));
         TRY(dalloc(rm->mem, &rm->xcomb, nt));
         TRYH(hipMemcpyAsync(rm->offsets_time, offsets_time_h, sizeof(float) * nt,
                             hipMemcpyHostToDevice, s));
         TRYH(hipMemcpyAsync(rm->xcomb, xcomb_h, sizeof(float) * nt, hipMemcpyHostToDevice, s));
-        TRY(dalloc(rm->mem, &rm->offsets_split,
-                   pump_split_offsets_bytes(rm->tmax_steps, rm->n_mc) / sizeof(uint16_t)));
+        TRY(dalloc(rm->mem, &rm->offsets_split, nsplit / sizeof(uint16_t)));
         TRY(pump_split_offsets(rm->offsets_time, rm->tmax_steps, rm->n_mc, rm->offsets_split, s));
     }
-    rm->n_pairs = (int64_t)num * (num - 1);
-    TRY(dalloc(rm->mem, &rm->copts, (size_t)rm->n_pairs));
-    TRY(dalloc(rm->mem, &rm->topts, (size_t)rm->n_pairs));
+    rm->n_pairs = (int64_t)np;
+    if (keep) {
+        TRY(dalloc(rm->mem, &rm->copts, np));
+        TRY(dalloc(rm->mem, &rm->topts, np));
+        TRY(dalloc(rm->mem, &rm->select_ws, select));
+    } else if (pairs) {
+        // the tables and the selection's scratch in one allocation, which
+        // rm_tables gives back
+        const size_t each = DevArena::padded(table);
+        char *all = static_cast<char *>(rm->mem.alloc_whole(2 * each + select));
+        if (!all)
+            return PUMP_E_NOMEM;
+        rm->copts = reinterpret_cast<float *>(all);
+        rm->topts = reinterpret_cast<float *>(all + each);
+        rm->select_ws = all + 2 * each;
+    }
     return PUMP_OK;
 }
 
@@ -87,18 +124,22 @@ int rm_tables(pump_roadmap *rm)
     rm->rn_idx = pump_rn_index(num, P.rn_perc);
     if (rm->rn_idx < 0 || rm->rn_idx >= rm->n_pairs)
         return PUMP_E_RANGE;
-    TRY(ensure_ws(rm,
-                  std::max(pump_select_rn_workspace(rm->n_pairs), pump_scan_workspace(num + 1))));
+    TRY(ensure_ws(rm, pump_scan_workspace(num + 1)));
+    TRY(dalloc(rm->mem, &rm->row_start, (size_t)num + 1));
+    TRY(dalloc(rm->mem, &rm->in_degree, (size_t)num));
+    TRY(dalloc(rm->mem, &rm->h, (size_t)num));
+    TRY(dalloc(rm->mem, &rm->is_free_samples, (size_t)num));
     tm.start();
-    TRY(pump_select_rn(rm->copts, rm->n_pairs, rm->rn_idx, &rm->rn, rm->ws, rm->ws_bytes, s));
+    TRY(pump_select_rn(rm->copts, rm->n_pairs, rm->rn_idx, &rm->rn, rm->select_ws,
+                       pump_select_rn_workspace(rm->n_pairs), s));
     rm->info.ms_select = tm.stop();
 
     // edges (mainPUMP.cu:313-348)
-    TRY(dalloc(rm->mem, &rm->row_start, (size_t)num + 1));
     tm.start();
     TRY(pump_count_edges(rm->copts, num, rm->rn, rm->row_start, &rm->n_edges, rm->ws, rm->ws_bytes,
                          s));
     const size_t E = (size_t)rm->n_edges;
+    reserve_edges(rm, E, pump_scan_workspace((int64_t)E + 1));
     TRY(dalloc(rm->mem, &rm->edge_src, E));
     TRY(dalloc(rm->mem, &rm->edge_dst, E));
     TRY(dalloc(rm->mem, &rm->copts_edge, E));
@@ -109,20 +150,18 @@ int rm_tables(pump_roadmap *rm)
 
     // maxNNSize and heuristic (mainPUMP.cu:350-369)
     tm.start();
-    TRY(dalloc(rm->mem, &rm->in_degree, (size_t)num));
     TRY(pump_max_nn_size(rm->row_start, rm->edge_dst, rm->n_edges, num, rm->in_degree, &rm->max_nn,
                          s));
-    TRY(dalloc(rm->mem, &rm->h, (size_t)num));
     TRY(pump_heuristic(rm->samples, num, rm->goal, P.tmax, rm->h, s));
     rm->info.ms_nn = tm.stop();
     if (!P.keep_pairs) {
         TRYH(hipStreamSynchronize(s));
-        dfree(rm->mem, rm->copts);
-        dfree(rm->mem, rm->topts);
+        dfree(rm->mem, rm->copts); // with what lies behind it
+        rm->topts = nullptr;
+        rm->select_ws = nullptr;
     }
 
     // sampleFree (mainPUMP.cu:429-439)
-    TRY(dalloc(rm->mem, &rm->is_free_samples, (size_t)num));
     tm.start();
     TRY(pump_sample_free(rm->obstacles, rm->n_obs, rm->samples, num, rm->is_free_samples, s));
     rm->info.ms_sample_free = tm.stop();
@@ -132,6 +171,7 @@ int rm_tables(pump_roadmap *rm)
     TRY(ensure_ws(rm, pump_scan_workspace((int64_t)E + 1)));
     TRY(pump_waypoint_offsets(rm->topts_edge, rm->n_edges, P.w_fixed, P.wp_dt, P.w_cap,
                               rm->wp_offsets, &rm->n_wp, rm->ws, rm->ws_bytes, s));
+    reserve_waypoints(rm, (size_t)rm->n_wp, (size_t)std::max(1, std::min(rm->n_obs, P.max_hs)), true);
     TRY(dalloc(rm->mem, &rm->disc, (size_t)rm->n_wp * 6));
     TRY(dalloc(rm->mem, &rm->is_free_edges, E));
     return PUMP_OK;
@@ -227,7 +267,7 @@ int build(pump_roadmap *rm, const float *samples_h, const float *obstacles_h,
           const float *offsets_time_h, const float *xcomb_h)
 {
     const auto t_begin = std::chrono::steady_clock::now();
-    TRY(rm_upload(rm, samples_h, obstacles_h, offsets_time_h, xcomb_h));
+    TRY(rm_upload(rm, samples_h, obstacles_h, offsets_time_h, xcomb_h, true));
     TRY(rm_pairs(rm));
     TRY(rm_tables(rm));
     TRY(rm_edge_pass(rm));
@@ -382,29 +422,29 @@ int from_tables(pump_roadmap *rm, const pump_roadmap_tables &t, const float *off
                 mask[e] |= 1ull << (k < 63 ? k : 63);
             }
         }
-    TRY(rm_upload(rm, t.samples, t.obstacles, offsets_time_h, xcomb_h));
-    dfree(rm->mem, rm->copts); // no pair tables: the roadmap starts from its edges
-    dfree(rm->mem, rm->topts);
-    rm->n_pairs = 0;
+    // no pair tables: the roadmap starts from its edges
+    TRY(rm_upload(rm, t.samples, t.obstacles, offsets_time_h, xcomb_h, false));
+    TRY(upload_n(rm, &rm->row_start, t.row_start, (size_t)num + 1, s));
+    TRY(upload_n(rm, &rm->h, t.h, (size_t)num, s));
+    TRY(upload_n(rm, &rm->is_free_samples, t.is_free_samples, (size_t)num, s));
+    TRY(dalloc(rm->mem, &rm->in_degree, (size_t)num));
+    reserve_edges(rm, E, 0);
     rm->rn = t.rn;
     rm->n_edges = t.n_edges;
     rm->n_wp = n_wp;
     rm->max_hs = mh;
     rm->maxd2 = pump_maxd2(rm->prm.offset_mult);
-    TRY(upload_n(rm, &rm->row_start, t.row_start, (size_t)num + 1, s));
     TRY(upload_n(rm, &rm->edge_src, (const int *)src.data(), E, s));
     TRY(upload_n(rm, &rm->edge_dst, t.edge_dst, E, s));
     TRY(upload_n(rm, &rm->copts_edge, t.copts_edge, E, s));
     TRY(upload_n(rm, &rm->topts_edge, t.topts_edge, E, s));
-    TRY(upload_n(rm, &rm->h, t.h, (size_t)num, s));
     TRY(upload_n(rm, &rm->is_free_edges, t.is_free_edges, E, s));
-    TRY(upload_n(rm, &rm->is_free_samples, t.is_free_samples, (size_t)num, s));
     TRY(upload_n(rm, &rm->wp_offsets, t.wp_offsets, E + 1, s));
+    TRY(upload_n(rm, &rm->edge_hs_mask, (const uint64_t *)mask.data(), E, s));
+    reserve_waypoints(rm, (size_t)n_wp, (size_t)mh, false);
     TRY(upload_n(rm, &rm->as, t.as, (size_t)n_wp * mh * 3, s));
     TRY(upload_n(rm, &rm->bs, t.bs, (size_t)n_wp * mh, s));
     TRY(upload_n(rm, &rm->count, (const int *)count.data(), (size_t)n_wp, s));
-    TRY(upload_n(rm, &rm->edge_hs_mask, (const uint64_t *)mask.data(), E, s));
-    TRY(dalloc(rm->mem, &rm->in_degree, (size_t)num));
     TRY(pump_max_nn_size(rm->row_start, rm->edge_dst, rm->n_edges, num, rm->in_degree, &rm->max_nn,
                          s));
     return rm_finish(rm, t_begin);
@@ -467,6 +507,7 @@ void pump::rmb::rm_release(pump_roadmap *rm)
     dfree(rm->mem, rm->obstacles);
     dfree(rm->mem, rm->copts);
     dfree(rm->mem, rm->topts);
+    dfree(rm->mem, rm->select_ws);
     dfree(rm->mem, rm->topts64);
     dfree(rm->mem, rm->row_start);
     dfree(rm->mem, rm->edge_src);

@@ -25,6 +25,7 @@ struct pump_roadmap {
     std::vector<float> samples_h;
     hipStream_t stream = nullptr;
     float *samples = nullptr, *obstacles = nullptr, *copts = nullptr, *topts = nullptr;
+    char *select_ws = nullptr; // scratch of the selection over the pair tables
     double *topts64 = nullptr;
     int64_t n_pairs = 0, rn_idx = 0;
     float rn = 0;
@@ -219,10 +220,10 @@ struct EventTimer {
     } while (0)
 
 // Phases of the roadmap build (mainPUMP.cu:248-504): uploads, all ordered
-// pairs, the tables from rn to the waypoint offsets, the fused edge pass
-// and the half-spaces; rm_finish fills the info record.
+// pairs (their tables only with pairs set), the tables from rn to the waypoint
+// offsets, the fused edge pass and the half-spaces; rm_finish fills the info record.
 int rm_upload(pump_roadmap *rm, const float *samples_h, const float *obstacles_h,
-              const float *offsets_time_h, const float *xcomb_h);
+              const float *offsets_time_h, const float *xcomb_h, bool pairs);
 int rm_pairs(pump_roadmap *rm);
 int rm_tables(pump_roadmap *rm);
 int rm_alloc_halfspaces(pump_roadmap *rm);

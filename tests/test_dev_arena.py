@@ -68,7 +68,12 @@ static void run(const char *what, const std::vector<size_t> &sizes, int from = -
     held.clear();
     {
         pump::rmb::DevArena a;
+        // before the requests, room for the first three, which one block then holds
+        if (sizes.size() > 3)
+            a.reserve({sizes[2], sizes[0], sizes[1]});
+        const size_t before = live.size();
         std::vector<std::pair<void *, size_t>> got;
+        int served = 0;
         for (size_t n : sizes) {
             void *p = a.alloc(n);
             if (!p) {
@@ -80,10 +85,24 @@ static void run(const char *what, const std::vector<size_t> &sizes, int from = -
             }
             check(p, n, what);
             got.push_back({p, n});
+            if (!count && sizes.size() > 3 && ++served == 3 && live.size() != before) {
+                std::printf("%s: reserved room not used\n", what);
+                std::exit(1);
+            }
             if (got.size() % 3 == 0) { // every third request gives the first one back
                 a.release(got[0].first);
                 held.erase((char *)got[0].first);
                 got.erase(got.begin());
+                if (void *w = a.alloc_whole(n)) { // goes back at once, whatever its size
+                    const size_t with = live.size();
+                    check(w, n, what);
+                    a.release(w);
+                    held.erase((char *)w);
+                    if (live.size() + 1 != with) {
+                        std::printf("%s: not given back\n", what);
+                        std::exit(1);
+                    }
+                }
             }
         }
     }

@@ -1,6 +1,7 @@
 """A roadmap's device memory: searches whose buffers grow within and past the
 blocks they are cut from give the results of a fresh roadmap, roadmaps of two
-threads do not meet, and what a roadmap takes goes back with it."""
+threads do not meet, what a roadmap takes goes back with it, and the pair
+tables that it does not keep go back with the build."""
 import ctypes
 import threading
 
@@ -94,3 +95,46 @@ def test_two_threads_and_return(noise):
     P.sync()
     # eight roadmaps came and went; the runtime may keep a block or two
     assert before - free_bytes() < 256 << 20
+
+
+@pytest.mark.parametrize("num", [700, 1500, 2500])  # tables below, at and past a cut range's size
+def test_pair_tables_go_back(num, noise):
+    s, o = problem(num, 7)
+    table = num * (num - 1) * 4
+    held = {}
+    for keep in (0, 1, 0, 1):  # the second time without the runtime's own first allocations
+        P.sync()
+        before = free_bytes()
+        rm = P.Roadmap(s, o, s[-1], *noise, prm(num, 64, keep_pairs=keep))
+        P.sync()
+        held[keep] = before - free_bytes()
+        print("pair tables", num, keep, held[keep] >> 20, flush=True)
+        d = rm.device()
+        assert bool(d.copts) == bool(d.topts) == bool(keep)
+        rm.close()
+    # 4 MiB: the granularity of two allocations
+    assert held[1] - held[0] >= 2 * table - (4 << 20)
+
+
+def test_batch_holds_what_its_problems_need(noise):
+    """No more than a quarter above the arrays of the problems (and 2 MiB, the
+    granularity of an allocation, for each array that stands alone)."""
+    num, n = 1200, 12
+    problems, need = [], 0
+    for j in range(n):
+        s, o = problem(num, 50 + j)
+        problems.append((s, o, s[-1], prm(num, 64)))
+    P.Batch(problems, *noise).close()  # the runtime's own first allocations
+    P.sync()
+    before = free_bytes()
+    b = P.Batch(problems, *noise)
+    P.sync()
+    held = before - free_bytes()
+    for j in range(n):
+        i = b.roadmap(j).info
+        E, W, hs = int(i.n_edges), int(i.n_waypoints), int(i.max_hs)
+        need += 45 * num + 33 * E + W * (24 + 16 * hs + 4)
+    noise_bytes = 200 * 2048 * 3 * 4 * 2 + P.lib.pump_split_offsets_bytes(200, 2048)
+    print("batch", held >> 20, (need + noise_bytes) >> 20, flush=True)
+    assert held <= 1.25 * (need + noise_bytes) + n * 6 * (2 << 20)
+    b.close()
