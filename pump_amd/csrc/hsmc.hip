@@ -181,7 +181,9 @@ __device__ __forceinline__ void hs_block(const HsJob &J, int64_t e0, char *smem,
     // along one axis has d2 > maxd2 (hsmc.cu:69) at every waypoint of the
     // tile, so only the boxes near those bounds are scanned, in index order.
     // The reach exceeds sqrt(maxd2) by far more than the rounding of the
-    // clamp distances; a NaN or infinite maxd2 scans every box.
+    // clamp distances; a NaN or infinite maxd2 scans every box, and so does
+    // the tile of a waypoint that is not finite, whose d2 can be NaN for any
+    // box (the skip passes those over).
     const float reach =
         (maxd2 >= 0.0f && maxd2 < INFINITY) ? sqrtf(maxd2) * 1.001f + 1e-6f : INFINITY;
     for (int64_t base = g_begin; base < g_end; base += kHsBlock) {
@@ -215,10 +217,12 @@ __device__ __forceinline__ void hs_block(const HsJob &J, int64_t e0, char *smem,
         int stored = 0;
         bool live = false; // some stored b passes the sentinel test of PUMP.cu:642
         if (__ballot(work) != 0ull) {
+            const bool finite = fabsf(pos[0]) < INFINITY && fabsf(pos[1]) < INFINITY &&
+                                fabsf(pos[2]) < INFINITY;
             float tlo[3], thi[3];
             for (int d = 0; d < 3; ++d) {
-                tlo[d] = wave_min(work ? pos[d] : INFINITY) - reach;
-                thi[d] = wave_max(work ? pos[d] : -INFINITY) + reach;
+                tlo[d] = wave_min(!work ? INFINITY : finite ? pos[d] : -INFINITY) - reach;
+                thi[d] = wave_max(!work ? -INFINITY : finite ? pos[d] : INFINITY) + reach;
             }
             for (int wd = 0; wd < n_words; ++wd) {
                 const int bb = wd * 64 + lane;

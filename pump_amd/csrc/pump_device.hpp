@@ -844,8 +844,10 @@ __device__ __forceinline__ float read_lane(float x, int l)
 // the rotation as its DPP operand, one instruction per step, and combines
 // the row results on the scalar unit, where a float min needs a separate
 // move and a canonicalisation per step.  A NaN orders beyond the infinity of
-// its sign, so a union of bounds that holds one compares false with
-// everything: nothing counts as separated from it.
+// its sign: a positive one is the result of the max and passed over by the
+// min, a negative one the other way round.  A lane whose bounds may be NaN and
+// must not be passed over gives infinite ones instead (edge_bbox, the
+// half-space cache); in the full Monte Carlo a NaN segment hits nothing.
 __device__ __forceinline__ int ordered_int(int i) { return i ^ ((i >> 31) & 0x7fffffff); }
 
 template <int kCtrl> __device__ __forceinline__ int dpp_rotate(int x)
