@@ -22,6 +22,7 @@ constexpr int kSelSample = 16384; // keys of the sample, 16 per thread of one wo
 constexpr int kSelRun = 16;       // neighbouring keys per place of the sample: one 64-byte line
 constexpr int kSelTile = 8192;    // keys per workgroup and round of the bracket pass
 constexpr int kSelMaxRegions = 1024;
+constexpr int64_t kSelScatterMax = 1 << 25;
 
 // The keys still in question are those with key - lo <= span; k is the rank
 // sought among them.  The next pass bins them by (key - lo) >> shift.
@@ -33,13 +34,12 @@ struct SelState {
     uint32_t lo, span, shift;
     int counted; // k is a rank among the keys in question (not before the first pick)
     int done;    // result holds the answer
-    int missed;  // the bracket does not hold rank k, or its keys did not fit
+    int missed;  // the collected keys do not do: passes go over the array
     float result;
 
-    __device__ bool bracket_holds() const
-    {
-        return k >= below && k - below < n_cand && full == 0;
-    }
+    // rank k lies inside the bracket
+    __device__ bool inside() const { return k >= below && k - below < n_cand; }
+    __device__ bool bracket_holds() const { return inside() && full == 0; }
 };
 
 __device__ __forceinline__ uint32_t order_key(float f)
@@ -66,6 +66,28 @@ __device__ __forceinline__ void sel_whole_range(SelState *st)
     st->lo = 0;
     st->span = 0xffffffffu;
     st->shift = sel_shift(st->span);
+}
+
+// The ranks in a sample of m keys that bracket rank k of n: five standard
+// deviations to either side of k's place.  One past an end of the sample
+// leaves the bracket open there, whatever lies beyond.
+struct SelRanks {
+    int lo, hi;
+    bool open_lo, open_hi;
+};
+
+__host__ __device__ __forceinline__ SelRanks sel_ranks(int64_t k, int64_t n, int m)
+{
+    const float place = (float)k / (float)n * (float)m;
+    const int margin = (int)(5.0f * sqrtf(fminf(place, (float)m - place) + 1.0f)) + 4;
+    SelRanks r;
+    r.lo = (int)place - margin;
+    r.hi = (int)place + margin;
+    r.open_lo = r.lo <= 0;
+    r.open_hi = r.hi >= m - 1;
+    r.lo = r.lo > 0 ? r.lo : 0;
+    r.hi = r.hi < m - 1 ? r.hi : m - 1;
+    return r;
 }
 
 // inclusive scan of v over the workgroup; sh: one entry per wave
@@ -102,9 +124,8 @@ __global__ __launch_bounds__(256) void k_sel_init(SelState *st, unsigned long lo
 
 // One workgroup: keys that bracket rank k, from a sample (kSelRun neighbours at
 // a scattered place in each of 1024 equal stretches), after two rounds of 2048
-// bins each.  The ranks in the sample are five standard deviations to either
-// side of k's place; a bracket that misses rank k all the same is found out by
-// its counts.  With n <= kSelSample the sample is the array and the key of
+// bins each (sel_ranks; a bracket that misses rank k all the same is found out
+// by its counts).  With n <= kSelSample the sample is the array and the key of
 // rank k itself comes out (done).  Lines, not single keys: the scattered loads
 // of 16384 keys took 20 us more on an array of 6.4e7; bins between the
 // smallest and the largest key, not of the leading bits: costs span a few
@@ -156,13 +177,10 @@ __global__ __launch_bounds__(1024) void k_sel_sample(const float *__restrict__ k
         atomicMin(&least, lo_key);
         atomicMax(&most, hi_key);
     }
-    const float place = (float)k / (float)n * (float)m;
-    const int margin = (int)(5.0f * sqrtf(fminf(place, (float)m - place) + 1.0f)) + 4;
-    const bool open_lo = !whole && (int)place - margin <= 0;
-    const bool open_hi = !whole && (int)place + margin >= m - 1;
+    const SelRanks R = sel_ranks((int64_t)k, n, m);
     uint32_t rank[2], lo[2], span[2], shift[2];
-    rank[0] = whole ? (uint32_t)k : (uint32_t)max(0, (int)place - margin);
-    rank[1] = whole ? (uint32_t)k : (uint32_t)min(m - 1, (int)place + margin);
+    rank[0] = whole ? (uint32_t)k : (uint32_t)R.lo;
+    rank[1] = whole ? (uint32_t)k : (uint32_t)R.hi;
     __syncthreads();
     for (int e = 0; e < 2; ++e) {
         lo[e] = least;
@@ -209,8 +227,8 @@ __global__ __launch_bounds__(1024) void k_sel_sample(const float *__restrict__ k
             st->done = 1;
             st->result = key_float(lo[0]);
         } else {
-            const uint32_t hi = open_hi ? 0xffffffffu : lo[1] + span[1];
-            st->lo = open_lo ? 0u : lo[0];
+            const uint32_t hi = R.open_hi ? 0xffffffffu : lo[1] + span[1];
+            st->lo = R.open_lo ? 0u : lo[0];
             st->span = hi - st->lo;
             st->shift = sel_shift(st->span);
         }
@@ -219,7 +237,13 @@ __global__ __launch_bounds__(1024) void k_sel_sample(const float *__restrict__ k
 
 // One pass over all keys: counts those below the bracket and collects those
 // inside it (a percent or so) in cand, each workgroup in a region of its own
-// (region_cap keys; its count in counts).  Bound by the read of the array:
+// (region_cap keys; its count in counts).  With scatter a workgroup reads
+// 1024 keys at a time, all over the array, and not 8192, so that a stretch
+// with many keys of the bracket (an array in order, a sample near all others)
+// goes to many regions: 1e6 keys in order 66 us for 90.  Long arrays go
+// without (kSelScatterMax): 6.4e7 keys take 121 us for 118, and there the
+// passes that follow a full region cost less than they did before the bracket
+// (in order 214 us, 344 before; the middle rank 230, 276 before).  Bound by the read of the array:
 // 6.4e7 keys in 60 us (4.3 TB/s); the selection 225 -> 107 us against three
 // histogram passes over the array, 5 launches for 7.  (Turning the counts into
 // the next state in the workgroup that ends last cost 100 us: every wave's
@@ -227,7 +251,7 @@ __global__ __launch_bounds__(1024) void k_sel_sample(const float *__restrict__ k
 __global__ __launch_bounds__(256) void k_sel_bracket(const float *__restrict__ keys, int64_t n,
                                                      SelState *st, float *__restrict__ cand,
                                                      uint32_t *__restrict__ counts,
-                                                     uint32_t region_cap)
+                                                     uint32_t region_cap, bool scatter)
 {
     __shared__ uint32_t held;
     __shared__ unsigned long long sh[4];
@@ -257,17 +281,19 @@ __global__ __launch_bounds__(256) void k_sel_bracket(const float *__restrict__ k
                 keep(keys[i], atomicAdd(&held, 1u));
         }
     }
-    for (int64_t q0 = (int64_t)blockIdx.x * (256 * kVec); q0 < n4;
+    // a thread's kVec vectors lie hop apart
+    const int64_t hop = scatter ? (int64_t)gridDim.x * 256 : 256;
+    for (int64_t q0 = (int64_t)blockIdx.x * (scatter ? 256 : 256 * kVec); q0 < n4;
          q0 += (int64_t)gridDim.x * (256 * kVec)) {
         float4 v[kVec];
 #pragma unroll
         for (int j = 0; j < kVec; ++j) {
-            const int64_t q = q0 + j * 256 + threadIdx.x;
+            const int64_t q = q0 + j * hop + threadIdx.x;
             v[j] = vec[q < n4 ? q : n4 - 1];
         }
 #pragma unroll
         for (int j = 0; j < kVec; ++j) {
-            const bool have = q0 + j * 256 + threadIdx.x < n4;
+            const bool have = q0 + j * hop + threadIdx.x < n4;
             const float f[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
             uint64_t in[4], any = 0ull;
             uint32_t c = 0;
@@ -354,7 +380,10 @@ __global__ __launch_bounds__(1024) void k_sel_pass(const float *__restrict__ key
 }
 
 // One workgroup: narrows the keys in question to the bin of rank k (2 or 3
-// passes leave one key) and clears the histogram.
+// passes leave one key) and clears the histogram.  Where the bracket holds
+// rank k but the regions do not hold its keys, the passes that follow go over
+// the array and count only the keys of the bracket: no more than the two that
+// 22 bits take, and none if they are all equal.
 __global__ __launch_bounds__(1024) void k_sel_pick(SelState *st, unsigned long long *hist,
                                                    bool whole)
 {
@@ -364,14 +393,21 @@ __global__ __launch_bounds__(1024) void k_sel_pick(SelState *st, unsigned long l
     if (now.done || (now.missed && !whole)) // whole: the pass was over the array
         return;
     if (!now.counted) {
-        if (!now.bracket_holds()) {
-            if (threadIdx.x == 0) {
-                st->missed = st->counted = 1;
-                sel_whole_range(st);
+        now.missed = !now.bracket_holds();
+        now.counted = 1;
+        if (now.inside())
+            now.k -= now.below;
+        else
+            sel_whole_range(&now);
+        if (now.missed) {
+            if (now.span == 0) {
+                now.result = key_float(now.lo);
+                now.done = 1;
             }
+            if (threadIdx.x == 0)
+                *st = now;
             return;
         }
-        now.k -= now.below;
     }
     const int b0 = 2 * threadIdx.x;
     const unsigned long long c0 = hist[b0], c1 = hist[b0 + 1];
@@ -838,8 +874,10 @@ constexpr size_t kSelHist = 280;
 static_assert(sizeof(SelState) <= kSelHist && kSelHist % 8 == 0, "layout of the selection");
 static size_t select_rn_base() { return kSelHist + kSelBins * sizeof(unsigned long long); }
 
-// room for the bracket's keys, 10 sqrt(16384 p) + 8 of 16384 (at most 4%) when
-// a share p or 1 - p of the keys lies below, in equal regions
+// Room for the bracket's keys, in equal regions: 10 sqrt(16384 p) + 8 of 16384
+// where a share p or 1 - p of the keys lies below, 5.7% at most (p = 1/2; 0.8%
+// for the 50 nearest of 8000), of the 6.25% and more that there is room for.
+// Past it the passes go over the array: a middle rank of clustered keys can.
 static int64_t select_rn_cand(int64_t n) { return n <= kSelSample ? 0 : n / 16 + 131072; }
 
 extern "C" size_t pump_select_rn_workspace(int64_t n_pairs)
@@ -879,12 +917,14 @@ extern "C" int pump_select_rn(const float *d_copts, int64_t n_pairs, int64_t rn_
         PUMP_LAUNCHED();
         if (n_pairs > kSelSample) {
             hipLaunchKernelGGL(k_sel_bracket, dim3(regions), dim3(256), 0, s, d_copts, n_pairs, st,
-                               cand, counts, region_cap);
+                               cand, counts, region_cap, n_pairs <= kSelScatterMax);
             PUMP_LAUNCHED();
-            pass(nullptr);
-            PUMP_LAUNCHED();
-            pass(nullptr);
-            PUMP_LAUNCHED();
+            // an open bracket has more than 22 bits
+            const SelRanks R = sel_ranks(rn_idx, n_pairs, kSelSample);
+            for (int p = 0; p < (R.open_lo || R.open_hi ? 3 : 2); ++p) {
+                pass(nullptr);
+                PUMP_LAUNCHED();
+            }
         }
     } else {
         hipLaunchKernelGGL(k_sel_init, dim3(1), dim3(256), 0, s, st, hist, k);
@@ -898,9 +938,8 @@ extern "C" int pump_select_rn(const float *d_copts, int64_t n_pairs, int64_t rn_
     PUMP_HIP(hipMemcpyAsync(&got, st, sizeof(got), hipMemcpyDeviceToHost, s));
     PUMP_HIP(hipStreamSynchronize(s));
     if (!got.done) {
-        // a bracket of more than 22 bits needs one more pass over its keys; one
-        // that missed rank k needs three over the array
-        for (int p = 0; p < (got.missed ? 3 : 1); ++p) {
+        // 11 bits a pass: over the array where the collected keys do not do
+        for (uint32_t left = got.span; left; left >>= 11) {
             pass(got.missed ? d_copts : nullptr);
             PUMP_LAUNCHED();
         }

@@ -53,6 +53,34 @@ def test_select_at_the_edges(n, kind):
                 assert select(g, at, n, k, ws) == s[k], (at, k, ws.nbytes)
 
 
+@pytest.mark.parametrize("n,kind", [(n, k) for n in (16385, 70001, 6000003) for k in (
+    "ordered", "equal", "two", "crowded")] + [((1 << 25) + 3, "ordered")])
+def test_select_where_the_regions_may_not_do(n, kind):
+    """Keys of the bracket that lie together, that are all equal, or that fall
+    to one workgroup (it reads every r-th stretch of 1024 keys): the regions
+    overflow and the passes go over the array, inside the bracket."""
+    rng = np.random.default_rng(n)
+    x = rng.lognormal(1.0, 0.7, n).astype(np.float32)
+    if kind == "ordered":
+        x = np.sort(x)
+    elif kind == "equal":
+        x[:] = np.float32(2.5)
+    elif kind == "two":
+        x = np.where(x < np.float32(3), np.float32(1), np.float32(2))
+    else:
+        regions = min((n + 8191) // 8192, 1024)
+        one = (np.arange(n) // 1024) % regions == 0  # with vectors from keys[0] on
+        x[one] = np.median(x) * rng.uniform(0.9999, 1.0001, one.sum()).astype(np.float32)
+    g = dev(x)
+    s = np.sort(x)
+    ws_n = P.lib.pump_select_rn_workspace(n)
+    ws = P.DeviceArray(shape=(ws_n,), dtype=np.uint8, fill=0x5b)
+    below = int((x < np.float32(2)).sum())
+    for k in sorted({0, n // 5000, n // 160, n // 2, below - 1, below, n - 1} & set(range(n))):
+        print("select", n, kind, k, flush=True)
+        assert select(g, 0, n, k, ws) == s[k], k
+
+
 @pytest.mark.parametrize("num", [2, 3, 5, 6, 257, 1025, 1026, 8192, 8194, 8201])
 def test_edge_rows_at_the_edges(num):
     rng = np.random.default_rng(num)
