@@ -3,11 +3,11 @@
 //
 // The reference runs one thread per particle in 32 workgroups of 64 and walks
 // the path's segments serially.  Here a workgroup owns 64 particles of one
-// path, one per lane of each of its waves, and the waves share the path's
-// segments.  At one segment the 64 particles lie within the noise of one
+// path, one per lane of each of its waves (small launches: 16, each on four
+// lanes), and the waves share the path's segments.  At one segment the 64 particles lie within the noise of one
 // another, so few boxes meet the union of their segment boxes and only those
 // are tested lane by lane; the boxes are tested against the union 64 at a
-// time, from registers.  (Lanes over the segments of one particle had the
+// time.  (Lanes over the segments of one particle had the
 // whole path's extent as union, and idle lanes past its end: 64 paths of 4096
 // particles among 200 walls, 43 segments each, took 197 us, 5.7e10
 // segment-checks/s, and take 40 us, 2.8e11.)  Bound: VALU issue, about a
@@ -23,13 +23,26 @@ namespace {
 
 constexpr int kMaxWaves = 16; // waves of a workgroup at most
 // Waves of a launch, where the path count and particles leave fewer: 4096,
-// 8192, 16384, 32768 give 60, 57, 54, 60 us for 64 paths of 4096 particles
-// among 200 walls and about the same elsewhere.
+// 8192, 16384, 32768 give 46, 43, 40, 44 us for 64 paths of 4096 particles
+// among 200 walls, 20, 18, 20, 23 for 32 paths among 64.
 constexpr int kTargetWaves = 16384;
+// A launch of few groups of 64 particles is one chain of a wave's segments
+// long, on a few compute units: up to kSplitGroups of them a particle gets
+// kSplit lanes with a run of segments each.  One path of 1024 particles, 64
+// and 200 boxes: 4.6 and 4.7 us, 6.3 and 6.2 with one lane; 128 groups (8192
+// particles) 6.2 and 5.0, 7.0 and 5.5; 192 groups 6.9 and 6.7, 6.4 and 6.3.
+constexpr int kSplit = 4, kSplitGroups = 128;
+// More than 64 boxes are held in registers where a wave has segments enough
+// to use them on: from kRegisterWaves waves per workgroup down (11 segments of
+// 43 each).  64 paths of 4096 particles, 128 and 256 boxes: 34 and 43 us, from
+// memory 36 and 48; 32 paths (8 waves) 22 and 31, from memory 21 and 26; 16
+// paths (16 waves) 18 and 30, from memory 14 and 17.
+constexpr int kRegisterWaves = 4;
 
-// kBoxes: boxes per lane held in registers (0: any count, from LDS or global
-// memory).
-template <int kBoxes>
+// kBoxes: boxes per lane held in registers (0: any count, from global memory).
+// kSub: lanes per particle, each with segments of its own; 64 / kSub particles
+// per workgroup.
+template <int kBoxes, int kSub>
 __global__ __launch_bounds__(64 * kMaxWaves) void k_mccp(
     const float *__restrict__ obstacles, int n_obs, const float *__restrict__ xcomb,
     int tmax_steps, int n_mc, float om, const float *__restrict__ paths, int64_t stride_rows,
@@ -40,8 +53,8 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_mccp(
     const int lane = threadIdx.x & 63;
     const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n_waves = blockDim.x >> 6;
-    const int first = blockIdx.x * 64;
-    const int p = first + lane < n_mc ? first + lane : n_mc - 1; // idle lanes repeat the last
+    const int mine = blockIdx.x * (64 / kSub) + lane / kSub;
+    const int p = mine < n_mc ? mine : n_mc - 1; // idle lanes repeat the last
     const float *path = paths + (int64_t)k * stride_rows * kDim;
     // segments t < T-2 (the reference skips the final segment); bounded by
     // the noise table and the path buffer
@@ -50,8 +63,13 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_mccp(
         nseg = tmax_steps - 1;
     if (nseg > (int)stride_rows - 1)
         nseg = (int)stride_rows - 1;
-    const int chunk = (nseg + n_waves - 1) / n_waves;
-    const int t0 = wid * chunk, t1 = t0 + chunk < nseg ? t0 + chunk : nseg;
+    // Segments in kSub runs per wave of chunk each: lane l % kSub = 0 goes from
+    // u = t0 to t1, the others that many chunks ahead.  A lane past the last
+    // segment waits there.
+    const int chunk = (nseg + kSub * n_waves - 1) / (kSub * n_waves);
+    const int t0 = wid * kSub * chunk, t1 = t0 + chunk < nseg ? t0 + chunk : nseg;
+    const int ahead = kSub > 1 ? lane % kSub * chunk : 0;
+    const auto seg = [&](int u) { return kSub > 1 ? min(u + ahead, nseg - 1) : u; };
     // this lane's boxes: lane, lane + 64, ...
     constexpr int kRegs = kBoxes > 0 ? kBoxes : 1;
     float blo[kRegs][3], bhi[kRegs][3];
@@ -68,26 +86,28 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_mccp(
     const float *xc = xcomb + (int64_t)p * 3 * tmax_steps;
     bool hit = false;
     if (t0 < t1) {
-        // the point at t0, and the next point's noise loaded ahead
+        // the first point, and the next point's noise loaded ahead
         float v[3], xn[3];
         int vmin[3], vmax[3]; // bounds over the wave, as ordered integers
         for (int d = 0; d < 3; ++d) {
-            v[d] = path[t0 * kDim + d] + xc[t0 * 3 + d] * om;
-            xn[d] = xc[(t0 + 1) * 3 + d];
+            v[d] = path[seg(t0) * kDim + d] + xc[seg(t0) * 3 + d] * om;
+            xn[d] = xc[(seg(t0) + 1) * 3 + d];
         }
         for (int d = 0; d < 3; ++d) {
             const int i = ordered_int(__float_as_int(v[d]));
             vmin[d] = wave_min_i(i);
             vmax[d] = wave_max_i(i);
         }
-        for (int t = t0; t < t1; ++t) {
+        for (int u = t0; u < t1; ++u) {
+            const int t = seg(u);
+            const bool done = kSub > 1 && u + ahead >= nseg;
             float w[3];
             int wmin[3], wmax[3];
             for (int d = 0; d < 3; ++d)
                 w[d] = path[(t + 1) * kDim + d] + xn[d] * om;
-            if (t + 1 < t1)
+            if (u + 1 < t1)
                 for (int d = 0; d < 3; ++d)
-                    xn[d] = xc[(t + 2) * 3 + d];
+                    xn[d] = xc[(seg(u + 1) + 1) * 3 + d];
             // The union of the particles' segment boxes: a box separated from
             // it (the broad phase's own <= test) is separated from each.
             float umin[3], umax[3];
@@ -116,7 +136,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_mccp(
                             lo[d] = read_lane(blo[c][d], l);
                             hi[d] = read_lane(bhi[c][d], l);
                         }
-                        if (!hit)
+                        if (!(hit || done))
                             hit = segment_hits_box(v, w, bmin, bmax, lo, hi);
                     }
                 }
@@ -139,7 +159,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_mccp(
                             clo[d] = read_lane(lo[d], l);
                             chi[d] = read_lane(hi[d], l);
                         }
-                        if (!hit)
+                        if (!(hit || done))
                             hit = segment_hits_box(v, w, bmin, bmax, clo, chi);
                     }
                 }
@@ -153,7 +173,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_mccp(
             }
         }
     }
-    const unsigned long long m = __ballot(hit && first + lane < n_mc);
+    const unsigned long long m = __ballot(hit && mine < n_mc);
     if (lane == 0)
         hit_mask[wid] = m;
     __syncthreads();
@@ -161,6 +181,10 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_mccp(
         unsigned long long all = 0;
         for (int i = 0; i < n_waves; ++i)
             all |= hit_mask[i];
+        for (int b = kSub / 2; b > 0; b /= 2) // a particle's lanes to its first
+            all |= all >> b;
+        if (kSub > 1)
+            all &= ~0ull / ((1ull << (kSub % 64)) - 1ull);
         if (all)
             atomicAdd(&hits[k], __popcll(all));
     }
@@ -197,7 +221,10 @@ extern "C" int pump_collision_probability_many(const float *d_obstacles, int n_o
         PUMP_LAUNCHED();
     }
     // waves per workgroup: enough that the launch has kTargetWaves of them
-    const unsigned groups = (unsigned)((n_mc + 63) / 64);
+    unsigned groups = (unsigned)((n_mc + 63) / 64);
+    const bool split = (int64_t)groups * n_paths <= kSplitGroups;
+    if (split)
+        groups = (unsigned)((n_mc + 64 / kSplit - 1) / (64 / kSplit));
     int waves = 1;
     while (waves < kMaxWaves && (int64_t)groups * n_paths * waves < kTargetWaves)
         waves *= 2;
@@ -206,14 +233,16 @@ extern "C" int pump_collision_probability_many(const float *d_obstacles, int n_o
         hipLaunchKernelGGL(kernel, grid, block, 0, s, d_obstacles, n_obs, d_xcomb, tmax_steps,
                            n_mc, offset_mult, d_paths, path_stride_rows, d_T, d_hits);
     };
-    if (n_obs <= 64)
-        launch(k_mccp<1>);
-    else if (n_obs <= 128)
-        launch(k_mccp<2>);
-    else if (n_obs <= 256)
-        launch(k_mccp<4>);
+    if (split)
+        launch(k_mccp<0, kSplit>);
+    else if (n_obs <= 64)
+        launch(k_mccp<1, 1>);
+    else if (n_obs <= 128 && waves <= kRegisterWaves)
+        launch(k_mccp<2, 1>);
+    else if (n_obs <= 256 && waves <= kRegisterWaves)
+        launch(k_mccp<4, 1>);
     else
-        launch(k_mccp<0>);
+        launch(k_mccp<0, 1>);
     PUMP_LAUNCHED();
     return PUMP_OK;
 }
