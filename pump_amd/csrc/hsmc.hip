@@ -1346,13 +1346,24 @@ static int launch_path(int n_new, const int64_t *wp_offsets, int W_fixed, const 
 }
 
 // The batched form runs from kBatchedMin paths on where it has a workspace.
-// Otherwise a workgroup per path below kPathFormMax paths and 64 paths per
+// Otherwise a workgroup per path below path_form_max paths and 64 paths per
 // wave above: 2000 particles in bit rows take 8 against 70-107 us at 500
 // paths, 40-46 against 78-264 at 16384 and 72-87 against 87-300 at 32768 (few
 // and many boxes), where the launch of the workgroups (2 ns each) decides;
-// at 65536 paths few boxes favour the waves.
-constexpr int kPathFormMax = 32768;
+// at 65536 paths few boxes favour the waves.  With fewer than 5 slots per
+// waypoint (a world of as few boxes) and rows of few particles the waves have
+// less to do and are the faster form earlier: 1 to 4 boxes, 128 particles 35
+// against 37-51 us at 16000 paths, 42 and 37-46 at 20000, 67 and 38-46 at
+// 32767; 1000 particles 43 and 42-60 at 20000, 50 and 45-69 at 24000.  (With 5
+// slots and up to 500 particles the waves are ahead from 28000 paths on among
+// 10 boxes, 49-60 for 67-70 us, and far behind among 150, 80-104 for 70-75:
+// the call does not tell them apart.)
 constexpr int kBatchedMin = 4096;
+static int path_form_max(int max_hs, int n_p)
+{
+    return max_hs >= 5 || n_p >= 2000 ? 32768 : n_p >= 1000 ? 24576 : 20480;
+}
+
 // The drop-in call, whose batched form also allocates its workspace: a
 // workgroup per path takes 48-62 against 63-75 us at 16384 paths (500 and
 // 2000 particles, few and many boxes) and 87-120 against 70-87 at 32768.
@@ -1430,7 +1441,7 @@ extern "C" int pump_propagate_valid_particles(
         }
         (void)hipGetLastError(); // the failed request is not an error of this call
     }
-    if (num_new_paths < kPathFormMax || use_block_kernel())
+    if (num_new_paths < path_form_max(max_hs, n_p) || use_block_kernel())
         return launch_path<false>(num_new_paths, d_wp_offsets, waypoints_count, d_wf_edge,
                                   d_wf_prev, d_as, d_bs, (const uint64_t *)nullptr, d_times,
                                   d_topts, dt, max_hs, d_offsets_time, tmax_steps, offset_mult,
@@ -1682,7 +1693,7 @@ static int launch_propagate(int n_new, int W_fixed, const int64_t *wp_offsets, c
         PUMP_LAUNCHED();
         return bins_finish(B, kBits, s);
     }
-    if (n_new < kPathFormMax || use_block_kernel())
+    if (n_new < path_form_max(max_hs, n_p) || use_block_kernel())
         return launch_path<kBits>(n_new, wp_offsets, W_fixed, wf_edge, wf_prev, as, bs, edge_mask,
                                   times, topts, dt, max_hs, offsets_time, tmax_steps, om, n_mc,
                                   src, dst, dst_base, n_p, path_cp, cp_base, clamped, row_src, s);

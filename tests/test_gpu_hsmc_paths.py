@@ -17,7 +17,9 @@ pytestmark = pytest.mark.gpu
     (1, (2, 6), 1, 40), (63, (2, 40), 5, 40), (64, (2, 40), 5, 40), (65, (2, 40), 5, 40),
     (1024, (2, 20), 5, 40), (1025, (2, 20), 5, 300), (2000, (60, 70), 5, 40),
     (130, (64, 65), 3, 40), (320, (200, 230), 5, 20), (96, (2, 9), 700, 12),
-    (96, (2, 9), 1024, 12), (272, (3, 4), 5, 4095)])
+    (96, (2, 9), 1024, 12), (272, (3, 4), 5, 4095),
+    # to the 64-paths-per-wave form with few slots and particles
+    (96, (2, 9), 1, 20479), (96, (2, 9), 1, 20480), (1000, (2, 3), 4, 24576)])
 def test_path_form_against_oracle(n_p, w_range, max_hs, n_new):
     d = random_hsmc_inputs(n_p + max_hs, n_edges=80, max_hs=max_hs, n_p=n_p, n_mc=n_p + 3, T=70,
                            n_new=n_new, n_parent=9, variable=True, w_range=w_range)
