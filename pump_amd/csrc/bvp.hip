@@ -307,6 +307,51 @@ __device__ __forceinline__ void pairs_persistent(const Src &src, int64_t n_pairs
     }
 }
 
+// A launch of one workgroup: each lane takes its pair to the end, without the
+// queue and the refills.  10 samples to the goal take 6.6 us for 8.6, 64 take
+// 11.4 for 15.3, all pairs of 16 samples 16-20 for 20; 300 samples to the goal
+// 20.4 for 19.8 and 1000 26 for 22, so that it ends there.
+template <class Src>
+__device__ __forceinline__ void pairs_one_set(const Src &src, int64_t n_pairs)
+{
+    const int64_t g = (int64_t)blockIdx.x * kPairBlock + threadIdx.x;
+    if (g >= n_pairs)
+        return;
+    PairTerms T;
+    DerivTerms D;
+    BisectState S;
+    int i = 0, j = 0, inst = 0, steps = 0; // steps: not counted here
+    float a[kDim], b[kDim], tmax, cost = 0.0f;
+    src.load(g, a, b, tmax, i, j, inst);
+    const auto cost_at = [&](float x) {
+        float a[kDim], b[kDim];
+        src.states(i, j, inst, a, b);
+        return cost_of_states(a[0], a[1], a[2], a[3], a[4], a[5], b[0], b[1], b[2], b[3], b[4],
+                              b[5], x);
+    };
+    pair_terms(T, D, a, b);
+    bisect_start(D, tmax, S, steps);
+    while (S.state < ST_DONE) {
+        float xa, xb, ca, cb;
+        if (!bisect_costs(T, S, xa, xb, ca, cb)) {
+            ca = cost_at(xa);
+            cb = cost_at(xb);
+        }
+        cost = ca;
+        bisect_update(S, ca, cb, steps);
+    }
+    if (cost == 0.0f) // the sign of a zero
+        cost = cost_at(S.x);
+    src.store(i, j, inst, S.x, cost);
+}
+
+__global__ __launch_bounds__(kPairBlock) void k_fill_pairs_one_set(
+    const float *__restrict__ samples, int num, float tmax, float *__restrict__ copts,
+    float *__restrict__ topts, int64_t n_pairs, DivMagic dm)
+{
+    pairs_one_set(OnePairSource{samples, num, tmax, copts, topts, dm}, n_pairs);
+}
+
 __global__ __launch_bounds__(kPairBlock) void k_fill_pairs_persistent(
     const float *__restrict__ samples, int num, float tmax, float *__restrict__ copts,
     float *__restrict__ topts, int64_t n_pairs, DivMagic dm, int chunk,
@@ -326,11 +371,15 @@ __global__ __launch_bounds__(kPairBlock) void k_fill_pairs_many(
 }
 
 // h[i] = cost(toptBisection(x_i, goal)) for i < num-1, h[num-1] = 0
+template <bool kOneSet>
 __global__ __launch_bounds__(kPairBlock) void k_heuristic(const GoalSource src, int num)
 {
     if (blockIdx.x == 0 && threadIdx.x == 0)
         src.h[num - 1] = 0.0f;
-    pairs_persistent(src, num - 1, kSet, nullptr, nullptr);
+    if constexpr (kOneSet)
+        pairs_one_set(src, num - 1);
+    else
+        pairs_persistent(src, num - 1, kSet, nullptr, nullptr);
 }
 
 __global__ void k_zero_counter(unsigned long long *c)
@@ -473,6 +522,12 @@ int fill_copts_topts(const float *d_samples, int num, float tmax, float *d_copts
     if (r != PUMP_OK)
         return r;
     const DivMagic dm = n_pairs < (1ll << 32) ? div_magic((uint32_t)(num - 1)) : DivMagic{0, 0, 0};
+    if (n_pairs <= kPairBlock) {
+        hipLaunchKernelGGL(k_fill_pairs_one_set, dim3(p.blocks), dim3(kPairBlock), 0, s, d_samples,
+                           num, tmax, d_copts, d_topts, n_pairs, dm);
+        PUMP_LAUNCHED();
+        return PUMP_OK;
+    }
     if (!p.claims && !steps) {
         hipLaunchKernelGGL(k_fill_pairs_persistent, dim3(p.blocks), dim3(kPairBlock), 0, s, d_samples, num,
                            tmax, d_copts, d_topts, n_pairs, dm, p.chunk,
@@ -531,8 +586,9 @@ extern "C" int pump_heuristic(const float *d_samples, int num, const float *goal
     for (int d = 0; d < kDim; ++d)
         src.goal[d] = goal_host[d];
     // a set of 64 samples per wave
-    hipLaunchKernelGGL(k_heuristic, dim3((num + kPairBlock - 1) / kPairBlock), dim3(kPairBlock), 0,
-                       as_stream(stream), src, num);
+    const unsigned blocks = (unsigned)((num + kPairBlock - 1) / kPairBlock);
+    hipLaunchKernelGGL(blocks == 1 ? k_heuristic<true> : k_heuristic<false>, dim3(blocks),
+                       dim3(kPairBlock), 0, as_stream(stream), src, num);
     PUMP_LAUNCHED();
     return PUMP_OK;
 }

@@ -32,9 +32,10 @@ def states(n, seed):
                            rng.uniform(-0.5, 0.5, (n, 3))], 1).astype(np.float32)
 
 
-# one pair, a part of a set, whole sets and one more, one set per wave, several
-# per wave, and (from 4.2 million pairs) claimed chunks
-@pytest.mark.parametrize("n", [2, 8, 9, 64, 65, 257, 513, 1100, 2200])
+# one pair, a part of a set, whole sets and one more, the last launch of one
+# workgroup (16 for the pairs, 256 to the goal), one set per wave, several per
+# wave, and (from 4.2 million pairs) claimed chunks
+@pytest.mark.parametrize("n", [2, 8, 9, 16, 17, 64, 65, 256, 257, 513, 1100, 2200])
 def test_pair_tables_over_launch_shapes(n):
     s = states(n, n)
     print("pairs", n, flush=True)
@@ -57,7 +58,8 @@ def test_pair_tables_of_special_states(tmax):
     s[30:35] *= np.float32(40)
     s[35:45, 3:] = 0
     print("special", tmax, flush=True)
-    c, t, _ = gpu_tables(s, tmax)
+    c, t, h = gpu_tables(s, tmax)
+    assert np.array_equal(h[:-1], c.reshape(60, 59)[:-1, -1], equal_nan=True)
     k = 0
     for i in range(60):
         for j in range(60):
