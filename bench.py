@@ -233,17 +233,20 @@ def main():
     pairs = {"pair_solves_per_s": info.n_pairs / (ms_pairs / 1e3), "ms": ms_pairs,
              "ms_in_build": info.ms_pairs, "n_pairs": int(info.n_pairs), "reps": reps}
     if info.pair_steps > 0:
-        # algorithmic flops: a cost evaluation is 40 FP64 + 14 FP32 operations
-        # (2pBVP.cu:97-107 as written: no fused multiply-adds), a bisection
-        # step two evaluations and the dcost quotient (110); a pair's final
-        # step needs one evaluation (-56).  Peak: FP64 vector, which is also
-        # the unpacked FP32 rate.
-        flops = 110.0 * info.pair_steps - 56.0 * info.n_pairs
+        # The operations of the steps whose costs the kernel evaluates: 101 FP64
+        # and FP32 ones each (a fused multiply-add as two; the final cost is one
+        # such step).  Steps that the derivative's sign settles and a pair's
+        # set-up are left out.  The share of evaluated steps comes from a sample
+        # of pairs in the same code on the host.  Peak: FP64 vector, which is
+        # also the unpacked FP32 rate.
+        steps = info.pair_steps / info.n_pairs
+        evaluated = steps * evaluated_share(P, samples, prm.tmax)
+        flops = 101.0 * evaluated * info.n_pairs
         tflops = flops / (ms_pairs / 1e3) / 1e12
         pairs["roofline"] = {"bound": "valu", "achieved": tflops, "peak": FP64_PEAK / 1e12,
                              "unit": "TFLOP/s", "frac": tflops * 1e12 / FP64_PEAK,
                              "kernel": "k_fill_pairs_persistent (pump_fill_copts_topts)",
-                             "steps_per_pair": info.pair_steps / info.n_pairs,
+                             "steps_per_pair": steps, "evaluated_steps_per_pair": evaluated,
                              "flops_per_pair": flops / info.n_pairs}
     # the re-run tables against the build's: its edge list holds, row by row,
     # the table's entries below rn and their destinations
@@ -263,7 +266,8 @@ def main():
     pairs["rows_match_build"] = same
     log(f"pair pass: {ms_pairs:.2f} ms ({info.ms_pairs:.2f} ms in the build), "
         f"{pairs['pair_solves_per_s']:.3e} pair-solves/s"
-        + (f", {pairs['roofline']['steps_per_pair']:.2f} bisection steps per pair, "
+        + (f", {pairs['roofline']['steps_per_pair']:.2f} bisection steps per pair "
+           f"({pairs['roofline']['evaluated_steps_per_pair']:.2f} evaluated), "
            f"{pairs['roofline']['achieved']:.1f} TFLOP/s "
            f"({pairs['roofline']['frac'] * 100:.1f}% of FP64 peak)" if "roofline" in pairs else "")
         + f", rows match the build {same}")
@@ -882,6 +886,21 @@ def batch_pass(P, n_inst, reps):
                     "particles_per_wave": int(b.info.mc_particles_per_wave)}}
     b.close()
     return out
+
+
+def evaluated_share(P, samples, tmax, n=4096):
+    """Of the bisection steps of n random pairs, the share that the pair pass
+    evaluates the cost for (the others follow from the derivative's sign)."""
+    rng = np.random.default_rng(11)
+    t, c, k = np.zeros(1, np.float32), np.zeros(1, np.float32), np.zeros(3, np.int32)
+    total = np.zeros(3, np.int64)
+    for i, j in rng.integers(0, len(samples), (n, 2)):
+        if i != j:
+            P.lib.pump_host_pair(P.fp(np.ascontiguousarray(samples[i])),
+                                 P.fp(np.ascontiguousarray(samples[j])), np.float32(tmax),
+                                 P.fp(t), P.fp(c), P.ip(k))
+            total += k
+    return float(total[1] / total[0])
 
 
 def _cpu_edges(rm, samples, obstacles, R, cores):
