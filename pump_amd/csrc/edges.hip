@@ -31,7 +31,9 @@ constexpr int kTile = 256;
 constexpr int kEdgeObs = 256;                  // boxes staged in LDS by the edge pass
 constexpr int kEdgeMaskWords = kEdgeObs / 64;  // candidate-mask words per edge
 constexpr int kSlabs = 16;                     // slabs per axis of the slab table
-constexpr int kMapCap = 2016;                  // block waypoints mapped to their edge in LDS
+// Waypoints of a workgroup's edges that are mapped to their edge in LDS; with
+// more of them (128 edges of 16 waypoints and up) each lane searches for its own.
+constexpr int kMapCap = 2016;
 
 // Per-edge record of an edge-pass workgroup in LDS: everything a lane needs
 // to evaluate any waypoint of the edge, read from one base address.
@@ -967,9 +969,11 @@ static int edges_per_block()
 // LDS reads per word, the edges' masks 20 instructions per box that meets a
 // wave's edges and a test per candidate and segment.  800,000 edges, random
 // boxes, masks and table: 30 boxes 56 and 61 us (FP32 waypoints 50 and 57), 64
-// boxes 71 and 64 (67 and 61), 128 boxes 118 and 79 (124 and 82); in the
-// corridor world, 1.6 million edges, 50 boxes 104 and 116 (FP32 waypoints),
-// 200 boxes 357 and 282.
+// boxes 71 and 64 (67 and 61), 128 boxes 118 and 79 (124 and 82).  In the
+// corridor world, 1.6 million edges: 50 boxes 104 and 116 (FP32 waypoints), 65
+// boxes 133 and 135 (128 and 130), 80 boxes 147 and 139 (143 and 141), 100
+// boxes 165 and 147 (165 and 154), 130 boxes 216 and 187 (221 and 200), 200
+// boxes 290 and 233 (355 and 281).
 constexpr int kSlabMinObs = 65;
 
 template <bool kCheck, bool kWrite, int EPB, bool kSlab = false>

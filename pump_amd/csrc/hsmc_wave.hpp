@@ -1,7 +1,7 @@
 // hsmc_wave.hpp -- wave-level building blocks of the half-space Monte Carlo
 // step (PUMP.cu:613-705): per-path edge data, waypoint half-space masks and
-// the particle test loop.  Used by the wave-per-path, batched and time-binned
-// forms.
+// the particle test loop.  Used by the workgroup-per-path, 64-paths-per-wave,
+// batched and time-binned forms.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -329,7 +329,7 @@ __device__ __forceinline__ int64_t wave_index(const VGrid &G)
 }
 __device__ __forceinline__ int64_t wave_count(const VGrid &G) { return G.nb * (blockDim.x >> 6); }
 
-constexpr int kWalkGroups = 4; // particle groups of 64 per walk, wave-per-path kernel
+constexpr int kWalkGroups = 4; // particle groups of 64 per walk, 64-paths-per-wave form
 constexpr int kHsGroups = 4;   // the same for the group form of the batched pass
 
 // A path that meets at least one stored half-space, as listed by the

@@ -4,13 +4,13 @@
 // The reference runs one thread per particle in 32 workgroups of 64 and walks
 // the path's segments serially.  Here a workgroup owns 64 particles of one
 // path, one per lane of each of its waves (small launches: 16, each on four
-// lanes), and the waves share the path's segments.  At one segment the 64 particles lie within the noise of one
-// another, so few boxes meet the union of their segment boxes and only those
-// are tested lane by lane; the boxes are tested against the union 64 at a
-// time.  (Lanes over the segments of one particle had the
-// whole path's extent as union, and idle lanes past its end: 64 paths of 4096
-// particles among 200 walls, 43 segments each, took 197 us, 5.7e10
-// segment-checks/s, and take 40 us, 2.8e11.)  Bound: VALU issue, about a
+// lanes), and the waves share the path's segments.  At one segment the 64
+// particles lie within the noise of one another, so few boxes meet the union
+// of their segment boxes and only those are tested lane by lane; the boxes are
+// tested against the union 64 at a time.  (Lanes over the segments of one
+// particle had the whole path's extent as union, and idle lanes past its end:
+// 64 paths of 4096 particles among 200 walls, 43 segments each, took 197 us,
+// 5.7e10 segment-checks/s, and take 40 us, 2.8e11.)  Bound: VALU issue, about a
 // third of it the bounds' reductions; the noise rows are read a lane each,
 // uncoalesced, from L2.  Paths of a batch are the grid's y dimension.
 #include "pump_device.hpp"
