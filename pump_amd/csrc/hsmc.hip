@@ -217,12 +217,14 @@ __device__ __forceinline__ void hs_block(const HsJob &J, int64_t e0, char *smem,
         int stored = 0;
         bool live = false; // some stored b passes the sentinel test of PUMP.cu:642
         if (__ballot(work) != 0ull) {
-            const bool finite = fabsf(pos[0]) < INFINITY && fabsf(pos[1]) < INFINITY &&
-                                fabsf(pos[2]) < INFINITY;
-            float tlo[3], thi[3];
+            // lanes without work hold zeros
+            const bool every =
+                __ballot(!(fabsf(pos[0]) + fabsf(pos[1]) + fabsf(pos[2]) < INFINITY)) != 0ull;
+            const float r = every ? INFINITY : reach;
+            float tlo[3], thi[3]; // with r infinite these are infinite or NaN
             for (int d = 0; d < 3; ++d) {
-                tlo[d] = wave_min(!work ? INFINITY : finite ? pos[d] : -INFINITY) - reach;
-                thi[d] = wave_max(!work ? -INFINITY : finite ? pos[d] : INFINITY) + reach;
+                tlo[d] = wave_min(work ? pos[d] : INFINITY) - r;
+                thi[d] = wave_max(work ? pos[d] : -INFINITY) + r;
             }
             for (int wd = 0; wd < n_words; ++wd) {
                 const int bb = wd * 64 + lane;
