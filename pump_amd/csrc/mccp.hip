@@ -10,9 +10,11 @@
 // tested against the union 64 at a time.  (Lanes over the segments of one
 // particle had the whole path's extent as union, and idle lanes past its end:
 // 64 paths of 4096 particles among 200 walls, 43 segments each, took 197 us,
-// 5.7e10 segment-checks/s, and take 40 us, 2.8e11.)  Bound: VALU issue, about a
-// third of it the bounds' reductions; the noise rows are read a lane each,
-// uncoalesced, from L2.  Paths of a batch are the grid's y dimension.
+// 5.7e10 segment-checks/s, and take 40 us, 2.8e11.)  Bound there: VALU issue
+// (70% busy by four cycles an instruction; of 110 instructions per segment and
+// wave 48 are the bounds' reductions) and the waves' chains of segments; 64
+// paths of 2048 particles among 30 boxes, 28% busy, by the chains.  The noise
+// rows are read a lane each, uncoalesced, from L2.  Paths of a batch are the grid's y dimension.
 #include "pump_device.hpp"
 #include "pump_internal.hpp"
 
