@@ -55,7 +55,7 @@ def same(a, b):
 
 @pytest.mark.parametrize("num,keep", [(40, 1), (600, 0), (2300, 1)])
 def test_growing_searches_match_fresh_ones(num, keep, noise):
-    # 2300 samples: pair tables of 21 MB, past the largest cut range
+    # 2300 samples: pair tables of 21 MB, past what shared blocks give
     s, o = problem(num, num)
     sizes = [(64, 1), (2048, 0), (128, 1), (2000, 1)]
     print("memory", num, keep, flush=True)
